@@ -90,6 +90,9 @@ AMLA_DEV u32x2 ldg8_nt(const void *p) {
 
 AMLA_DEV bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
+// F.silu of a bf16 value, rounded to bf16 as torch does (inference/ops.py:189).
+AMLA_DEV float silu_bf16(float g) { return round_bf16(g / (1.f + expf(-g))); }
+
 // LDS address operand of __builtin_amdgcn_global_load_lds
 #define LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 

@@ -110,16 +110,20 @@ struct GemvGroups {
 GemvPlan plan_gemv_grouped(int M, int N, int K);
 int launch_gemv_grouped(const GemvParams &p, GemvGroups groups, const GemvPlan &plan, hipStream_t stream);
 // Routed-expert work scheduled on the device (amla_moe_experts_dev): entries
-// of (expert, first row, rows, unused) int32, their count in device memory,
-// and the device table of expert weights [6][E]: gate_w, gate_s, up_w, up_s,
-// down_w, down_s.  Row r of an entry's x / y is row (first row + r) of the
-// gathered buffers.
+// of (expert, first position, rows, unused) int32, their count in device
+// memory, and the device table of expert weights [6][E]: gate_w, gate_s, up_w,
+// up_s, down_w, down_s.  Row r of an entry is position (first position + r) of
+// the slots sorted by expert: [gate | up] reads hidden row gather[position] and
+// leaves h row [position], down reads h row [position] and writes expert_out
+// row scatter[position].
 struct MoeSched {
   const void *const *wtab;
   const int32_t *ent;
   const int32_t *count;
   int E;
-  int down;  // 0: [gate | up] as two weight segments (n_split = gate rows), 1: down
+  int down;               // 0: [gate | up] as two weight segments (n_split = gate rows), 1: down
+  const int32_t *rowmap;  // gather (down = 0) or scatter (down = 1)
+  bool part_by_entry;     // skinny K-part sums of entry g at row 16 g, else at row (first position)
 };
 AMLA_DEV void moe_sched_weights(GemvParams &p, const MoeSched &s, int e) {
   const void *const *t = s.wtab + (s.down ? 4 : 0) * s.E;
@@ -128,14 +132,38 @@ AMLA_DEV void moe_sched_weights(GemvParams &p, const MoeSched &s, int e) {
   p.w1 = s.down ? nullptr : static_cast<const uint8_t *>(t[2 * s.E + e]);
   p.s1 = s.down ? nullptr : static_cast<const float *>(t[3 * s.E + e]);
 }
-// Skinny GEMMs (GEMV_PLAIN) of the scheduled entries, each with at most max_m
-// rows; grid max_entries x plan.groups.  plan: plan_gemv_grouped(max_m, N, K);
-// p.part holds plan.kparts * (rows of all entries) * N fp32 when kparts > 1
-// (entry at first row r0 uses part + kparts * r0 * N).
+// Skinny GEMMs of the scheduled entries, each with at most 16 rows; grid
+// max_entries x plan.groups.  plan: plan_gemv_grouped(16 or less, N, K);
+// p.part holds plan.kparts * rows * N fp32 when kparts > 1 (rows: 16 per entry
+// or every position, MoeSched::part_by_entry).  down = 0: p.x hidden, p.y the
+// [gate | up] rows by position (used with one K part only), h the silu(gate) *
+// up rows; down = 1: p.x h, p.y expert_out, h unused.
 int launch_gemv_sched(const GemvParams &p, const MoeSched &s, int max_entries, int max_m, const GemvPlan &plan,
-                      hipStream_t stream);
-// Large-M fp8 GEMM tiles of the scheduled entries (rows <= 256 each).
-int launch_gemm_sched(const GemvParams &p, const MoeSched &s, int max_entries, hipStream_t stream);
+                      uint16_t *h, hipStream_t stream);
+// The scheduled entries of up to TILE_ROWS rows on the large tiles
+// (tile_gemm.hip).  down = 0: x hidden (ldx = K), y = h (N = ldy =
+// intermediate size); down = 1: x = h, y = expert_out.
+constexpr int TILE_ROWS = 128;
+struct MoeTileParams {
+  const uint16_t *x;
+  uint16_t *y;
+  int ldx, ldy, K, N;
+  int ntiles;  // column tiles (set by the launch)
+};
+int launch_tile_sched(const MoeTileParams &p, const MoeSched &s, int max_entries, hipStream_t stream);
+// The same tiles from a host list (amla_moe_experts): rows first .. first +
+// rows - 1 of x and of y, the bytes as launch_tile_sched leaves them.
+constexpr int TILE_MAX_GROUPS = 64;
+struct TileGroup {
+  const void *w0, *w1;
+  const float *s0, *s1;
+  int first, rows;
+};
+struct TileGroups {
+  int n;
+  TileGroup g[TILE_MAX_GROUPS];
+};
+int launch_tile_grouped(const MoeTileParams &p, const TileGroups &groups, bool down, hipStream_t stream);
 // Large-M fp8 GEMM with the same modes (M > 64).  With split_ws of at least
 // gemm_ws_bytes(M, N, K) bytes, tiles past the last full round of 256
 // workgroups are cut into K parts (fp32 partial sums in split_ws, summed in

@@ -29,8 +29,6 @@ namespace amla {
 
 // ---------------------------------------------------------------- silu * up
 
-AMLA_DEV float silu_bf16(float g) { return round_bf16(g / (1.f + expf(-g))); }
-
 // h[i] = bf16( bf16(silu(g[i])) * u[i] ); eight elements per thread step.
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t *__restrict__ g, const uint16_t *__restrict__ u,
                                                        int64_t n8, int64_t n, uint16_t *__restrict__ h) {
@@ -88,11 +86,8 @@ static int launch_silu_mul(const uint16_t *g, const uint16_t *u, int64_t n, uint
 }
 
 // h[r, j] = bf16( bf16(silu(gu[r, j])) * gu[r, n + j] ) for rows r of [gate | up]
-// (drows: the row count in device memory, else rows)
 __global__ __launch_bounds__(256) void silu_mul_rows_kernel(const uint16_t *__restrict__ gu, int rows, int n,
-                                                            uint16_t *__restrict__ h,
-                                                            const int32_t *__restrict__ drows = nullptr) {
-  if (drows) rows = *drows;
+                                                            uint16_t *__restrict__ h) {
   for (int r = blockIdx.y; r < rows; r += gridDim.y) {
     const uint16_t *g = gu + (size_t)r * 2 * n, *u = g + n;
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n / 8; c += gridDim.x * blockDim.x) {
@@ -468,6 +463,7 @@ namespace amla {
 // copy their lists into the workspace
 constexpr int MOE_ARG_SLOTS = 512;
 constexpr int MOE_MAX_SLOTS = 65536;  // slots per chunk
+constexpr int MOE_SKINNY_ROWS = 16;   // largest group on the skinny path (one MFMA row tile)
 
 struct RowList {
   int32_t row[MOE_ARG_SLOTS];
@@ -475,14 +471,12 @@ struct RowList {
 
 // dst row i (of `rows`) = src row L[i]  (gather), or dst row L[i] = src row i
 // (scatter); L = dlist when given (device memory), else the by-value list
-// (drows: the row count in device memory, else rows)
 template <bool SCATTER>
 __global__ __launch_bounds__(256) void move_rows_kernel(const uint16_t *__restrict__ src, int64_t d, int rows,
                                                         RowList list, const int32_t *__restrict__ dlist,
-                                                        uint16_t *__restrict__ dst,
-                                                        const int32_t *__restrict__ drows = nullptr) {
+                                                        uint16_t *__restrict__ dst) {
   const int i = blockIdx.x;
-  if (i >= (drows ? *drows : rows)) return;
+  if (i >= rows) return;
   const int li = dlist ? dlist[i] : list.row[i];
   const uint16_t *s = src + (size_t)(SCATTER ? i : li) * d;
   uint16_t *t = dst + (size_t)(SCATTER ? li : i) * d;
@@ -499,10 +493,7 @@ static MoeLayout moe_layout(int64_t m, int64_t d, int top_k, int64_t n) {
   MoeLayout L;
   L.chunk_tokens = (int)std::min<int64_t>(m, (m * top_k <= MOE_ARG_SLOTS ? MOE_ARG_SLOTS : MOE_MAX_SLOTS) / top_k);
   const size_t slots = (size_t)L.chunk_tokens * top_k;
-  // largest expert group on the skinny path: any run of one expert up to 64
-  // slots (a token may list an expert more than once, so a run can be longer
-  // than the chunk's token count); the K-part count grows with the group size
-  const int mg = (int)std::min<size_t>(slots, 64);
+  const int mg = (int)std::min<size_t>(slots, MOE_SKINNY_ROWS);  // largest expert group on the skinny path
   size_t off = 0;
   L.lists = off;
   off = align_up(off + (slots > MOE_ARG_SLOTS ? 2 * slots * 4 : 0), 256);
@@ -612,7 +603,8 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
     const int nruns = (int)run_begin.size() - 1;
     int max_small = 0;
     for (int r = 0; r < nruns; ++r)
-      if (run_begin[r + 1] - run_begin[r] <= 64) max_small = std::max(max_small, run_begin[r + 1] - run_begin[r]);
+      if (run_begin[r + 1] - run_begin[r] <= MOE_SKINNY_ROWS)
+        max_small = std::max(max_small, run_begin[r + 1] - run_begin[r]);
     GemvParams pg = {};  // [gate | up] x (cnt, D) -> gu (cnt, 2n)
     pg.ldx = D;
     pg.N = 2 * n;
@@ -629,29 +621,9 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
     pd.seq_len = 1;
     const GemvPlan plan_g = plan_gemv_grouped(std::max(max_small, 1), 2 * n, D);
     const GemvPlan plan_d = plan_gemv_grouped(std::max(max_small, 1), D, n);
-    // experts with more than 64 of these tokens: one large-M GEMM each
-    for (int r = 0; r < nruns; ++r) {
-      const int i0 = run_begin[r], cnt = run_begin[r + 1] - i0;
-      if (cnt <= 64) continue;
-      const int64_t e = ix[order[i0]];
-      GemvParams p = pg;
-      p.x = xs + (size_t)i0 * D;
-      p.M = cnt;
-      p.w0 = static_cast<const uint8_t *>(gate_w[e]);
-      p.s0 = gate_s[e];
-      p.w1 = static_cast<const uint8_t *>(up_w[e]);
-      p.s1 = up_s[e];
-      p.y = gu + (size_t)i0 * 2 * n;
-      if ((rc = launch_gemm(p, GEMV_PLAIN, st))) return rc;
-    }
-    // the others: grouped skinny GEMMs, GEMV_MAX_GROUPS experts per launch
+    const MoeTileParams tg = {xs, hb, D, n, D, n, 0}, td = {hb, ys, n, D, n, D, 0};
     for (int pass = 0; pass < 2; ++pass) {
-      if (pass == 1) {
-        // silu * up over every row of [gate | up]
-        silu_mul_rows_kernel<<<dim3((unsigned)std::max(1, std::min(n / 8 / 256, 16)), (unsigned)ns), 256, 0, st>>>(
-            gu, ns, n, hb);
-        if ((rc = check_launch("moe_experts silu_mul"))) return rc;
-      }
+      // groups of up to 16 rows: grouped skinny GEMMs, GEMV_MAX_GROUPS experts per launch
       const GemvPlan &pl = pass == 0 ? plan_g : plan_d;
       const GemvParams &base = pass == 0 ? pg : pd;
       if (pl.kparts > 1 && (size_t)pl.kparts * ns * base.N * 4 > L.part_bytes)
@@ -668,7 +640,7 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
         }
         if (r == nruns) break;
         const int i0 = run_begin[r], cnt = run_begin[r + 1] - i0;
-        if (cnt > 64) continue;
+        if (cnt > MOE_SKINNY_ROWS) continue;
         const int64_t e = ix[order[i0]];
         GemvGroup &g = gr.g[gr.n++];
         g.M = cnt;
@@ -691,18 +663,34 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
           g.part = pl.kparts > 1 ? part + (size_t)pl.kparts * i0 * D : nullptr;
         }
       }
-    }
-    for (int r = 0; r < nruns; ++r) {
-      const int i0 = run_begin[r], cnt = run_begin[r + 1] - i0;
-      if (cnt <= 64) continue;
-      const int64_t e = ix[order[i0]];
-      GemvParams q = pd;
-      q.x = hb + (size_t)i0 * n;
-      q.M = cnt;
-      q.w0 = static_cast<const uint8_t *>(down_w[e]);
-      q.s0 = down_s[e];
-      q.y = ys + (size_t)i0 * D;
-      if ((rc = launch_gemm(q, GEMV_PLAIN, st))) return rc;
+      if (pass == 0 && max_small) {
+        // silu * up over every row of [gate | up] (the tiles below write the larger groups' rows of h)
+        silu_mul_rows_kernel<<<dim3((unsigned)std::max(1, std::min(n / 8 / 256, 16)), (unsigned)std::min(ns, 65535)),
+                               256, 0, st>>>(gu, ns, n, hb);
+        if ((rc = check_launch("moe_experts silu_mul"))) return rc;
+      }
+      // larger groups: tiles of up to 128 rows, silu * up in their epilogue
+      TileGroups tl;
+      tl.n = 0;
+      for (int r = 0; r <= nruns; ++r) {
+        const int i0 = r < nruns ? run_begin[r] : 0, cnt = r < nruns ? run_begin[r + 1] - i0 : 0;
+        if (r < nruns && cnt <= MOE_SKINNY_ROWS) continue;
+        const int64_t e = r < nruns ? ix[order[i0]] : 0;
+        for (int c = 0; c < cnt; c += TILE_ROWS) {
+          TileGroup &g = tl.g[tl.n++];
+          g.w0 = pass == 0 ? gate_w[e] : down_w[e];
+          g.s0 = pass == 0 ? gate_s[e] : down_s[e];
+          g.w1 = pass == 0 ? up_w[e] : nullptr;
+          g.s1 = pass == 0 ? up_s[e] : nullptr;
+          g.first = i0 + c;
+          g.rows = std::min(TILE_ROWS, cnt - c);
+          if (tl.n == TILE_MAX_GROUPS) {
+            if ((rc = launch_tile_grouped(pass == 0 ? tg : td, tl, pass == 1, st))) return rc;
+            tl.n = 0;
+          }
+        }
+      }
+      if (tl.n && (rc = launch_tile_grouped(pass == 0 ? tg : td, tl, pass == 1, st))) return rc;
     }
     move_rows_kernel<true><<<ns, 256, 0, st>>>(ys, d, ns, scatter, dsc, eout);
     if ((rc = check_launch("moe_experts scatter"))) return rc;
@@ -725,27 +713,26 @@ constexpr int MSORT_WAVES = 16;     // 1024 threads
 constexpr int MSORT_MAXE = 512;     // experts per layer
 constexpr int MSORT_EBITS = 9;      // bits of an expert index
 constexpr int MOE_DEV_MAX_SLOTS = 65536;
-constexpr int MOE_TILE_ROWS = 256;  // rows of a GEMM tile entry
-
 struct MoeDevLayout {
-  int sb;                      // largest group on the skinny path
-  int sb1;                     // largest group of the one-tile skinny launch (<= 16 rows)
-  int max_small, max_small4, max_tiles;  // schedule entries (worst case)
-  size_t hdr, cls, gather, scatter, small, small4, tiles, xs, ys, gu, h, part, total;
+  bool has_tiles;            // groups of more than MOE_SKINNY_ROWS rows take the large tiles
+  int skinny_rows;           // rows of the largest skinny entry
+  int max_small, max_tiles;  // schedule entries (worst case)
+  bool part_by_entry;        // K-part sums at 16 rows per skinny entry, else at the entry's position
+  size_t hdr, cls, gather, scatter, small, tiles, gu, h, part, total;
 };
 
 static MoeDevLayout moe_dev_layout(int64_t m, int64_t d, int top_k, int64_t n, int64_t E) {
   MoeDevLayout L;
   const int64_t S = m * top_k;
-  // a token names an expert once in a routing, so a group has at most m rows;
-  // larger groups (repeated indices) and groups over 64 rows take the GEMM
-  L.sb = (int)std::min<int64_t>(std::min<int64_t>(m, 64), S);
-  // skinny groups of up to 16 rows and of 17..sb rows take separate launches
-  // (one x tile, or the tiles the largest needs), each sized for its own worst case
-  L.sb1 = std::min(L.sb, 16);
-  L.max_small = (int)std::min<int64_t>(E, S);
-  L.max_small4 = L.sb > L.sb1 ? (int)std::min<int64_t>(E, S / (L.sb1 + 1)) : 0;
-  L.max_tiles = (int)((S + MOE_TILE_ROWS - 1) / MOE_TILE_ROWS + std::min<int64_t>(E, S / (L.sb + 1)));
+  // Groups of up to 16 rows (decode) stream through the skinny GEMM, larger
+  // ones through tiles of up to 128 rows.  A token names an expert once in a
+  // routing, so m <= 16 tokens make no group above m; should a caller repeat
+  // an index there, the group is cut into skinny entries of m rows, and the
+  // tile launches (4.6 us each, empty) are left out.
+  L.has_tiles = m > MOE_SKINNY_ROWS;
+  L.skinny_rows = (int)std::min<int64_t>(m, MOE_SKINNY_ROWS);
+  L.max_small = (int)std::min<int64_t>(S, std::min<int64_t>(E, S) + (L.has_tiles ? 0 : S / L.skinny_rows));
+  L.max_tiles = L.has_tiles ? (int)(S / TILE_ROWS + std::min<int64_t>(E, S / (MOE_SKINNY_ROWS + 1))) : 0;
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align_up(off + bytes, 256); return o; };
   L.hdr = take(16);
@@ -753,17 +740,19 @@ static MoeDevLayout moe_dev_layout(int64_t m, int64_t d, int top_k, int64_t n, i
   L.gather = take((size_t)S * 4);
   L.scatter = take((size_t)S * 4);
   L.small = take((size_t)L.max_small * 16);
-  L.small4 = take((size_t)std::max(L.max_small4, 1) * 16);
   L.tiles = take((size_t)std::max(L.max_tiles, 1) * 16);
-  L.xs = take((size_t)S * d * 2);
-  L.ys = take((size_t)S * d * 2);
-  L.gu = take((size_t)S * 2 * n * 2);
   L.h = take((size_t)S * n * 2);
-  const GemvPlan a = plan_gemv_grouped(L.sb, (int)(2 * n), (int)d), b = plan_gemv_grouped(L.sb, (int)d, (int)n);
-  const size_t pa = a.kparts > 1 ? (size_t)a.kparts * S * 2 * n * 4 : 0;
-  const size_t pb = b.kparts > 1 ? (size_t)b.kparts * S * d * 4 : 0;
+  // [gate | up] rows (one K part) or K-part sums of the skinny entries
+  const GemvPlan a = plan_gemv_grouped(MOE_SKINNY_ROWS, (int)(2 * n), (int)d),
+                 b = plan_gemv_grouped(MOE_SKINNY_ROWS, (int)d, (int)n);
+  L.gu = take(a.kparts > 1 ? 16 : (size_t)S * 2 * n * 2);
+  L.part_by_entry = S > (int64_t)MOE_SKINNY_ROWS * L.max_small;
+  const size_t rows = L.part_by_entry ? (size_t)MOE_SKINNY_ROWS * L.max_small : (size_t)S;
+  const size_t pa = a.kparts > 1 ? a.kparts * rows * 2 * n * 4 : 0;
+  const size_t pb = b.kparts > 1 ? b.kparts * rows * d * 4 : 0;
   L.part = take(std::max<size_t>(std::max(pa, pb), 16));
-  L.total = off;
+  // never below the size callers could count on before the rows were gathered in place
+  L.total = std::max(off, (size_t)S * (2 * d + 3 * n) * 2);
   return L;
 }
 
@@ -787,23 +776,24 @@ AMLA_DEV int block_scan_incl(int v, int *wsum, int lane, int wave) {
 // position (rank among equal experts of the 64-slot step by ballots), so the
 // order is slot order within each expert whatever the timing.  Outputs:
 //   gather[p] = token of position p, scatter[p] = slot of position p;
-//   small[]   = (expert, first position, rows) of experts with 1..sb1 slots;
-//   small4[]  = the same for experts with sb1+1..sb slots;
-//   tiles[]   = (expert, first position, rows <= 256) of the larger ones;
-//   hdr       = {routed slots, small + small4 entries, tile entries, skipped slots};
-//   cls       = {small entries, small4 entries}.
+//   small[]   = (expert, first position, rows <= sr) of groups of up to sr
+//               slots (of every group, cut at sr, without has_tiles);
+//   tiles[]   = (expert, first position, rows <= 128) of the larger groups;
+//   cls       = {small entries, tile entries};
+//   hdr       = {routed slots, groups of 1 .. sb slots, 256-row tiles of the
+//               larger groups, skipped slots}, sb = min(tokens, 64).
 // Slots with a negative index are left out; an index >= E, or an expert with a
 // null or misaligned weight, is left out and counted as skipped.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const int64_t *__restrict__ idx, int S, int top_k, int E,
-                                                        int sb, int sb1, const void *const *__restrict__ wtab,
+                                                        int sb, int sr, bool has_tiles,
+                                                        const void *const *__restrict__ wtab,
                                                         int32_t *__restrict__ hdr, int32_t *__restrict__ cls,
                                                         int32_t *__restrict__ gather, int32_t *__restrict__ scatter,
-                                                        int32_t *__restrict__ small, int32_t *__restrict__ small4,
-                                                        int32_t *__restrict__ tiles) {
+                                                        int32_t *__restrict__ small, int32_t *__restrict__ tiles) {
   __shared__ int32_t cur[MSORT_WAVES][MSORT_MAXE];  // per-wave counts, then per-wave next positions
   __shared__ int32_t eok[MSORT_MAXE];
-  __shared__ int32_t wsum[4][MSORT_WAVES];
-  __shared__ int32_t skipped;
+  __shared__ int32_t wsum[3][MSORT_WAVES];
+  __shared__ int32_t skipped, groups, tiles256;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < MSORT_WAVES * MSORT_MAXE; i += 1024) (&cur[0][0])[i] = 0;
   for (int e = tid; e < E; e += 1024) {
@@ -815,7 +805,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int64_t *__restric
     }
     eok[e] = ok;
   }
-  if (tid == 0) skipped = 0;
+  if (tid == 0) skipped = groups = tiles256 = 0;
   __syncthreads();
   const int b0 = (int)((int64_t)S * wave / MSORT_WAVES), b1 = (int)((int64_t)S * (wave + 1) / MSORT_WAVES);
   auto expert_of = [&](int i) -> int {  // -1: left out, -2: skipped
@@ -841,39 +831,35 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int64_t *__restric
       tot += c;
     }
   }
-  const int is_small = tot >= 1 && tot <= sb1;
-  const int is_small4 = tot > sb1 && tot <= sb;
-  const int ntile = tot > sb ? (tot + MOE_TILE_ROWS - 1) / MOE_TILE_ROWS : 0;
+  if (tot > sb) atomicAdd(&tiles256, (tot + 255) / 256);
+  else if (tot > 0) atomicAdd(&groups, 1);
+  const bool big = has_tiles && tot > sr;
+  const int nsmall = big ? 0 : (tot + sr - 1) / sr;
+  const int ntile = big ? (tot + TILE_ROWS - 1) / TILE_ROWS : 0;
   const int pos_incl = block_scan_incl(tot, wsum[0], lane, wave);
-  const int small_incl = block_scan_incl(is_small, wsum[1], lane, wave);
-  const int small4_incl = block_scan_incl(is_small4, wsum[3], lane, wave);
+  const int small_incl = block_scan_incl(nsmall, wsum[1], lane, wave);
   const int tile_incl = block_scan_incl(ntile, wsum[2], lane, wave);
   const int first = pos_incl - tot;
   if (tid < E) {
 #pragma unroll
     for (int w = 0; w < MSORT_WAVES; ++w) cur[w][tid] += first;
-    if (is_small) {
-      int32_t *en = small + 4 * (small_incl - 1);
-      en[0] = tid; en[1] = first; en[2] = tot; en[3] = 0;
-    }
-    if (is_small4) {
-      int32_t *en = small4 + 4 * (small4_incl - 1);
-      en[0] = tid; en[1] = first; en[2] = tot; en[3] = 0;
-    }
-    for (int j = 0; j < ntile; ++j) {
-      int32_t *en = tiles + 4 * (tile_incl - ntile + j);
-      en[0] = tid; en[1] = first + j * MOE_TILE_ROWS; en[2] = min(MOE_TILE_ROWS, tot - j * MOE_TILE_ROWS); en[3] = 0;
+    const int rows = big ? TILE_ROWS : sr;
+    int32_t *en = big ? tiles + 4 * (tile_incl - ntile) : small + 4 * (small_incl - nsmall);
+    for (int j = 0; j < nsmall + ntile; ++j, en += 4) {
+      en[0] = tid; en[1] = first + j * rows; en[2] = min(rows, tot - j * rows); en[3] = 0;
     }
   }
   if (tid == 1023) {
     hdr[0] = pos_incl;
-    hdr[1] = small_incl + small4_incl;
-    hdr[2] = tile_incl;
     cls[0] = small_incl;
-    cls[1] = small4_incl;
+    cls[1] = tile_incl;
   }
   __syncthreads();
-  if (tid == 0) hdr[3] = skipped;
+  if (tid == 0) {
+    hdr[1] = groups;
+    hdr[2] = tiles256;
+    hdr[3] = skipped;
+  }
   // placement, in slot order per wave
   for (int base = b0; base < b1; base += 64) {
     const int i = base + lane;
@@ -931,39 +917,36 @@ int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, co
   int32_t *hdr = reinterpret_cast<int32_t *>(ws + L.hdr);
   int32_t *gather = reinterpret_cast<int32_t *>(ws + L.gather), *scatter = reinterpret_cast<int32_t *>(ws + L.scatter);
   int32_t *small = reinterpret_cast<int32_t *>(ws + L.small), *tiles = reinterpret_cast<int32_t *>(ws + L.tiles);
-  uint16_t *xs = reinterpret_cast<uint16_t *>(ws + L.xs), *ys = reinterpret_cast<uint16_t *>(ws + L.ys);
   uint16_t *gu = reinterpret_cast<uint16_t *>(ws + L.gu), *hb = reinterpret_cast<uint16_t *>(ws + L.h);
   float *part = reinterpret_cast<float *>(ws + L.part);
+  const uint16_t *hid = static_cast<const uint16_t *>(hidden);
+  uint16_t *eout = static_cast<uint16_t *>(expert_out);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int S = (int)(m * top_k), n = (int)n_inter, D = (int)d, E = (int)n_experts;
   int rc;
-  int32_t *cls = reinterpret_cast<int32_t *>(ws + L.cls), *small4 = reinterpret_cast<int32_t *>(ws + L.small4);
-  moe_sort_kernel<<<1, 1024, 0, st>>>(indices, S, top_k, E, L.sb, L.sb1, weight_table, hdr, cls, gather, scatter,
-                                      small, small4, tiles);
+  int32_t *cls = reinterpret_cast<int32_t *>(ws + L.cls);
+  moe_sort_kernel<<<1, 1024, 0, st>>>(indices, S, top_k, E, (int)std::min<int64_t>(m, 64), L.skinny_rows, L.has_tiles,
+                                      weight_table, hdr, cls, gather, scatter, small, tiles);
   if ((rc = check_launch("moe_experts_dev schedule"))) return rc;
-  RowList none = {};
-  move_rows_kernel<false><<<S, 256, 0, st>>>(static_cast<const uint16_t *>(hidden), d, S, none, gather, xs, hdr);
-  if ((rc = check_launch("moe_experts_dev gather"))) return rc;
-  const MoeSched small_gu = {weight_table, small, cls, E, 0}, tiles_gu = {weight_table, tiles, hdr + 2, E, 0};
-  const MoeSched small_dn = {weight_table, small, cls, E, 1}, tiles_dn = {weight_table, tiles, hdr + 2, E, 1};
-  const MoeSched small4_gu = {weight_table, small4, cls + 1, E, 0}, small4_dn = {weight_table, small4, cls + 1, E, 1};
-  GemvParams pg = {};  // [gate | up] x (rows, D) -> gu (rows, 2n)
-  pg.x = xs; pg.ldx = D; pg.N = 2 * n; pg.K = D; pg.n_split = n; pg.y = gu; pg.ldy = 2 * n; pg.seq_len = 1;
+  const MoeSched small_gu = {weight_table, small, cls, E, 0, gather, L.part_by_entry},
+                 small_dn = {weight_table, small, cls, E, 1, scatter, L.part_by_entry};
+  const MoeSched tiles_gu = {weight_table, tiles, cls + 1, E, 0, gather, false},
+                 tiles_dn = {weight_table, tiles, cls + 1, E, 1, scatter, false};
+  const int sm = L.skinny_rows;
+  // h rows (by position) = silu(gate) * up of hidden rows gather[]
+  GemvParams pg = {};
+  pg.x = hid; pg.ldx = D; pg.N = 2 * n; pg.K = D; pg.n_split = n; pg.y = gu; pg.ldy = 2 * n; pg.seq_len = 1;
   pg.part = part;
-  GemvParams pd = {};  // down h (rows, n) -> ys (rows, D)
-  pd.x = hb; pd.ldx = n; pd.N = D; pd.K = n; pd.n_split = D; pd.y = ys; pd.ldy = D; pd.seq_len = 1;
+  const MoeTileParams tg = {hid, hb, D, n, D, n, 0};
+  if ((rc = launch_tile_sched(tg, tiles_gu, L.max_tiles, st))) return rc;
+  if ((rc = launch_gemv_sched(pg, small_gu, L.max_small, sm, plan_gemv_grouped(sm, 2 * n, D), hb, st))) return rc;
+  // expert_out rows scatter[] = down(h)
+  GemvParams pd = {};
+  pd.x = hb; pd.ldx = n; pd.N = D; pd.K = n; pd.n_split = D; pd.y = eout; pd.ldy = D; pd.seq_len = 1;
   pd.part = part;
-  if ((rc = launch_gemm_sched(pg, tiles_gu, L.max_tiles, st))) return rc;
-  if ((rc = launch_gemv_sched(pg, small_gu, L.max_small, L.sb1, plan_gemv_grouped(L.sb1, 2 * n, D), st))) return rc;
-  if ((rc = launch_gemv_sched(pg, small4_gu, L.max_small4, L.sb, plan_gemv_grouped(L.sb, 2 * n, D), st))) return rc;
-  silu_mul_rows_kernel<<<dim3((unsigned)std::max(1, std::min(n / 8 / 256, 16)), (unsigned)std::min(S, 65535)), 256,
-                         0, st>>>(gu, S, n, hb, hdr);
-  if ((rc = check_launch("moe_experts_dev silu_mul"))) return rc;
-  if ((rc = launch_gemm_sched(pd, tiles_dn, L.max_tiles, st))) return rc;
-  if ((rc = launch_gemv_sched(pd, small_dn, L.max_small, L.sb1, plan_gemv_grouped(L.sb1, D, n), st))) return rc;
-  if ((rc = launch_gemv_sched(pd, small4_dn, L.max_small4, L.sb, plan_gemv_grouped(L.sb, D, n), st))) return rc;
-  move_rows_kernel<true><<<S, 256, 0, st>>>(ys, d, S, none, scatter, static_cast<uint16_t *>(expert_out), hdr);
-  return check_launch("moe_experts_dev scatter");
+  const MoeTileParams td = {hb, eout, n, D, n, D, 0};
+  if ((rc = launch_tile_sched(td, tiles_dn, L.max_tiles, st))) return rc;
+  return launch_gemv_sched(pd, small_dn, L.max_small, sm, plan_gemv_grouped(sm, D, n), nullptr, st);
 }
 
 }  // extern "C"

@@ -217,8 +217,10 @@ __host__ __device__ inline int gemv_nbuf(int tile_bytes) { return tile_bytes >= 
 __host__ __device__ constexpr int gemv_kpb_max(int MT) { return MT == 4 ? 12 : GEMV_KPB; }
 __host__ __device__ inline int gemv_kpb4(int kpb) { return (kpb + 3) & ~3; }
 
-template <int MT, int MODE>
-AMLA_DEV void gemv_body(const GemvParams &p, int unit, int rg, int kparts, int kpb) {
+// xrow / yrow (MAP only, either may be null): row m of x / y is row xrow[m] / yrow[m].
+template <int MT, int MODE, bool MAP = false>
+AMLA_DEV void gemv_body(const GemvParams &p, int unit, int rg, int kparts, int kpb, const int32_t *xrow = nullptr,
+                        const int32_t *yrow = nullptr) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
@@ -266,6 +268,14 @@ AMLA_DEV void gemv_body(const GemvParams &p, int unit, int rg, int kparts, int k
     asm volatile("" ::: "memory");
   };
 
+  // x rows of this lane, read before the weight copies go out (loads complete
+  // in order: after them the x loads would wait for the first tiles)
+  int xm[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int m = 16 * t + li;
+    xm[t] = MAP && xrow ? xrow[min(m, p.M - 1)] : m;
+  }
   // the first weight tiles are in flight while x is read
   if (tile_begin < tile_end) {
 #pragma unroll
@@ -282,7 +292,7 @@ AMLA_DEV void gemv_body(const GemvParams &p, int unit, int rg, int kparts, int k
     for (int j = 0; j < NJ; ++j) {
       const int bl = wave + 4 * j, m = 16 * t + li;
       const bool ok = bl < nbp && m < p.M;
-      const uint16_t *xp = p.x + (size_t)m * p.ldx + (size_t)(kb_begin + bl) * 128 + lg * 16;
+      const uint16_t *xp = p.x + (size_t)xm[t] * p.ldx + (size_t)(kb_begin + bl) * 128 + lg * 16;
 #pragma unroll
       for (int q = 0; q < 4; ++q) xr[t][j][q] = ok ? ldg16(xp + (q & 1) * 8 + (q >> 1) * 64) : u32x4{0, 0, 0, 0};
     }
@@ -385,7 +395,7 @@ AMLA_DEV void gemv_body(const GemvParams &p, int unit, int rg, int kparts, int k
     const int n = (tile_begin + tl) * 16 + 4 * (ln >> 4);
     if (m >= p.M) continue;
     const f32x4 v = done[(tl * MT + t) * 64 + ln];
-    if (kparts == 1) store4<MODE>(p, m, n, v);
+    if (kparts == 1) store4<MODE>(p, MAP && yrow ? yrow[m] : m, n, v);
     else *reinterpret_cast<f32x4 *>(p.part + ((size_t)part * p.M + m) * p.N + n) = v;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last trips' (unused) copies land before exit
@@ -423,7 +433,7 @@ size_t gemv_lds_bytes(int MT, int kpb, int rg, int kparts) {
 // Sums the K parts of gemv_kernel in part order and applies the epilogue.
 // All parts are loaded before the first add (independent loads in flight).
 template <int MODE>
-AMLA_DEV void gemv_finish_body(const GemvParams &p, int64_t i, int kparts) {
+AMLA_DEV void gemv_finish_body(const GemvParams &p, int64_t i, int kparts, const int32_t *yrow = nullptr) {
   const int64_t total = (int64_t)p.M * (p.N >> 2);
   if (i >= total) return;
   const int m = (int)(i / (p.N >> 2));
@@ -436,7 +446,7 @@ AMLA_DEV void gemv_finish_body(const GemvParams &p, int64_t i, int kparts) {
 #pragma unroll
   for (int q = 1; q < GEMV_MAX_PARTS; ++q)
     if (q < kparts) s += v[q];
-  store4<MODE>(p, m, n, s);
+  store4<MODE>(p, yrow ? yrow[m] : m, n, s);
 }
 
 template <int MODE>
@@ -454,9 +464,9 @@ __global__ __launch_bounds__(64) void gemv_finish_grouped(GemvParams p, GemvGrou
   gemv_finish_body<GEMV_PLAIN>(q, (int64_t)(blockIdx.x % gr.units) * 64 + threadIdx.x, kparts);
 }
 
-// Skinny GEMMs of a device schedule (routed experts): entry g = blockIdx.x /
-// units; entries past the device count return at once (uniform per workgroup).
-template <int MT>
+// Skinny GEMMs of a device schedule (routed experts, up to 16 rows each):
+// entry g = blockIdx.x / units; entries past the device count return at once
+// (uniform per workgroup).
 __global__ __launch_bounds__(256, 2) void gemv_sched_kernel(GemvParams p, MoeSched s, int units, int rg, int kparts,
                                                          int kpb) {
   const int g = blockIdx.x / units;
@@ -464,23 +474,74 @@ __global__ __launch_bounds__(256, 2) void gemv_sched_kernel(GemvParams p, MoeSch
   const int32_t *en = s.ent + 4 * g;
   const int e = en[0], r0 = en[1];
   p.M = en[2];
-  p.x += (size_t)r0 * p.ldx;
-  p.y += (size_t)r0 * p.ldy;
-  p.part += (size_t)kparts * r0 * p.N;
+  if (s.down) p.x += (size_t)r0 * p.ldx;
+  else p.y += (size_t)r0 * p.ldy;
+  p.part += (size_t)kparts * (s.part_by_entry ? 16 * g : r0) * p.N;
   moe_sched_weights(p, s, e);
-  gemv_body<MT, GEMV_PLAIN>(p, blockIdx.x % units, rg, kparts, kpb);
+  gemv_body<1, GEMV_PLAIN, true>(p, blockIdx.x % units, rg, kparts, kpb, s.down ? nullptr : s.rowmap + r0,
+                                 s.down ? s.rowmap + r0 : nullptr);
 }
 
-// gemv_finish for the entries of gemv_sched_kernel: units blocks of 64 per entry.
+// gemv_finish for the down entries of gemv_sched_kernel: units blocks of 64 per entry.
 __global__ __launch_bounds__(64) void gemv_finish_sched(GemvParams p, MoeSched s, int units, int kparts) {
   const int g = blockIdx.x / units;
   if (g >= *s.count) return;
   const int32_t *en = s.ent + 4 * g;
   const int r0 = en[1];
   p.M = en[2];
-  p.y += (size_t)r0 * p.ldy;
-  p.part += (size_t)kparts * r0 * p.N;
-  gemv_finish_body<GEMV_PLAIN>(p, (int64_t)(blockIdx.x % units) * 64 + threadIdx.x, kparts);
+  p.part += (size_t)kparts * (s.part_by_entry ? 16 * g : r0) * p.N;
+  gemv_finish_body<GEMV_PLAIN>(p, (int64_t)(blockIdx.x % units) * 64 + threadIdx.x, kparts, s.rowmap + r0);
+}
+
+// The gate | up entries of gemv_sched_kernel: sums the K parts in part order
+// (or, with one K part, reads the stored bf16 rows) and writes
+// h = bf16( bf16(silu(gate)) * up ), four columns per thread.
+__global__ __launch_bounds__(64) void gu_silu_sched_kernel(GemvParams p, MoeSched s, int units, int kparts,
+                                                           uint16_t *__restrict__ h) {
+  const int g = blockIdx.x / units;
+  if (g >= *s.count) return;
+  const int32_t *en = s.ent + 4 * g;
+  const int r0 = en[1], n = p.n_split;
+  const int64_t i = (int64_t)(blockIdx.x % units) * 64 + threadIdx.x;
+  if (i >= (int64_t)en[2] * (n >> 2)) return;
+  const int m = (int)(i / (n >> 2)), j = (int)(i % (n >> 2)) * 4;
+  float gv[4], uv[4];
+  if (kparts > 1) {
+    const float *part = p.part + (size_t)kparts * (s.part_by_entry ? 16 * g : r0) * p.N;
+    f32x4 gq[GEMV_MAX_PARTS], uq[GEMV_MAX_PARTS];
+#pragma unroll
+    for (int q = 0; q < GEMV_MAX_PARTS; ++q)
+      if (q < kparts) {
+        const float *row = part + ((size_t)q * en[2] + m) * p.N;
+        gq[q] = *reinterpret_cast<const f32x4 *>(row + j);
+        uq[q] = *reinterpret_cast<const f32x4 *>(row + n + j);
+      }
+    f32x4 gs = gq[0], us = uq[0];
+#pragma unroll
+    for (int q = 1; q < GEMV_MAX_PARTS; ++q)
+      if (q < kparts) {
+        gs += gq[q];
+        us += uq[q];
+      }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      gv[k] = round_bf16(gs[k]);
+      uv[k] = round_bf16(us[k]);
+    }
+  } else {
+    const uint16_t *row = p.y + (size_t)(r0 + m) * p.ldy;
+    const u32x2 gw = ldg8(row + j), uw = ldg8(row + n + j);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      gv[2 * k] = lo_bf(gw[k]);
+      gv[2 * k + 1] = hi_bf(gw[k]);
+      uv[2 * k] = lo_bf(uw[k]);
+      uv[2 * k + 1] = hi_bf(uw[k]);
+    }
+  }
+  const u32x2 o = {pack_bf16(silu_bf16(gv[0]) * uv[0], silu_bf16(gv[1]) * uv[1]),
+                   pack_bf16(silu_bf16(gv[2]) * uv[2], silu_bf16(gv[3]) * uv[3])};
+  *reinterpret_cast<u32x2 *>(h + (size_t)(r0 + m) * n + j) = o;
 }
 
 // One workgroup per row m: sums the K parts of every output of the row in
@@ -1861,38 +1922,31 @@ int launch_gemv_grouped(const GemvParams &p, GemvGroups gr, const GemvPlan &pl, 
   return check_launch("grouped fp8 skinny GEMM");
 }
 
-template <int MT>
-static void launch_sched_mt(const GemvParams &p, const MoeSched &s, int max_entries, const GemvPlan &pl,
-                            hipStream_t st) {
-  static bool attr_set = false;  // raise the dynamic LDS limit once per process
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void *)gemv_sched_kernel<MT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    attr_set = true;
-  }
-  gemv_sched_kernel<MT><<<dim3((unsigned)(max_entries * pl.groups)), 256, pl.lds, st>>>(p, s, pl.groups, pl.rg,
-                                                                                      pl.kparts, pl.kpb);
-}
-
 int launch_gemv_sched(const GemvParams &p, const MoeSched &s, int max_entries, int max_m, const GemvPlan &pl,
-                      hipStream_t st) {
+                      uint16_t *h, hipStream_t st) {
   if (max_entries <= 0) return AMLA_OK;
-  if (max_m < 1 || max_m > 64) return fail(AMLA_EINVAL, "scheduled skinny GEMM: max rows %d", max_m);
-  if (p.N % 16 || p.K % 128 || pl.kparts > GEMV_MAX_PARTS || (!s.down && p.n_split % 128))
+  if (max_m < 1 || max_m > 16) return fail(AMLA_EINVAL, "scheduled skinny GEMM: max rows %d", max_m);
+  if (p.N % 16 || p.K % 128 || pl.kparts > GEMV_MAX_PARTS || (!s.down && (p.n_split % 128 || p.N != 2 * p.n_split)))
     return fail(AMLA_EUNSUPPORTED, "scheduled skinny GEMM: unsupported shape N=%d K=%d", p.N, p.K);
   if (pl.kparts > 1 && !p.part) return fail(AMLA_EWORKSPACE, "scheduled skinny GEMM: missing partial sums");
-  const int MT = max_m <= 16 ? 1 : (max_m <= 32 ? 2 : 4);
-  if (gemv_lds_bytes(MT, pl.kpb, pl.rg, pl.kparts) > pl.lds || pl.kpb > gemv_kpb_max(MT))
+  if (gemv_lds_bytes(1, pl.kpb, pl.rg, pl.kparts) > pl.lds || pl.kpb > gemv_kpb_max(1))
     return fail(AMLA_EINVAL, "scheduled skinny GEMM: plan for a smaller M");
-  if ((int64_t)max_entries * pl.groups > INT32_MAX) return fail(AMLA_EUNSUPPORTED, "scheduled skinny GEMM: grid");
-  if (MT == 1) launch_sched_mt<1>(p, s, max_entries, pl, st);
-  else if (MT == 2) launch_sched_mt<2>(p, s, max_entries, pl, st);
-  else launch_sched_mt<4>(p, s, max_entries, pl, st);
-  if (pl.kparts > 1) {
-    const int units = (int)(((int64_t)max_m * (p.N / 4) + 63) / 64);
-    gemv_finish_sched<<<dim3((unsigned)(max_entries * units)), 64, 0, st>>>(p, s, units, pl.kparts);
+  const int64_t units = ((int64_t)max_m * ((s.down ? p.N : p.n_split) / 4) + 63) / 64;
+  if ((int64_t)max_entries * pl.groups > INT32_MAX || max_entries * units > INT32_MAX)
+    return fail(AMLA_EUNSUPPORTED, "scheduled skinny GEMM: grid");
+  static bool attr_set = false;  // raise the dynamic LDS limit once per process
+  if (!attr_set) {
+    (void)hipFuncSetAttribute((const void *)gemv_sched_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    attr_set = true;
   }
-  return check_launch("scheduled fp8 skinny GEMM");
+  gemv_sched_kernel<<<dim3((unsigned)(max_entries * pl.groups)), 256, pl.lds, st>>>(p, s, pl.groups, pl.rg, pl.kparts,
+                                                                                   pl.kpb);
+  const int rc = check_launch("scheduled fp8 skinny GEMM");
+  if (rc) return rc;
+  const dim3 grid((unsigned)(max_entries * units));
+  if (!s.down) gu_silu_sched_kernel<<<grid, 64, 0, st>>>(p, s, (int)units, pl.kparts, h);
+  else if (pl.kparts > 1) gemv_finish_sched<<<grid, 64, 0, st>>>(p, s, (int)units, pl.kparts);
+  return check_launch("scheduled fp8 skinny GEMM finish");
 }
 
 // ---------------------------------------------------------------- rms_norm

@@ -400,21 +400,6 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(GemvParams p, GemmSpli
   }
 }
 
-// Tiles of the routed experts from a device schedule: workgroup (x, y) takes
-// output columns 256 x of entry y (expert e, rows r0 .. r0 + rows - 1 of x and
-// y, rows <= 256); entries past the count return at once.
-__global__ __launch_bounds__(G_NW * 64, 1) void gemm_sched_kernel(GemvParams p, MoeSched s) {
-  const int t = blockIdx.y;
-  if (t >= *s.count) return;
-  const int32_t *en = s.ent + 4 * t;
-  const int e = en[0], r0 = en[1];
-  p.M = en[2];
-  p.x += (size_t)r0 * p.ldx;
-  p.y += (size_t)r0 * p.ldy;
-  moe_sched_weights(p, s, e);
-  gemm_body<GEMV_PLAIN>(p, true, blockIdx.x * G_BN, 0, 0, p.K >> 7, nullptr);
-}
-
 // Tiles past the last full round of 256 workgroups are cut into K parts so
 // that the launch ends with the machine full: time ~ (rounds of 256 work
 // items) x (tile time / parts) + the partial sums written and read back (256
@@ -497,22 +482,6 @@ int launch_gemm(const GemvParams &p, int mode, hipStream_t st, float *split_ws, 
     default: gemm_finish_kernel<GEMV_QROPE><<<fgrid, 256, 0, st>>>(p, sp); break;
   }
   return check_launch("fp8 GEMM K-part finish");
-}
-
-int launch_gemm_sched(const GemvParams &p, const MoeSched &s, int max_entries, hipStream_t st) {
-  if (max_entries <= 0) return AMLA_OK;
-  if (p.K % 128 || p.N % 8 || p.ldx % 8 || p.ldy % 8 || !aligned16(p.x) || !aligned16(p.y))
-    return fail(AMLA_EUNSUPPORTED, "scheduled fp8 GEMM needs K %% 128 == 0, N %% 8 == 0 and 16-byte aligned rows");
-  if (!s.down && p.n_split % G_BN)
-    return fail(AMLA_EUNSUPPORTED, "scheduled fp8 GEMM: the first weight segment must be a multiple of 256 rows");
-  if (max_entries > 65535) return fail(AMLA_EUNSUPPORTED, "scheduled fp8 GEMM: %d entries", max_entries);
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void *)gemm_sched_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, G_LDS);
-    attr_set = true;
-  }
-  gemm_sched_kernel<<<dim3((p.N + G_BN - 1) / G_BN, max_entries), G_NW * 64, G_LDS, st>>>(p, s);
-  return check_launch("scheduled fp8 GEMM");
 }
 
 // ---------------------------------------------------------------- K10 causal flash attention

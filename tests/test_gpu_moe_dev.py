@@ -224,3 +224,46 @@ def test_moe_block_in_a_hip_graph():
         if r == 0:
             assert_parity(static_out, F.moe_block(x, gw, shared, lambda e: table[e], cfg), "graph replay vs oracle")
     assert len(routes) > 1, "the inputs should route differently"
+
+
+@pytest.mark.parametrize("d", [256, 384])
+def test_moe_experts_groups_at_the_tile_edges(d):
+    """Groups around every edge of the row tiles (16 rows on the skinny path, then 32, 64, 96 and
+    128 rows of a large tile, and more than one tile), a hidden size whose last 256-column tile is
+    half, and zero block scales in every projection: grouping on the device and on the host
+    against the oracle, and against each other bit for bit (the same tiles run either way)."""
+    print(f"[case] moe_experts tile edges d={d}", flush=True)
+    rows = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 160, 257]
+    E, i, m = len(rows), 256, sum(rows)
+    g = torch.Generator().manual_seed(d)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(m, generator=g)].view(m, 1)
+    h = _x((m, d), f"mdev-edge{d}")
+    table = {e: _mlp(d, i, f"mdev-edge{e}") for e in range(E)}
+    for e in range(E):   # zero scales: first, middle or last K block of one row block
+        for k in ("gate_proj", "up_proj", "down_proj"):
+            s = table[e][k][1]
+            s[e % s.shape[0], e % s.shape[1]] = 0.0
+    stacked = _stacked(table, E)
+    got, hdr = _run_dev(h, idx, stacked, E, i)
+    assert hdr[0] == m and hdr[3] == 0
+    assert_parity(got, _want(h, idx, table), f"moe_experts_dev tile edges d={d}")
+    tables, _ = ops._stacked_expert_tables(stacked, E, d, torch.device(DEV))
+    host = torch.empty(m, 1, d, dtype=torch.bfloat16, device=DEV)
+    ops._moe_experts_call(h.to(DEV), idx.contiguous(), tables, i, E, host)
+    torch.cuda.synchronize()
+    assert torch.equal(host.cpu(), got)
+
+
+@pytest.mark.parametrize("m,K", [(1, 40), (5, 13), (16, 20)])
+def test_moe_experts_dev_few_tokens_repeating_one_expert(m, K):
+    """Up to 16 tokens that name one expert over and over: its group is longer than the skinny
+    path's rows and is cut into entries of m rows."""
+    print(f"[case] moe_experts_dev m={m} K={K} one expert", flush=True)
+    E, d, i = 3, 256, 256
+    h = _x((m, d), f"mdev-rep{m}")
+    idx = torch.ones(m, K, dtype=torch.int64)
+    idx[0, 0], idx[m - 1, K - 1] = 0, 2
+    table = {e: _mlp(d, i, f"mdev-rep{e}") for e in range(E)}
+    got, hdr = _run_dev(h, idx, _stacked(table, E), E, i)
+    assert hdr[0] == m * K and hdr[3] == 0
+    assert_parity(got, _want(h, idx, table), f"moe_experts_dev repeated m={m} K={K}")
