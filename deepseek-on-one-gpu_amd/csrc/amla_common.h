@@ -104,6 +104,30 @@ AMLA_DEV void wait_vmcnt() {
   else asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
+// Maximum / minimum over the 64 lanes of a wave, in every lane, by lane swaps
+// inside the vector unit (a shuffle goes through LDS, ~10x the latency).
+template <int CTRL>
+AMLA_DEV uint32_t dpp_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+}
+template <typename F>
+AMLA_DEV uint32_t wave_reduce_u32(uint32_t v, F f) {
+  v = f(v, dpp_u32<0xB1>(v));   // quad_perm [1,0,3,2]
+  v = f(v, dpp_u32<0x4E>(v));   // quad_perm [2,3,0,1]
+  v = f(v, dpp_u32<0x141>(v));  // row_half_mirror
+  v = f(v, dpp_u32<0x140>(v));  // row_mirror
+  const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  v = f(a[0], a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return f(b[0], b[1]);
+}
+AMLA_DEV uint32_t wave_max_u32(uint32_t v) {
+  return wave_reduce_u32(v, [](uint32_t x, uint32_t y) { return x > y ? x : y; });
+}
+AMLA_DEV uint32_t wave_min_u32(uint32_t v) {
+  return wave_reduce_u32(v, [](uint32_t x, uint32_t y) { return x < y ? x : y; });
+}
+
 // Butterfly reductions inside a wave.
 AMLA_DEV float wave_sum(float v) {
 #pragma unroll

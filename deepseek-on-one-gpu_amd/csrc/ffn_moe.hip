@@ -284,8 +284,72 @@ __global__ __launch_bounds__(256) void route_logits_kernel(const uint16_t *__res
   }
 }
 
+// The same partial logits for many tokens: 64 tokens x 64 experts per
+// workgroup.  With 16 x 16 tiles every hidden row is read once per 16 experts
+// (0.92 GB through the L2s at 2000 tokens x 256 experts, 106 us); here once
+// per 64 (0.23 GB).  The four waves take interleaved 32-wide K steps, each on
+// the whole tile (2 x 2 MFMAs of 32 x 32), and add their tiles in wave order.
+constexpr int ROUTE_WIDE_M = 64;  // tokens above which the wide tile is used: below, too few workgroups
+__global__ __launch_bounds__(256) void route_logits_wide_kernel(const uint16_t *__restrict__ hidden,
+                                                                const uint16_t *__restrict__ gw, int M, int D, int E,
+                                                                float *__restrict__ part) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int e0 = blockIdx.x * 64, m0 = blockIdx.y * 64, z = blockIdx.z, nz = gridDim.z;
+  const int j32 = lane & 31, hh = lane >> 5;
+  const uint16_t *hp[2], *wp[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    hp[i] = hidden + (size_t)min(m0 + 32 * i + j32, M - 1) * D + 16 * hh;
+    wp[i] = gw + (size_t)min(e0 + 32 * i + j32, E - 1) * D + 16 * hh;
+  }
+  f32x16 acc[2][2];  // [expert half][token half]: lane holds token column j32
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[g][j][r] = 0.f;
+  const int steps = D / 32;
+#pragma unroll 4
+  for (int ks = wave + 4 * z; ks < steps; ks += 4 * nz) {
+    bf16x8 h[2][2], w[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        h[i][c] = as_bf16x8(ldg16(hp[i] + ks * 32 + 8 * c));
+        w[i][c] = as_bf16x8(ldg16(wp[i] + ks * 32 + 8 * c));
+      }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[g][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[g][c], h[j][c], acc[g][j], 0, 0, 0);
+  }
+  // [wave][token][expert], rows padded so that the 32 tokens of a store hit different banks
+  constexpr int PITCH = 64 + 4;
+  __shared__ float red[4][64 * PITCH];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4 *>(&red[wave][(32 * j + j32) * PITCH + 32 * g + 8 * q + 4 * hh]) =
+            f32x4{acc[g][j][4 * q], acc[g][j][4 * q + 1], acc[g][j][4 * q + 2], acc[g][j][4 * q + 3]};
+  __syncthreads();
+  float *logits = part + (size_t)z * M * E;
+  const int e = e0 + lane;
+  for (int t = wave; t < 64; t += 4) {
+    const int o = t * PITCH + lane;
+    const float v = ((red[0][o] + red[1][o]) + red[2][o]) + red[3][o];
+    if (m0 + t < M && e < E) logits[(size_t)(m0 + t) * E + e] = v;
+  }
+}
+
 constexpr int ROUTE_MAX_E = 1024;           // experts per token handled by one wave
-constexpr int ROUTE_EPL = ROUTE_MAX_E / 64;  // experts per lane (lane l: l, l + 64, ..)
 constexpr int ROUTE_MAX_Z = 8;               // K splits of the logits (route_ksplit)
 
 // One wave per token: scores = sigmoid(logits); rank the n_group groups by
@@ -297,15 +361,16 @@ constexpr int ROUTE_MAX_Z = 8;               // K splits of the logits (route_ks
 // larger maximum, or an equal one at a lower index: the order of picking the
 // best remaining group topk_group times); the top_k rounds are wave
 // reductions.
+template <int EPL>  // experts per lane (lane l: l, l + 64, ..): E <= 64 EPL
 __global__ __launch_bounds__(64) void route_select_kernel(const float *__restrict__ part, int M, int ksplit, int E,
                                                           int n_group, int topk_group, int top_k, int norm,
                                                           int64_t *__restrict__ idx_out, float *__restrict__ w_out) {
   __shared__ int gmax[64];  // group maxima as the bits of non-negative floats (ordered like the values)
   const int lane = threadIdx.x, m = blockIdx.x;
   const int gs = E / n_group;
-  float sc[ROUTE_EPL];
+  float sc[EPL];
 #pragma unroll
-  for (int i = 0; i < ROUTE_EPL; ++i) {
+  for (int i = 0; i < EPL; ++i) {
     const int e = lane + 64 * i;
     float v[ROUTE_MAX_Z];
 #pragma unroll
@@ -319,7 +384,7 @@ __global__ __launch_bounds__(64) void route_select_kernel(const float *__restric
   if (lane < n_group) gmax[lane] = 0;  // +0.0f: every score is >= 0
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < ROUTE_EPL; ++i) {
+  for (int i = 0; i < EPL; ++i) {
     const int e = lane + 64 * i;
     if (e < E) atomicMax(&gmax[e / gs], __float_as_int(sc[i]));
   }
@@ -338,29 +403,31 @@ __global__ __launch_bounds__(64) void route_select_kernel(const float *__restric
   // candidate scores: experts of dropped groups take part as 0.0 (the
   // reference's masked_scores), chosen ones are removed as -1
 #pragma unroll
-  for (int i = 0; i < ROUTE_EPL; ++i) {
+  for (int i = 0; i < EPL; ++i) {
     const int e = lane + 64 * i;
     if (e < E && !((keep >> (e / gs)) & 1)) sc[i] = 0.f;
   }
   float sum = 0.f, my_w = 0.f;
   int my_idx = 0;
   for (int t = 0; t < top_k; ++t) {
-    float bv = -2.f;
-    int bi = E;
+    // Best score over the lanes, then the lowest index that has it.  Scores are
+    // >= 0, so their bits order like the values; keys: NaN or no expert 0,
+    // already chosen 1 (only left when the others are NaN), else bits + 2.
+    uint32_t bk = 0;
+    int bl = E;
 #pragma unroll
-    for (int i = 0; i < ROUTE_EPL; ++i)
-      if (sc[i] > bv) {  // ascending e per lane: ties keep the lower index
-        bv = sc[i];
-        bi = lane + 64 * i;
+    for (int i = 0; i < EPL; ++i) {
+      const uint32_t key = sc[i] >= 0.f ? __float_as_uint(sc[i]) + 2u : (sc[i] == -1.f ? 1u : 0u);
+      if (key > bk) {  // ascending e per lane: ties keep the lower index
+        bk = key;
+        bl = lane + 64 * i;
       }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
-      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
     }
+    const uint32_t key = wave_max_u32(bk);
+    const int bi = (int)wave_min_u32(bk == key ? (uint32_t)bl : 0xffffffffu);
+    const float bv = key >= 2u ? __uint_as_float(key - 2u) : (key == 1u ? -1.f : -2.f);
 #pragma unroll
-    for (int i = 0; i < ROUTE_EPL; ++i)
+    for (int i = 0; i < EPL; ++i)
       if (lane + 64 * i == bi) sc[i] = -1.f;
     if (lane == t) {
       my_idx = bi;
@@ -393,12 +460,59 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t *__rest
   }
 }
 
+// moe_combine_kernel with eight columns per thread (d % 8 == 0, 16-byte
+// aligned rows): the top_k rows' 16-byte loads of a thread go out together,
+// eight at a time.  Bound: HBM, (top_k + 2) rows per token; 2000 tokens x 8 of
+// 7168 (287 MB) 146 us with one column per thread.
+__global__ __launch_bounds__(256) void moe_combine8_kernel(const uint16_t *__restrict__ shared,
+                                                           const uint16_t *__restrict__ eout,
+                                                           const float *__restrict__ w, int top_k, int d8,
+                                                           int64_t items, float scale, uint16_t *__restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= items) return;
+  const int64_t m = i / d8;
+  const int c = (int)(i - m * d8);
+  const u32x4 sh = ldg16(shared + i * 8);
+  const uint16_t *src = eout + (m * top_k * d8 + c) * 8;
+  const float *wm = w + m * top_k;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < top_k; k0 += 8) {
+    u32x4 v[8];
+    float wk[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int kk = min(k0 + k, top_k - 1);
+      v[k] = ldg16_nt(src + (int64_t)kk * d8 * 8);
+      wk[k] = round_bf16(wm[kk]);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (k0 + k < top_k) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          acc[2 * e] = round_bf16(acc[2 * e] + round_bf16(wk[k] * lo_bf(v[k][e])));
+          acc[2 * e + 1] = round_bf16(acc[2 * e + 1] + round_bf16(wk[k] * hi_bf(v[k][e])));
+        }
+      }
+  }
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    o[e] = pack_bf16(lo_bf(sh[e]) + round_bf16(acc[2 * e] * scale), hi_bf(sh[e]) + round_bf16(acc[2 * e + 1] * scale));
+  *reinterpret_cast<u32x4 *>(out + i * 8) = o;
+}
+
 }  // namespace amla
 
 extern "C" {
 
 // K splits of the router logits: about 128 workgroups for decode-sized batches
+// (16 x 16 tiles), 512 for the 64 x 64 tiles
 static int route_ksplit(int64_t m, int64_t n_experts) {
+  if (m > ROUTE_WIDE_M) {
+    const int64_t wide = ((n_experts + 63) / 64) * ((m + 63) / 64);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(ROUTE_MAX_Z, 512 / std::max<int64_t>(wide, 1)));
+  }
   const int64_t tiles = ((n_experts + 15) / 16) * ((m + 15) / 16);
   return (int)std::max<int64_t>(1, std::min<int64_t>(ROUTE_MAX_Z, 128 / std::max<int64_t>(tiles, 1)));
 }
@@ -430,13 +544,18 @@ int amla_moe_route(const void *hidden, int64_t m, int64_t d, const void *gate_we
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   float *part = static_cast<float *>(workspace);
   const int ks = route_ksplit(m, n_experts);
-  route_logits_kernel<<<dim3((unsigned)((n_experts + 15) / 16), (unsigned)((m + 15) / 16), (unsigned)ks), 256, 0,
-                        st>>>(static_cast<const uint16_t *>(hidden), static_cast<const uint16_t *>(gate_weight),
-                              (int)m, (int)d, (int)n_experts, part);
+  const uint16_t *hid = static_cast<const uint16_t *>(hidden), *gw = static_cast<const uint16_t *>(gate_weight);
+  if (m > ROUTE_WIDE_M)
+    route_logits_wide_kernel<<<dim3((unsigned)((n_experts + 63) / 64), (unsigned)((m + 63) / 64), (unsigned)ks), 256, 0,
+                               st>>>(hid, gw, (int)m, (int)d, (int)n_experts, part);
+  else
+    route_logits_kernel<<<dim3((unsigned)((n_experts + 15) / 16), (unsigned)((m + 15) / 16), (unsigned)ks), 256, 0,
+                          st>>>(hid, gw, (int)m, (int)d, (int)n_experts, part);
   int rc;
   if ((rc = check_launch("moe_route logits"))) return rc;
-  route_select_kernel<<<dim3((unsigned)m), 64, 0, st>>>(part, (int)m, ks, (int)n_experts, n_group, topk_group, top_k,
-                                                        norm_topk_prob, indices, weights);
+  const auto select = n_experts <= 256 ? route_select_kernel<4> : route_select_kernel<ROUTE_MAX_E / 64>;
+  select<<<dim3((unsigned)m), 64, 0, st>>>(part, (int)m, ks, (int)n_experts, n_group, topk_group, top_k, norm_topk_prob,
+                                           indices, weights);
   return check_launch("moe_route select");
 }
 
@@ -446,6 +565,15 @@ int amla_moe_combine(const void *shared_out, const void *expert_out, const float
   if (m < 0 || top_k <= 0 || d <= 0) return fail(AMLA_EINVAL, "moe_combine: bad sizes");
   if (m == 0) return AMLA_OK;
   if (m > 65535) return fail(AMLA_EUNSUPPORTED, "moe_combine: at most 65535 tokens per call");
+  if (d % 8 == 0 && d / 8 <= INT32_MAX && aligned16(shared_out) && aligned16(expert_out) && aligned16(out)) {
+    const int64_t items = m * (d / 8), blocks = (items + 255) / 256;
+    if (blocks <= INT32_MAX) {
+      moe_combine8_kernel<<<dim3((unsigned)blocks), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+          static_cast<const uint16_t *>(shared_out), static_cast<const uint16_t *>(expert_out), weights, top_k,
+          (int)(d / 8), items, routed_scaling_factor, static_cast<uint16_t *>(out));
+      return check_launch("moe_combine");
+    }
+  }
   const unsigned bx = (unsigned)std::min<int64_t>((d + 255) / 256, 64);
   moe_combine_kernel<<<dim3(bx, (unsigned)m), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t *>(shared_out), static_cast<const uint16_t *>(expert_out), weights, top_k, d,
