@@ -123,7 +123,6 @@ struct MoeSched {
   int E;
   int down;               // 0: [gate | up] as two weight segments (n_split = gate rows), 1: down
   const int32_t *rowmap;  // gather (down = 0) or scatter (down = 1)
-  bool part_by_entry;     // skinny K-part sums of entry g at row 16 g, else at row (first position)
 };
 AMLA_DEV void moe_sched_weights(GemvParams &p, const MoeSched &s, int e) {
   const void *const *t = s.wtab + (s.down ? 4 : 0) * s.E;
@@ -134,8 +133,8 @@ AMLA_DEV void moe_sched_weights(GemvParams &p, const MoeSched &s, int e) {
 }
 // Skinny GEMMs of the scheduled entries, each with at most 16 rows; grid
 // max_entries x plan.groups.  plan: plan_gemv_grouped(16 or less, N, K);
-// p.part holds plan.kparts * rows * N fp32 when kparts > 1 (rows: 16 per entry
-// or every position, MoeSched::part_by_entry).  down = 0: p.x hidden, p.y the
+// p.part holds plan.kparts * positions * N fp32 when kparts > 1 (an entry at
+// position r0 uses part + kparts * r0 * N).  down = 0: p.x hidden, p.y the
 // [gate | up] rows by position (used with one K part only), h the silu(gate) *
 // up rows; down = 1: p.x h, p.y expert_out, h unused.
 int launch_gemv_sched(const GemvParams &p, const MoeSched &s, int max_entries, int max_m, const GemvPlan &plan,

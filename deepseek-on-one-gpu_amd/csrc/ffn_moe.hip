@@ -842,43 +842,40 @@ constexpr int MSORT_MAXE = 512;     // experts per layer
 constexpr int MSORT_EBITS = 9;      // bits of an expert index
 constexpr int MOE_DEV_MAX_SLOTS = 65536;
 struct MoeDevLayout {
-  bool has_tiles;            // groups of more than MOE_SKINNY_ROWS rows take the large tiles
-  int skinny_rows;           // rows of the largest skinny entry
-  int max_small, max_tiles;  // schedule entries (worst case)
-  bool part_by_entry;        // K-part sums at 16 rows per skinny entry, else at the entry's position
-  size_t hdr, cls, gather, scatter, small, tiles, gu, h, part, total;
+  bool tiles;       // groups on the large tiles, else on the skinny GEMM
+  int rows;         // rows of the largest schedule entry
+  int max_entries;  // schedule entries (worst case)
+  size_t hdr, count, gather, scatter, ent, gu, h, part, total;
 };
 
 static MoeDevLayout moe_dev_layout(int64_t m, int64_t d, int top_k, int64_t n, int64_t E) {
   MoeDevLayout L;
   const int64_t S = m * top_k;
-  // Groups of up to 16 rows (decode) stream through the skinny GEMM, larger
-  // ones through tiles of up to 128 rows.  A token names an expert once in a
-  // routing, so m <= 16 tokens make no group above m; should a caller repeat
-  // an index there, the group is cut into skinny entries of m rows, and the
-  // tile launches (4.6 us each, empty) are left out.
-  L.has_tiles = m > MOE_SKINNY_ROWS;
-  L.skinny_rows = (int)std::min<int64_t>(m, MOE_SKINNY_ROWS);
-  L.max_small = (int)std::min<int64_t>(S, std::min<int64_t>(E, S) + (L.has_tiles ? 0 : S / L.skinny_rows));
-  L.max_tiles = L.has_tiles ? (int)(S / TILE_ROWS + std::min<int64_t>(E, S / (MOE_SKINNY_ROWS + 1))) : 0;
+  // Up to 32 tokens the groups (1-2 rows per expert) stream through the skinny
+  // GEMM, above that through the large tiles.  [gate | up] + down with their
+  // passes at R1 shapes, skinny against tiles: 3 tokens 185 / 214 us, 8 tokens
+  // 443 / 472, 16 tokens 754 / 788, 40 tokens 1376 / 1377, 128 tokens 2091 /
+  // 1885, 300 tokens 2343 / 1936.  Longer groups are cut into entries.
+  L.tiles = m > 32;
+  L.rows = L.tiles ? TILE_ROWS : (int)std::min<int64_t>(m, MOE_SKINNY_ROWS);
+  L.max_entries = (int)std::min<int64_t>(S, std::min<int64_t>(E, S) + S / L.rows);
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align_up(off + bytes, 256); return o; };
   L.hdr = take(16);
-  L.cls = take(8);
+  L.count = take(4);
   L.gather = take((size_t)S * 4);
   L.scatter = take((size_t)S * 4);
-  L.small = take((size_t)L.max_small * 16);
-  L.tiles = take((size_t)std::max(L.max_tiles, 1) * 16);
+  L.ent = take((size_t)L.max_entries * 16);
   L.h = take((size_t)S * n * 2);
-  // [gate | up] rows (one K part) or K-part sums of the skinny entries
-  const GemvPlan a = plan_gemv_grouped(MOE_SKINNY_ROWS, (int)(2 * n), (int)d),
-                 b = plan_gemv_grouped(MOE_SKINNY_ROWS, (int)d, (int)n);
-  L.gu = take(a.kparts > 1 ? 16 : (size_t)S * 2 * n * 2);
-  L.part_by_entry = S > (int64_t)MOE_SKINNY_ROWS * L.max_small;
-  const size_t rows = L.part_by_entry ? (size_t)MOE_SKINNY_ROWS * L.max_small : (size_t)S;
-  const size_t pa = a.kparts > 1 ? a.kparts * rows * 2 * n * 4 : 0;
-  const size_t pb = b.kparts > 1 ? b.kparts * rows * d * 4 : 0;
-  L.part = take(std::max<size_t>(std::max(pa, pb), 16));
+  // skinny GEMM: [gate | up] rows (one K part) or K-part sums
+  L.gu = L.part = off;
+  if (!L.tiles) {
+    const GemvPlan a = plan_gemv_grouped(L.rows, (int)(2 * n), (int)d), b = plan_gemv_grouped(L.rows, (int)d, (int)n);
+    L.gu = take(a.kparts > 1 ? 16 : (size_t)S * 2 * n * 2);
+    const size_t pa = a.kparts > 1 ? (size_t)a.kparts * S * 2 * n * 4 : 0;
+    const size_t pb = b.kparts > 1 ? (size_t)b.kparts * S * d * 4 : 0;
+    L.part = take(std::max<size_t>(std::max(pa, pb), 16));
+  }
   // never below the size callers could count on before the rows were gathered in place
   L.total = std::max(off, (size_t)S * (2 * d + 3 * n) * 2);
   return L;
@@ -904,23 +901,21 @@ AMLA_DEV int block_scan_incl(int v, int *wsum, int lane, int wave) {
 // position (rank among equal experts of the 64-slot step by ballots), so the
 // order is slot order within each expert whatever the timing.  Outputs:
 //   gather[p] = token of position p, scatter[p] = slot of position p;
-//   small[]   = (expert, first position, rows <= sr) of groups of up to sr
-//               slots (of every group, cut at sr, without has_tiles);
-//   tiles[]   = (expert, first position, rows <= 128) of the larger groups;
-//   cls       = {small entries, tile entries};
+//   ent[]     = (expert, first position, rows <= rows_max) of every group,
+//               cut at rows_max;
+//   count     = entries;
 //   hdr       = {routed slots, groups of 1 .. sb slots, 256-row tiles of the
 //               larger groups, skipped slots}, sb = min(tokens, 64).
 // Slots with a negative index are left out; an index >= E, or an expert with a
 // null or misaligned weight, is left out and counted as skipped.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const int64_t *__restrict__ idx, int S, int top_k, int E,
-                                                        int sb, int sr, bool has_tiles,
-                                                        const void *const *__restrict__ wtab,
-                                                        int32_t *__restrict__ hdr, int32_t *__restrict__ cls,
+                                                        int sb, int rows_max, const void *const *__restrict__ wtab,
+                                                        int32_t *__restrict__ hdr, int32_t *__restrict__ count,
                                                         int32_t *__restrict__ gather, int32_t *__restrict__ scatter,
-                                                        int32_t *__restrict__ small, int32_t *__restrict__ tiles) {
+                                                        int32_t *__restrict__ ent) {
   __shared__ int32_t cur[MSORT_WAVES][MSORT_MAXE];  // per-wave counts, then per-wave next positions
   __shared__ int32_t eok[MSORT_MAXE];
-  __shared__ int32_t wsum[3][MSORT_WAVES];
+  __shared__ int32_t wsum[2][MSORT_WAVES];
   __shared__ int32_t skipped, groups, tiles256;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < MSORT_WAVES * MSORT_MAXE; i += 1024) (&cur[0][0])[i] = 0;
@@ -961,26 +956,21 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int64_t *__restric
   }
   if (tot > sb) atomicAdd(&tiles256, (tot + 255) / 256);
   else if (tot > 0) atomicAdd(&groups, 1);
-  const bool big = has_tiles && tot > sr;
-  const int nsmall = big ? 0 : (tot + sr - 1) / sr;
-  const int ntile = big ? (tot + TILE_ROWS - 1) / TILE_ROWS : 0;
+  const int nent = (tot + rows_max - 1) / rows_max;
   const int pos_incl = block_scan_incl(tot, wsum[0], lane, wave);
-  const int small_incl = block_scan_incl(nsmall, wsum[1], lane, wave);
-  const int tile_incl = block_scan_incl(ntile, wsum[2], lane, wave);
+  const int ent_incl = block_scan_incl(nent, wsum[1], lane, wave);
   const int first = pos_incl - tot;
   if (tid < E) {
 #pragma unroll
     for (int w = 0; w < MSORT_WAVES; ++w) cur[w][tid] += first;
-    const int rows = big ? TILE_ROWS : sr;
-    int32_t *en = big ? tiles + 4 * (tile_incl - ntile) : small + 4 * (small_incl - nsmall);
-    for (int j = 0; j < nsmall + ntile; ++j, en += 4) {
-      en[0] = tid; en[1] = first + j * rows; en[2] = min(rows, tot - j * rows); en[3] = 0;
+    int32_t *en = ent + 4 * (ent_incl - nent);
+    for (int j = 0; j < nent; ++j, en += 4) {
+      en[0] = tid; en[1] = first + j * rows_max; en[2] = min(rows_max, tot - j * rows_max); en[3] = 0;
     }
   }
   if (tid == 1023) {
     hdr[0] = pos_incl;
-    cls[0] = small_incl;
-    cls[1] = tile_incl;
+    *count = ent_incl;
   }
   __syncthreads();
   if (tid == 0) {
@@ -1044,7 +1034,7 @@ int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, co
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   int32_t *hdr = reinterpret_cast<int32_t *>(ws + L.hdr);
   int32_t *gather = reinterpret_cast<int32_t *>(ws + L.gather), *scatter = reinterpret_cast<int32_t *>(ws + L.scatter);
-  int32_t *small = reinterpret_cast<int32_t *>(ws + L.small), *tiles = reinterpret_cast<int32_t *>(ws + L.tiles);
+  int32_t *ent = reinterpret_cast<int32_t *>(ws + L.ent), *count = reinterpret_cast<int32_t *>(ws + L.count);
   uint16_t *gu = reinterpret_cast<uint16_t *>(ws + L.gu), *hb = reinterpret_cast<uint16_t *>(ws + L.h);
   float *part = reinterpret_cast<float *>(ws + L.part);
   const uint16_t *hid = static_cast<const uint16_t *>(hidden);
@@ -1052,29 +1042,25 @@ int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, co
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int S = (int)(m * top_k), n = (int)n_inter, D = (int)d, E = (int)n_experts;
   int rc;
-  int32_t *cls = reinterpret_cast<int32_t *>(ws + L.cls);
-  moe_sort_kernel<<<1, 1024, 0, st>>>(indices, S, top_k, E, (int)std::min<int64_t>(m, 64), L.skinny_rows, L.has_tiles,
-                                      weight_table, hdr, cls, gather, scatter, small, tiles);
+  moe_sort_kernel<<<1, 1024, 0, st>>>(indices, S, top_k, E, (int)std::min<int64_t>(m, 64), L.rows, weight_table, hdr,
+                                      count, gather, scatter, ent);
   if ((rc = check_launch("moe_experts_dev schedule"))) return rc;
-  const MoeSched small_gu = {weight_table, small, cls, E, 0, gather, L.part_by_entry},
-                 small_dn = {weight_table, small, cls, E, 1, scatter, L.part_by_entry};
-  const MoeSched tiles_gu = {weight_table, tiles, cls + 1, E, 0, gather, false},
-                 tiles_dn = {weight_table, tiles, cls + 1, E, 1, scatter, false};
-  const int sm = L.skinny_rows;
-  // h rows (by position) = silu(gate) * up of hidden rows gather[]
+  // h rows (by position) = silu(gate) * up of hidden rows gather[], then
+  // expert_out rows scatter[] = down(h)
+  const MoeSched gu_s = {weight_table, ent, count, E, 0, gather}, dn_s = {weight_table, ent, count, E, 1, scatter};
+  if (L.tiles) {
+    const MoeTileParams tg = {hid, hb, D, n, D, n, 0}, td = {hb, eout, n, D, n, D, 0};
+    if ((rc = launch_tile_sched(tg, gu_s, L.max_entries, st))) return rc;
+    return launch_tile_sched(td, dn_s, L.max_entries, st);
+  }
   GemvParams pg = {};
   pg.x = hid; pg.ldx = D; pg.N = 2 * n; pg.K = D; pg.n_split = n; pg.y = gu; pg.ldy = 2 * n; pg.seq_len = 1;
   pg.part = part;
-  const MoeTileParams tg = {hid, hb, D, n, D, n, 0};
-  if ((rc = launch_tile_sched(tg, tiles_gu, L.max_tiles, st))) return rc;
-  if ((rc = launch_gemv_sched(pg, small_gu, L.max_small, sm, plan_gemv_grouped(sm, 2 * n, D), hb, st))) return rc;
-  // expert_out rows scatter[] = down(h)
+  if ((rc = launch_gemv_sched(pg, gu_s, L.max_entries, L.rows, plan_gemv_grouped(L.rows, 2 * n, D), hb, st))) return rc;
   GemvParams pd = {};
   pd.x = hb; pd.ldx = n; pd.N = D; pd.K = n; pd.n_split = D; pd.y = eout; pd.ldy = D; pd.seq_len = 1;
   pd.part = part;
-  const MoeTileParams td = {hb, eout, n, D, n, D, 0};
-  if ((rc = launch_tile_sched(td, tiles_dn, L.max_tiles, st))) return rc;
-  return launch_gemv_sched(pd, small_dn, L.max_small, sm, plan_gemv_grouped(sm, D, n), nullptr, st);
+  return launch_gemv_sched(pd, dn_s, L.max_entries, L.rows, plan_gemv_grouped(L.rows, D, n), nullptr, st);
 }
 
 }  // extern "C"

@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256, 2) void gemv_sched_kernel(GemvParams p, MoeSch
   p.M = en[2];
   if (s.down) p.x += (size_t)r0 * p.ldx;
   else p.y += (size_t)r0 * p.ldy;
-  p.part += (size_t)kparts * (s.part_by_entry ? 16 * g : r0) * p.N;
+  p.part += (size_t)kparts * r0 * p.N;
   moe_sched_weights(p, s, e);
   gemv_body<1, GEMV_PLAIN, true>(p, blockIdx.x % units, rg, kparts, kpb, s.down ? nullptr : s.rowmap + r0,
                                  s.down ? s.rowmap + r0 : nullptr);
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(64) void gemv_finish_sched(GemvParams p, MoeSched s
   const int32_t *en = s.ent + 4 * g;
   const int r0 = en[1];
   p.M = en[2];
-  p.part += (size_t)kparts * (s.part_by_entry ? 16 * g : r0) * p.N;
+  p.part += (size_t)kparts * r0 * p.N;
   gemv_finish_body<GEMV_PLAIN>(p, (int64_t)(blockIdx.x % units) * 64 + threadIdx.x, kparts, s.rowmap + r0);
 }
 
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(64) void gu_silu_sched_kernel(GemvParams p, MoeSche
   const int m = (int)(i / (n >> 2)), j = (int)(i % (n >> 2)) * 4;
   float gv[4], uv[4];
   if (kparts > 1) {
-    const float *part = p.part + (size_t)kparts * (s.part_by_entry ? 16 * g : r0) * p.N;
+    const float *part = p.part + (size_t)kparts * r0 * p.N;
     f32x4 gq[GEMV_MAX_PARTS], uq[GEMV_MAX_PARTS];
 #pragma unroll
     for (int q = 0; q < GEMV_MAX_PARTS; ++q)

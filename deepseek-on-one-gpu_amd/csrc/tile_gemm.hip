@@ -20,13 +20,12 @@ namespace amla {
 //
 // What bounds it: with few rows per expert the weight stream from HBM (64 rows
 // are 128 FLOP per weight byte), above about 128 rows the MFMAs.  MI355X, 256
-// R1 experts, 2000 tokens x 8 (62 rows per expert on average): [gate | up] with
-// silu * up 1.66 ms (5.0 TB/s of the 8.3 GB it fetches), down 0.89 ms, against
-// 2.72 + 0.03 and 1.49 ms for a 256 x 256 tile GEMM for groups above 64 rows
-// beside a skinny GEMM with fp32 K parts for the others; 8000 tokens (250 rows
-// per expert) 4.8 + 2.4 ms against 5.4 + 0.1 and 2.8.  Gathering and scattering
-// the rows here saved two more passes (0.14 ms at 2000 tokens).  Groups of up
-// to 16 rows stay on the skinny GEMM (gemv_sched_kernel, 6.5 TB/s at 8 tokens).
+// R1 experts, top 8: 300 tokens (9 rows per expert) [gate | up] with silu * up
+// 1.28 ms (5.9 TB/s), down 0.66 ms, where the skinny GEMM with fp32 K parts and
+// finishing passes took 1.55 + 0.82 ms; 2000 tokens (62 rows) 1.66 + 0.89 ms
+// against 2.75 + 1.62 for that and 256 x 256 tiles for groups above 64 rows;
+// 8000 tokens (250 rows) 4.8 + 2.4 ms against 5.6 + 2.9.  Gathering and
+// scattering the rows here saved two more passes (0.14 ms at 2000 tokens).
 //
 // K stages of 64 in LDS: fp8 weight rows (64 B, chunk c of row r at
 // c ^ ((r >> 2) & 3)), bf16 activation rows (128 B, chunk c of row r at
