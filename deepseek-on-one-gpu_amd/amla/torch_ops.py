@@ -61,7 +61,7 @@ def _linear(x: Tensor, weight: Tensor, scale_inv: Tensor, f32: bool) -> Tensor:
     if m == 0:
         return y
     L = lib()
-    need = L.amla_fp8_linear_workspace_bytes(m, n, k) if m <= 64 else 0
+    need = L.amla_fp8_linear_workspace_bytes(m, n, k)
     ws = _scratch(x.device, need) if need else None
     fn = L.amla_fp8_linear_f32 if f32 else L.amla_fp8_linear
     check(fn(x.data_ptr(), m, k, x.stride(0), weight.data_ptr(), scale_inv.data_ptr(), n, y.data_ptr(), n,

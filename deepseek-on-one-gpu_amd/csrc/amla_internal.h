@@ -25,6 +25,7 @@ enum GemvMode : int {
   GEMV_QKVA = 2,   // rows < n_split -> y; the rest -> latent / rope-key cache rows
   GEMV_QROPE = 3,  // y = bf16(acc); rows with (n % head_dim) >= nope rotated by RoPE at pos(m)
   GEMV_F32 = 4,    // y[m, n] = acc as fp32 (y is a float buffer, ldy counted in floats)
+  GEMV_SILU = 5,   // launch_gemm only: w0, w1 two (N, K) weights, y[m, n] = bf16(bf16(silu(w0 row)) * w1 row)
 };
 
 struct GemvParams {
@@ -164,21 +165,23 @@ struct TileGroups {
 };
 int launch_tile_grouped(const MoeTileParams &p, const TileGroups &groups, bool down, hipStream_t stream);
 // Large-M fp8 GEMM with the same modes (M > 64).  With split_ws of at least
-// gemm_ws_bytes(M, N, K) bytes, tiles past the last full round of 256
+// gemm_ws_bytes(M, N, K) bytes, tiles past the last full round of 512
 // workgroups are cut into K parts (fp32 partial sums in split_ws, summed in
 // part order by a finishing kernel); without it every tile takes the whole K.
 constexpr int GEMV_MAX_PARTS = 32;  // K parts of the skinny GEMM (summed by its finishing passes)
-constexpr int GEMM_MAX_PARTS = 8;
+constexpr int GEMM_MAX_PARTS = 16;
+constexpr int TILE_PART_F32 = 256 * 128;  // fp32 partial sums of one tile
 struct GemmSplit {
-  int full;        // tiles with the whole K
-  int parts;       // K parts of each later tile
-  int n_tiles;     // 256-column tiles
-  int items;       // workgroups
-  float *partial;  // [split tile][part][256 x 256] fp32 in the workgroup's lane order
-  size_t bytes;    // of partial
+  int n_tiles, m_tiles;  // tiles of 256 columns (SILU: 128) x 128 rows
+  int full;              // tiles with the whole K
+  int rest;              // later tiles, cut into
+  int parts;             // K parts each
+  int full_blocks;       // workgroups before the parts
+  float *partial;        // [split tile][part][TILE_PART_F32] in the lanes' own order
+  size_t bytes;          // of partial
 };
-GemmSplit plan_gemm_split(int M, int N, int K);
-size_t gemm_ws_bytes(int M, int N, int K);
+GemmSplit plan_gemm_split(int M, int N, int K, int mode);
+size_t gemm_ws_bytes(int M, int N, int K, int mode = GEMV_PLAIN);
 int launch_gemm(const GemvParams &p, int mode, hipStream_t stream, float *split_ws = nullptr,
                 size_t split_ws_bytes = 0);
 

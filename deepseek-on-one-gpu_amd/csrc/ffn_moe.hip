@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void silu_mul_rows_kernel(const uint16_t *__re
 
 // One fp8 linear (y = bf16(x W^T)), skinny or large-M path.
 static int fp8_linear_into(const uint16_t *x, int m, int k, const uint8_t *w, const float *s, int n, uint16_t *y,
-                           float *part, hipStream_t st) {
+                           float *part, size_t part_bytes, hipStream_t st) {
   GemvParams p = {};
   p.x = x;
   p.M = m;
@@ -119,29 +119,31 @@ static int fp8_linear_into(const uint16_t *x, int m, int k, const uint8_t *w, co
   p.y = y;
   p.ldy = n;
   p.seq_len = 1;
-  if (m > 64) return launch_gemm(p, GEMV_PLAIN, st);
+  if (m > 64) return launch_gemm(p, GEMV_PLAIN, st, part, part_bytes);
   const GemvPlan pl = plan_linear(m, n, k);
   p.part = part;
   return launch_gemv(p, GEMV_PLAIN, pl, st);
 }
 
 struct SwigluLayout {
-  size_t gu, h, part, total;
+  size_t gu, h, part, part_bytes, total;
 };
 
-// [gate | up] rows (m, 2n), then h (m, n), then the K-part sums of the skinny path
+// [gate | up] rows (m, 2n) (skinny path), then h (m, n), then the K-part sums
 static SwigluLayout swiglu_layout(int64_t m, int64_t k, int64_t n) {
   SwigluLayout L;
   size_t off = 0;
   L.gu = off;
-  off = align_up(off + (size_t)m * 2 * n * 2, 256);
+  if (m <= 64) off = align_up(off + (size_t)m * 2 * n * 2, 256);
   L.h = off;
   off = align_up(off + (size_t)m * n * 2, 256);
-  size_t part = 0;
-  if (m <= 64 && m > 0)
-    part = std::max(plan_linear((int)m, (int)(2 * n), (int)k).part_bytes, plan_linear((int)m, (int)k, (int)n).part_bytes);
+  if (m <= 64)
+    L.part_bytes =
+        std::max(plan_linear((int)m, (int)(2 * n), (int)k).part_bytes, plan_linear((int)m, (int)k, (int)n).part_bytes);
+  else
+    L.part_bytes = std::max(gemm_ws_bytes((int)m, (int)n, (int)k, GEMV_SILU), gemm_ws_bytes((int)m, (int)k, (int)n));
   L.part = off;
-  off = align_up(off + part, 256);
+  off = align_up(off + L.part_bytes, 256);
   L.total = off;
   return L;
 }
@@ -161,7 +163,7 @@ int amla_silu_mul(const void *gate, const void *up, int64_t numel, void *out, vo
 }
 
 size_t amla_swiglu_workspace_bytes(int64_t m, int64_t k, int64_t n) {
-  if (m <= 0 || k <= 0 || n <= 0) return 0;
+  if (m <= 0 || k <= 0 || n <= 0 || m > INT32_MAX || k > INT32_MAX || n > INT32_MAX) return 0;
   return swiglu_layout(m, k, n).total;
 }
 
@@ -190,6 +192,25 @@ int amla_swiglu(const void *x, int64_t m, int64_t k, const void *gate_w, const f
   float *part = reinterpret_cast<float *>(ws + L.part);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   int rc;
+  if (m > 64) {
+    // silu(gate) * up in the epilogue of one GEMM over both weights
+    GemvParams p = {};
+    p.x = static_cast<const uint16_t *>(x);
+    p.M = (int)m;
+    p.ldx = (int)k;
+    p.w0 = static_cast<const uint8_t *>(gate_w);
+    p.s0 = gate_s;
+    p.w1 = static_cast<const uint8_t *>(up_w);
+    p.s1 = up_s;
+    p.N = (int)n;
+    p.K = (int)k;
+    p.y = h;
+    p.ldy = (int)n;
+    p.seq_len = 1;
+    if ((rc = launch_gemm(p, GEMV_SILU, st, part, L.part_bytes))) return rc;
+    return fp8_linear_into(h, (int)m, (int)n, static_cast<const uint8_t *>(down_w), down_s, (int)k,
+                           static_cast<uint16_t *>(y), part, L.part_bytes, st);
+  }
   // gate and up as one GEMM over the two stacked weights: rows (m, [gate | up])
   GemvParams p = {};
   p.x = static_cast<const uint16_t *>(x);
@@ -206,41 +227,24 @@ int amla_swiglu(const void *x, int64_t m, int64_t k, const void *gate_w, const f
   p.ldy = (int)(2 * n);
   p.seq_len = 1;
   p.part = part;
-  if (m > 64 && n % 256 == 0) rc = launch_gemm(p, GEMV_PLAIN, st);
-  else if (m > 64) {
-    // the large-M GEMM tiles 256 rows: a 128-row split point takes two launches
-    GemvParams a = p, b = p;
-    a.w1 = nullptr;
-    a.N = (int)n;
-    a.n_split = (int)n;
-    b.w0 = p.w1;
-    b.s0 = p.s1;
-    b.w1 = nullptr;
-    b.N = (int)n;
-    b.n_split = (int)n;
-    b.y = gu + n;
-    rc = launch_gemm(a, GEMV_PLAIN, st);
-    if (!rc) rc = launch_gemm(b, GEMV_PLAIN, st);
-  } else {
-    const GemvPlan pl = plan_linear((int)m, (int)(2 * n), (int)k);
-    if (pl.kparts > 1) {
-      // the K-part finish and silu * up in one pass (n % 128 == 0)
-      if ((rc = launch_gemv(p, GEMV_PLAIN, pl, st, false))) return rc;
-      const int64_t items = m * (n / 4);
-      gu_finish_silu_kernel<<<(unsigned)((items + 63) / 64), 64, 0, st>>>(part, (int)m, (int)n, pl.kparts, h);
-      if ((rc = check_launch("swiglu gate|up finish + silu_mul"))) return rc;
-      return fp8_linear_into(h, (int)m, (int)n, static_cast<const uint8_t *>(down_w), down_s, (int)k,
-                             static_cast<uint16_t *>(y), part, st);
-    }
-    rc = launch_gemv(p, GEMV_PLAIN, pl, st);
+  const GemvPlan pl = plan_linear((int)m, (int)(2 * n), (int)k);
+  if (pl.kparts > 1) {
+    // the K-part finish and silu * up in one pass (n % 128 == 0)
+    if ((rc = launch_gemv(p, GEMV_PLAIN, pl, st, false))) return rc;
+    const int64_t items = m * (n / 4);
+    gu_finish_silu_kernel<<<(unsigned)((items + 63) / 64), 64, 0, st>>>(part, (int)m, (int)n, pl.kparts, h);
+    if ((rc = check_launch("swiglu gate|up finish + silu_mul"))) return rc;
+    return fp8_linear_into(h, (int)m, (int)n, static_cast<const uint8_t *>(down_w), down_s, (int)k,
+                           static_cast<uint16_t *>(y), part, L.part_bytes, st);
   }
+  rc = launch_gemv(p, GEMV_PLAIN, pl, st);
   if (rc) return rc;
   silu_mul_rows_kernel<<<dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(n / 8 / 256, 16)),
                               (unsigned)std::min<int64_t>(m, 65535)),
                          256, 0, st>>>(gu, (int)m, (int)n, h);
   if ((rc = check_launch("swiglu silu_mul"))) return rc;
   return fp8_linear_into(h, (int)m, (int)n, static_cast<const uint8_t *>(down_w), down_s, (int)k,
-                         static_cast<uint16_t *>(y), part, st);
+                         static_cast<uint16_t *>(y), part, L.part_bytes, st);
 }
 
 }  // extern "C"

@@ -2070,7 +2070,8 @@ int amla_fp8_block_dequant(const void *weight, const float *scale_inv, int64_t n
 }
 
 size_t amla_fp8_linear_workspace_bytes(int64_t m, int64_t n, int64_t k) {
-  if (m < 1 || m > 64 || n <= 0 || k <= 0 || n % 16 || k % 128 || n > INT32_MAX || k > INT32_MAX) return 0;
+  if (m < 1 || m > INT32_MAX || n <= 0 || k <= 0 || n % 16 || k % 128 || n > INT32_MAX || k > INT32_MAX) return 0;
+  if (m > 64) return gemm_ws_bytes((int)m, (int)n, (int)k);
   return plan_linear((int)m, (int)n, (int)k).part_bytes;
 }
 
@@ -2100,7 +2101,7 @@ int amla_fp8_linear(const void *x, int64_t m, int64_t k, int64_t ldx, const void
   p.ldy = (int)ldy;
   p.seq_len = 1;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (m > 64) return launch_gemm(p, GEMV_PLAIN, st);
+  if (m > 64) return launch_gemm(p, GEMV_PLAIN, st, static_cast<float *>(workspace), workspace_bytes);
   const GemvPlan pl = plan_linear((int)m, (int)n, (int)k);
   if (pl.part_bytes) {
     if (!workspace || workspace_bytes < pl.part_bytes || !aligned16(workspace))
@@ -2137,7 +2138,7 @@ int amla_fp8_linear_f32(const void *x, int64_t m, int64_t k, int64_t ldx, const 
   p.ldy = (int)ldy;
   p.seq_len = 1;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (m > 64) return launch_gemm(p, GEMV_F32, st);
+  if (m > 64) return launch_gemm(p, GEMV_F32, st, static_cast<float *>(workspace), workspace_bytes);
   const GemvPlan pl = plan_linear((int)m, (int)n, (int)k);
   if (pl.part_bytes) {
     if (!workspace || workspace_bytes < pl.part_bytes || !aligned16(workspace))

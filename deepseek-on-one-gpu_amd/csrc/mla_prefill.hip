@@ -17,472 +17,14 @@
 
 #include "amla_common.h"
 #include "amla_internal.h"
+#include "gemm_epilogue.h"
 
 namespace amla {
-
-// Epilogue shared with the skinny GEMM (fp8_linear.hip); same contract.
-AMLA_DEV int prow_position(const GemvParams &p, int m) { return p.pos[m / p.seq_len] + m % p.seq_len; }
-
-template <int MODE>
-AMLA_DEV void pstore4(const GemvParams &p, int m, int n, f32x4 v) {
-  if (MODE == GEMV_PLAIN) {
-    u32x2 o = {pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
-    *reinterpret_cast<u32x2 *>(p.y + (size_t)m * p.ldy + n) = o;
-  } else if (MODE == GEMV_F32) {
-    *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(p.y) + (size_t)m * p.ldy + n) = v;
-  } else if (MODE == GEMV_RESID) {
-    const u32x2 r = *reinterpret_cast<const u32x2 *>(p.res + (size_t)m * p.ldr + n);
-    u32x2 o = {pack_bf16(lo_bf(r.x) + round_bf16(v.x), hi_bf(r.x) + round_bf16(v.y)),
-               pack_bf16(lo_bf(r.y) + round_bf16(v.z), hi_bf(r.y) + round_bf16(v.w))};
-    *reinterpret_cast<u32x2 *>(p.y + (size_t)m * p.ldy + n) = o;
-  } else if (MODE == GEMV_QKVA) {
-    u32x2 o = {pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
-    if (n < p.n_split) {
-      *reinterpret_cast<u32x2 *>(p.y + (size_t)m * p.ldy + n) = o;
-    } else {
-      const int b = m / p.seq_len;
-      const int64_t row = prow_position(p, m);
-      if (row >= p.max_rows) return;  // a device position past the cache: nothing is written
-      const int nn = n - p.n_split;
-      uint16_t *dst = nn < p.kv_lora ? p.ckv + b * p.ckv_bstride + row * p.kv_lora + nn
-                                     : p.kpe + b * p.kpe_bstride + row * p.rope + (nn - p.kv_lora);
-      *reinterpret_cast<u32x2 *>(dst) = o;
-    }
-  } else {
-    float a0 = round_bf16(v.x), a1 = round_bf16(v.y), a2 = round_bf16(v.z), a3 = round_bf16(v.w);
-    const int d = n % p.head_dim;
-    if (d >= p.nope) {
-      const int i = (d - p.nope) >> 1;
-      const int64_t row = min(prow_position(p, m), p.rope_rows - 1);  // in bounds for any device position
-      const f32x4 cs = *reinterpret_cast<const f32x4 *>(p.rope_table + (row * (p.rope >> 1) + i) * 2);
-      const float r0 = __fsub_rn(__fmul_rn(a0, cs.x), __fmul_rn(a1, cs.y));
-      const float r1 = __fadd_rn(__fmul_rn(a0, cs.y), __fmul_rn(a1, cs.x));
-      const float r2 = __fsub_rn(__fmul_rn(a2, cs.z), __fmul_rn(a3, cs.w));
-      const float r3 = __fadd_rn(__fmul_rn(a2, cs.w), __fmul_rn(a3, cs.z));
-      a0 = r0; a1 = r1; a2 = r2; a3 = r3;
-    }
-    u32x2 o = {pack_bf16(a0, a1), pack_bf16(a2, a3)};
-    *reinterpret_cast<u32x2 *>(p.y + (size_t)m * p.ldy + n) = o;
-  }
-}
-
-// ---------------------------------------------------------------- K3 GEMM
-
-
-// Eight consecutive outputs n .. n+7 (n % 8 == 0) already rounded to bf16.
-template <int MODE>
-AMLA_DEV void pstore8(const GemvParams &p, int m, int n, u32x4 v) {
-  if (MODE == GEMV_F32) {
-    // not reached: fp32 outputs take the unstaged epilogue (launch_gemm)
-  } else if (MODE == GEMV_PLAIN) {
-    *reinterpret_cast<u32x4 *>(p.y + (size_t)m * p.ldy + n) = v;
-  } else if (MODE == GEMV_RESID) {
-    const u32x4 r = *reinterpret_cast<const u32x4 *>(p.res + (size_t)m * p.ldr + n);
-    u32x4 o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = pack_bf16(lo_bf(r[i]) + lo_bf(v[i]), hi_bf(r[i]) + hi_bf(v[i]));
-    *reinterpret_cast<u32x4 *>(p.y + (size_t)m * p.ldy + n) = o;
-  } else if (MODE == GEMV_QKVA) {
-    if (n < p.n_split) {
-      *reinterpret_cast<u32x4 *>(p.y + (size_t)m * p.ldy + n) = v;
-    } else {
-      const int b = m / p.seq_len;
-      const int64_t row = prow_position(p, m);
-      if (row >= p.max_rows) return;  // a device position past the cache: nothing is written
-      const int nn = n - p.n_split;
-      uint16_t *dst = nn < p.kv_lora ? p.ckv + b * p.ckv_bstride + row * p.kv_lora + nn
-                                     : p.kpe + b * p.kpe_bstride + row * p.rope + (nn - p.kv_lora);
-      *reinterpret_cast<u32x4 *>(dst) = v;
-    }
-  } else {
-    const int d = n % p.head_dim;
-    u32x4 o = v;
-    if (d >= p.nope) {
-      const int64_t row = min(prow_position(p, m), p.rope_rows - 1);  // in bounds for any device position
-      const float *tab = p.rope_table + (row * (p.rope >> 1) + ((d - p.nope) >> 1)) * 2;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float a0 = lo_bf(v[i]), a1 = hi_bf(v[i]);
-        const float c = tab[2 * i], s = tab[2 * i + 1];
-        o[i] = pack_bf16(__fsub_rn(__fmul_rn(a0, c), __fmul_rn(a1, s)), __fadd_rn(__fmul_rn(a0, s), __fmul_rn(a1, c)));
-      }
-    }
-    *reinterpret_cast<u32x4 *>(p.y + (size_t)m * p.ldy + n) = o;
-  }
-}
 
 AMLA_DEV f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-
-// Workgroup tile 256 weight rows (n) x 256 activation rows (m), K stage 64,
-// three LDS stages filled by direct global-to-LDS copies: fp8 weight rows
-// (64 B) and bf16 activation rows (128 B), 16-byte chunks swizzled per row
-// (chunk c of weight row r at c ^ ((r >> 2) & 3), of activation row r at
-// c ^ ((r >> 1) & 7)) so that the 16 lanes of each fragment-read group hit
-// distinct banks.  Eight waves (two
-// per SIMD), each 128 (n) x 64 (m) with 32x32x16 MFMAs; weight fragments are
-// converted exactly from fp8 to bf16 in registers.
-//
-// Block scales: a wave's 128 weight rows are one scale block, so the scale of
-// a 128-wide K block is one number s_kb for the whole wave tile.  The
-// accumulator is kept in units of the current block's scale: entering block
-// kb it is multiplied by s_{kb-1} / s_kb, and the result is acc * s_last.
-// This equals sum_kb s_kb * partial_kb up to fp32 rounding of the ratios
-// (~1e-5 relative over 128 blocks, far below the bf16 output rounding).  A
-// block with s_kb == 0 dequantises to zero and is skipped.
-constexpr int G_BN = 256, G_BM = 256, G_BK = 64, G_NST = 3, G_NW = 8;
-constexpr int G_WOFF = 0, G_XOFF = G_BN * G_BK;  // fp8 weight rows, then bf16 activation rows
-constexpr int G_STAGE = G_BN * G_BK + G_BM * G_BK * 2;
-constexpr int G_LDS = G_NST * G_STAGE;           // 144 KB
-constexpr int G_DMA = G_STAGE / 1024 / G_NW;     // copies per wave per stage
-constexpr int G_EPITCH = 128 * 2 + 8;           // LDS row pitch of the staged output block
-constexpr int G_WAVE_F4 = 4 * 2 * 4 * 64;        // f32x4 partial sums of one wave's 128 x 64 block
-constexpr int G_TILE_F4 = G_NW * G_WAVE_F4;      // ... of one 256 x 256 tile (256 KB)
-static_assert(G_NW * 64 * G_EPITCH <= G_LDS, "staged output block exceeds LDS");
-
-// One 256 x 256 output tile at (n0, m0) over the 128-wide K blocks
-// [kb_begin, kb_end).  partial != nullptr: the tile's fp32 sums (scaled) go to
-// partial in the lanes' own order (gemm_finish_kernel sums the K parts),
-// else through the epilogue.
-template <int MODE>
-AMLA_DEV void gemm_body(const GemvParams &p, bool staged_out, const int n0, const int m0, const int kb_begin,
-                        const int kb_end, float *partial) {
-  extern __shared__ __align__(16) uint8_t gsm[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wn = wave & 1, wm = wave >> 1;
-  const int j32 = lane & 31, hh = lane >> 5;
-  const bool seg1 = (MODE == GEMV_QKVA || p.w1) && n0 >= p.n_split;
-  const uint8_t *W = seg1 ? p.w1 : p.w0;
-  const float *S = seg1 ? p.s1 : p.s0;
-  const int nl0 = seg1 ? n0 - p.n_split : n0;
-  const int nvalid = (seg1 ? p.N - p.n_split : p.n_split) - nl0;  // rows of this segment from nl0
-  const int KB = p.K >> 7;
-  const bool wave_rows = wn * 128 < nvalid;
-  const __attribute__((address_space(4))) float *srow = (const __attribute__((address_space(4))) float *)(
-      S + (size_t)((nl0 + min(wn * 128, nvalid - 1)) >> 7) * KB);
-
-  // copies: wave w fills weight rows 32w .. +31 (two copies of 16 rows) and
-  // activation rows 32w .. +31 (four copies of 8 rows) of each stage
-  const bool wfull = nvalid >= G_BN, xfull = m0 + G_BM <= p.M;
-  const uint32_t wrow = (uint32_t)(lane >> 2) * p.K, xrow = (uint32_t)(lane >> 3) * p.ldx * 2;
-  auto dma = [&](int it, uint8_t *st) {
-    const int k0 = it * G_BK;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int r0 = 32 * wave + 16 * j;
-      const uint8_t *src;
-      if (wfull) {
-        src = W + (size_t)(nl0 + r0) * p.K + k0 + wrow + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
-      } else {
-        const int r = min(r0 + (lane >> 2), nvalid - 1);
-        src = W + (size_t)(nl0 + r) * p.K + k0 + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
-      }
-      __builtin_amdgcn_global_load_lds(src, LDS_PTR(st + G_WOFF + r0 * G_BK), 16, 0, 0);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r0 = 32 * wave + 8 * j;
-      const uint8_t *src;
-      if (xfull) {
-        src = reinterpret_cast<const uint8_t *>(p.x + (size_t)(m0 + r0) * p.ldx + k0) + xrow +
-              16 * ((lane & 7) ^ ((4 * j + (lane >> 4)) & 7));
-      } else {
-        const int r = min(m0 + r0 + (lane >> 3), p.M - 1);
-        src = reinterpret_cast<const uint8_t *>(p.x + (size_t)r * p.ldx + k0) +
-              16 * ((lane & 7) ^ ((4 * j + (lane >> 4)) & 7));
-      }
-      __builtin_amdgcn_global_load_lds(src, LDS_PTR(st + G_XOFF + r0 * (G_BK * 2)), 16, 0, 0);
-    }
-  };
-
-  // fragment offsets: weight rows wn*128 + 32 g + j32, chunk (2 pr + hh) of
-  // the 64-byte row (K 32 pr + 16 hh .. +15, two MFMA steps of 8); activation
-  // rows wm*64 + 32 j + j32, chunks 4 pr + 2 hh + s (K 32 pr + 16 hh + 8 s ..)
-  uint32_t aoff[2], boff[2][2];
-#pragma unroll
-  for (int pr = 0; pr < 2; ++pr) {
-    aoff[pr] = G_WOFF + (wn * 128 + j32) * G_BK + 16 * ((2 * pr + hh) ^ ((j32 >> 2) & 3));
-#pragma unroll
-    for (int st = 0; st < 2; ++st)
-      boff[pr][st] = G_XOFF + (wm * 64 + j32) * (G_BK * 2) + 16 * ((4 * pr + 2 * hh + st) ^ ((j32 >> 1) & 7));
-  }
-
-  f32x16 acc[4][2];
-#pragma unroll
-  for (int g = 0; g < 4; ++g)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[g][j][r] = 0.f;
-  float s_run = 0.f;
-  bool skip = false;
-
-  const int iters = 2 * kb_end;  // 64-wide K stages, two per scale block
-  dma(2 * kb_begin, gsm);
-  if (2 * kb_begin + 1 < iters) dma(2 * kb_begin + 1, gsm + G_STAGE);
-  int stg = 0;
-  for (int it = 2 * kb_begin; it < iters; ++it) {
-    if (it + 1 < iters) wait_vmcnt<G_DMA>();
-    else wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (it + 2 < iters) dma(it + 2, gsm + (stg == 0 ? 2 : stg - 1) * G_STAGE);
-    if ((it & 1) == 0) {
-      const float sk = srow[it >> 1];
-      skip = sk == 0.f;
-      if (!skip) {
-        if (s_run != 0.f) {
-          const float r = __fdiv_rn(s_run, sk);
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[g][j] *= r;
-        }
-        s_run = sk;
-      }
-    }
-    if (!skip) {
-      const uint8_t *st = gsm + stg * G_STAGE;
-#pragma unroll
-      for (int pr = 0; pr < 2; ++pr) {
-        u32x4 araw[4], bx[2][2];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) araw[g] = *reinterpret_cast<const u32x4 *>(st + aoff[pr] + g * 32 * G_BK);
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2)
-            bx[j][s2] = *reinterpret_cast<const u32x4 *>(st + boff[pr][s2] + j * 32 * (G_BK * 2));
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-            const uint32_t w0 = araw[g][2 * s2], w1 = araw[g][2 * s2 + 1];
-            const bf16x2_t c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, false);
-            const bf16x2_t c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, true);
-            const bf16x2_t c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, false);
-            const bf16x2_t c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, true);
-            const bf16x8 a = {c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[g][j] = mfma32(a, as_bf16x8(bx[j][s2]), acc[g][j]);
-          }
-      }
-    }
-    stg = stg == G_NST - 1 ? 0 : stg + 1;
-  }
-
-  // C[n][m]: lane holds m = 32 j + j32 of its rows, n = 32 g + 8 q + 4 hh .. +3.
-  if (partial) {
-    // [wave][g][j][q][lane] f32x4: every store is 1 KB contiguous per wave
-    f32x4 *dst = reinterpret_cast<f32x4 *>(partial) + (size_t)wave * G_WAVE_F4;
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          dst[((g * 2 + j) * 4 + q) * 64 + lane] =
-              f32x4{acc[g][j][4 * q], acc[g][j][4 * q + 1], acc[g][j][4 * q + 2], acc[g][j][4 * q + 3]} * s_run;
-    return;
-  }
-  if (!staged_out) {
-    // outputs without 16-byte aligned rows: 8-byte stores straight from the accumulators
-    if (wave_rows) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int m = m0 + wm * 64 + 32 * j + j32;
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int n = n0 + wn * 128 + 32 * g + 8 * q + 4 * hh;
-            if (n < p.N)
-              pstore4<MODE>(p, m, n,
-                            f32x4{acc[g][j][4 * q], acc[g][j][4 * q + 1], acc[g][j][4 * q + 2], acc[g][j][4 * q + 3]} *
-                                s_run);
-          }
-      }
-    }
-    return;
-  }
-  // bf16(C * s) goes through LDS (this wave's 64 x 128 block, rows of m) so
-  // that every global store is 16 bytes of one output row.
-  __builtin_amdgcn_s_barrier();  // every wave is past its last fragment read
-  asm volatile("" ::: "memory");
-  uint8_t *cst = gsm + wave * (64 * G_EPITCH);
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x4 v =
-            f32x4{acc[g][j][4 * q], acc[g][j][4 * q + 1], acc[g][j][4 * q + 2], acc[g][j][4 * q + 3]} * s_run;
-        *reinterpret_cast<u32x2 *>(cst + (32 * j + j32) * G_EPITCH + (32 * g + 8 * q + 4 * hh) * 2) =
-            u32x2{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
-      }
-  if (wave_rows) {
-    const int c16 = lane & 15;
-#pragma unroll 4
-    for (int r4 = 0; r4 < 16; ++r4) {
-      const int ml = 4 * r4 + (lane >> 4);
-      const int m = m0 + wm * 64 + ml, n = n0 + wn * 128 + 8 * c16;
-      const u32x4 v = *reinterpret_cast<const u32x4 *>(cst + ml * G_EPITCH + c16 * 16);
-      if (m < p.M && n < p.N) pstore8<MODE>(p, m, n, v);
-    }
-  }
-}
-
-// Workgroup i: tile i (t = m_tile * n_tiles + n_tile) with the whole K while
-// i < sp.full, else K part (i - full) % parts of tile full + (i - full) / parts.
-template <int MODE>
-__global__ __launch_bounds__(G_NW * 64, 1) void gemm_kernel(GemvParams p, bool staged_out, GemmSplit sp) {
-  const int i = blockIdx.x, KB = p.K >> 7;
-  int t = i, kb0 = 0, kb1 = KB;
-  float *partial = nullptr;
-  if (i >= sp.full) {
-    const int st = (i - sp.full) / sp.parts, q = (i - sp.full) % sp.parts;
-    t = sp.full + st;
-    kb0 = q * KB / sp.parts;
-    kb1 = (q + 1) * KB / sp.parts;
-    partial = sp.partial + (size_t)(st * sp.parts + q) * G_TILE_F4 * 4;
-  }
-  gemm_body<MODE>(p, staged_out, (t % sp.n_tiles) * G_BN, (t / sp.n_tiles) * G_BM, kb0, kb1, partial);
-}
-
-// Sums the K parts of the split tiles in part order and applies the epilogue.
-// Workgroup = one wave block (64 rows x 128 columns) of one split tile: the
-// parts are read in the lane order they were written (coalesced), summed in
-// part order, staged in LDS as rows, and stored 8 outputs per thread through
-// the same epilogue as the staged tiles (16-byte row stores).
-template <int MODE>
-__global__ __launch_bounds__(256) void gemm_finish_kernel(GemvParams p, GemmSplit sp) {
-  __shared__ float rows[64][128 + 4];
-  const int tid = threadIdx.x;
-  const int st = blockIdx.x / G_NW, wave = blockIdx.x % G_NW;
-  const f32x4 *src = reinterpret_cast<const f32x4 *>(sp.partial) + (size_t)st * sp.parts * G_TILE_F4 +
-                     (size_t)wave * G_WAVE_F4;
-  constexpr int PER = G_WAVE_F4 / 256;  // f32x4 per thread
-  f32x4 sum[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) sum[k] = src[k * 256 + tid];
-  for (int q = 1; q < sp.parts; ++q) {
-    f32x4 v[PER];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) v[k] = src[(size_t)q * G_TILE_F4 + k * 256 + tid];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) sum[k] += v[k];
-  }
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int rr = k * 256 + tid;  // ((g * 2 + j) * 4 + q) * 64 + lane
-    const int gjq = rr >> 6, lane = rr & 63;
-    const int g = gjq >> 3, j = (gjq >> 2) & 1, q = gjq & 3;
-    *reinterpret_cast<f32x4 *>(&rows[32 * j + (lane & 31)][32 * g + 8 * q + 4 * (lane >> 5)]) = sum[k];
-  }
-  __syncthreads();
-  const int t = sp.full + st;
-  const int m0 = (t / sp.n_tiles) * G_BM + (wave >> 1) * 64, n0 = (t % sp.n_tiles) * G_BN + (wave & 1) * 128;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int e = k * 256 + tid, r = e >> 4, c = (e & 15) * 8;
-    const int m = m0 + r, n = n0 + c;
-    if (m < p.M && n < p.N) {
-      const float *v = &rows[r][c];
-      pstore8<MODE>(p, m, n, u32x4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]),
-                                   pack_bf16(v[6], v[7])});
-    }
-  }
-}
-
-// Tiles past the last full round of 256 workgroups are cut into K parts so
-// that the launch ends with the machine full: time ~ (rounds of 256 work
-// items) x (tile time / parts) + the partial sums written and read back (256
-// KB per part); a tile's time is taken as proportional to K (~500 us at
-// K = 16384 on MI355X), the partial traffic at ~5 TB/s.
-GemmSplit plan_gemm_split(int M, int N, int K) {
-  GemmSplit sp = {};
-  sp.n_tiles = (N + G_BN - 1) / G_BN;
-  const int tiles = sp.n_tiles * ((M + G_BM - 1) / G_BM);
-  const int KB = K / 128;
-  const int full = tiles / 256 * 256, rest = tiles - full;
-  const double t_tile = 500.0 * K / 16384.0;  // us
-  int best = 1;
-  double best_cost = rest ? t_tile : 0.0;
-  for (int s = 2; s <= std::min(GEMM_MAX_PARTS, KB) && rest; ++s) {
-    const double cost = (double)((rest * s + 255) / 256) * t_tile / s + rest * s * (0.25 * 2 / 5e6 * 1e6);
-    if (cost < best_cost * 0.95) {
-      best_cost = cost;
-      best = s;
-    }
-  }
-  sp.full = best > 1 ? full : tiles;
-  sp.parts = best;
-  sp.items = sp.full + (tiles - sp.full) * best;
-  sp.bytes = best > 1 ? (size_t)(tiles - sp.full) * best * G_TILE_F4 * 16 : 0;
-  return sp;
-}
-
-size_t gemm_ws_bytes(int M, int N, int K) { return plan_gemm_split(M, N, K).bytes; }
-
-int launch_gemm(const GemvParams &p, int mode, hipStream_t st, float *split_ws, size_t split_ws_bytes) {
-  if (p.K % 128 || p.N % 4) return fail(AMLA_EUNSUPPORTED, "fp8 GEMM needs K %% 128 == 0 and N %% 4 == 0");
-  if (p.ldx % 8) return fail(AMLA_EUNSUPPORTED, "fp8 GEMM needs 16-byte aligned activation rows");
-  if ((mode == GEMV_QKVA && p.max_rows <= 0) || (mode == GEMV_QROPE && p.rope_rows <= 0))
-    return fail(AMLA_EINVAL, "fp8 GEMM: cache rows / rope rows of the epilogue not set");
-  if ((mode == GEMV_QKVA || p.w1) && p.n_split % G_BN)
-    return fail(AMLA_EUNSUPPORTED, "fp8 GEMM: the first weight segment must be a multiple of 256 rows");
-  static bool attr_set[5] = {false, false, false, false, false};  // dynamic LDS above 64 KB, once per mode
-  const void *fn = mode == GEMV_PLAIN  ? (const void *)gemm_kernel<GEMV_PLAIN>
-                   : mode == GEMV_RESID ? (const void *)gemm_kernel<GEMV_RESID>
-                   : mode == GEMV_QKVA  ? (const void *)gemm_kernel<GEMV_QKVA>
-                   : mode == GEMV_F32   ? (const void *)gemm_kernel<GEMV_F32>
-                                        : (const void *)gemm_kernel<GEMV_QROPE>;
-  if (mode < 0 || mode > 4) return fail(AMLA_EINVAL, "fp8 GEMM: unknown epilogue mode %d", mode);
-  if (!attr_set[mode]) {
-    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, G_LDS);
-    attr_set[mode] = true;
-  }
-  // 16-byte output stores need N, the row strides and the bases of every
-  // output (and of the residual) on 8-element boundaries
-  bool staged = p.N % 8 == 0 && p.ldy % 8 == 0 && aligned16(p.y);
-  if (mode == GEMV_RESID) staged = staged && p.ldr % 8 == 0 && aligned16(p.res);
-  if (mode == GEMV_QKVA)
-    staged = staged && aligned16(p.ckv) && aligned16(p.kpe) && p.kv_lora % 8 == 0 && p.rope % 8 == 0 &&
-             p.ckv_bstride % 8 == 0 && p.kpe_bstride % 8 == 0;
-  if (mode == GEMV_QROPE) staged = staged && p.head_dim % 8 == 0 && p.nope % 8 == 0;
-  if (mode == GEMV_F32) staged = false;  // fp32 rows: 16-byte stores of four outputs from the accumulators
-  GemmSplit sp = plan_gemm_split(p.M, p.N, p.K);
-  if (sp.parts > 1 && (!staged || !split_ws || split_ws_bytes < sp.bytes || !aligned16(split_ws))) {
-    // no room for the partial sums (or outputs without 16-byte stores): whole tiles
-    sp.full = sp.items = sp.n_tiles * ((p.M + G_BM - 1) / G_BM);
-    sp.parts = 1;
-  }
-  sp.partial = split_ws;
-  const dim3 grid(sp.items);
-  switch (mode) {
-    case GEMV_PLAIN: gemm_kernel<GEMV_PLAIN><<<grid, G_NW * 64, G_LDS, st>>>(p, staged, sp); break;
-    case GEMV_RESID: gemm_kernel<GEMV_RESID><<<grid, G_NW * 64, G_LDS, st>>>(p, staged, sp); break;
-    case GEMV_QKVA: gemm_kernel<GEMV_QKVA><<<grid, G_NW * 64, G_LDS, st>>>(p, staged, sp); break;
-    case GEMV_F32: gemm_kernel<GEMV_F32><<<grid, G_NW * 64, G_LDS, st>>>(p, staged, sp); break;
-    default: gemm_kernel<GEMV_QROPE><<<grid, G_NW * 64, G_LDS, st>>>(p, staged, sp); break;
-  }
-  int rc = check_launch("fp8 GEMM");
-  if (rc || sp.parts == 1) return rc;
-  const dim3 fgrid((unsigned)((sp.items - sp.full) / sp.parts * G_NW));
-  switch (mode) {
-    case GEMV_PLAIN: gemm_finish_kernel<GEMV_PLAIN><<<fgrid, 256, 0, st>>>(p, sp); break;
-    case GEMV_RESID: gemm_finish_kernel<GEMV_RESID><<<fgrid, 256, 0, st>>>(p, sp); break;
-    case GEMV_QKVA: gemm_finish_kernel<GEMV_QKVA><<<fgrid, 256, 0, st>>>(p, sp); break;
-    default: gemm_finish_kernel<GEMV_QROPE><<<fgrid, 256, 0, st>>>(p, sp); break;
-  }
-  return check_launch("fp8 GEMM K-part finish");
-}
 
 // ---------------------------------------------------------------- K10 causal flash attention
 

@@ -3,10 +3,12 @@
 //
 // y[m, n] = sum_k x[m, k] w[n, k] scale_inv[n/128, k/128], w e4m3fn converted
 // exactly to bf16 in registers, 32x32x16 bf16 MFMAs, fp32 sums.
+#include <algorithm>
 #include <type_traits>
 
 #include "amla_common.h"
 #include "amla_internal.h"
+#include "gemm_epilogue.h"
 
 namespace amla {
 
@@ -46,16 +48,28 @@ static_assert(tile_stages(2) * (T_WBYTES + 64 * T_XROW) <= T_ZERO && tile_stages
 struct TileArgs {
   const uint8_t *w[2];   // first row of each segment
   const float *s[2];     // scale row (K / 128) of each segment
+  int wrows[2];          // rows of each segment (128, fewer at the end of a matrix: the last one is repeated)
   const uint16_t *x;     // activation rows
   const int32_t *xrow;   // row of x for tile row r, or null: row r
   uint16_t *y;           // outputs, column 0 of the tile
   const int32_t *yrow;   // row of y for tile row r, or null: row r
   int ldx, ldy, K, rows;
-  bool two;              // segment 1 is stored (PLAIN; always multiplied)
+  int kb0, kb1;          // 128-wide K blocks
+  bool two;              // segment 1 is stored (always multiplied)
 };
 
-template <int NJ, bool SILU>
-AMLA_DEV void tile_body(const TileArgs &a) {
+// A tile's sums: acc[segment][row group of 32], in units of s_run[segment].
+template <int NJ>
+struct TileSums {
+  f32x16 acc[2][NJ];
+  float s_run[2];
+};
+
+template <int NJ>
+struct TileMain {
+  static AMLA_DEV void run(const TileArgs &a, TileSums<NJ> &sums) {
+  auto &acc = sums.acc;
+  auto &s_run = sums.s_run;
   extern __shared__ __align__(16) uint8_t tsm[];
   constexpr int NST = tile_stages(NJ);
   constexpr int STAGE = T_WBYTES + 32 * NJ * T_XROW;
@@ -63,14 +77,16 @@ AMLA_DEV void tile_body(const TileArgs &a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j32 = lane & 31, hh = lane >> 5;
-  const int KB = a.K >> 7;
 
   // copies: the wave's own 2 x 32 weight rows (16 rows of 64 B each) and its
   // quarter of the activation rows (8 rows of 128 B each)
-  const uint32_t wlane = (uint32_t)(lane >> 2) * a.K + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
-  const uint8_t *wsrc[2];
+  const uint8_t *wsrc[2][2];
 #pragma unroll
-  for (int g = 0; g < 2; ++g) wsrc[g] = a.w[g] + (size_t)(32 * wave) * a.K;
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      wsrc[g][c] = a.w[g] + (size_t)min(32 * wave + 16 * c + (lane >> 2), a.wrows[g] - 1) * a.K +
+                   16 * ((lane & 3) ^ ((lane >> 4) & 3));
   const uint8_t *xsrc[NJ];
 #pragma unroll
   for (int c = 0; c < NJ; ++c) {
@@ -85,7 +101,7 @@ AMLA_DEV void tile_body(const TileArgs &a) {
     for (int g = 0; g < 2; ++g)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        __builtin_amdgcn_global_load_lds(wsrc[g] + (size_t)(16 * c) * a.K + it * T_BK + wlane,
+        __builtin_amdgcn_global_load_lds(wsrc[g][c] + it * T_BK,
                                          LDS_PTR(st + (128 * g + 32 * wave + 16 * c) * T_BK), 16, 0, 0);
 #pragma unroll
     for (int c = 0; c < NJ; ++c)
@@ -105,89 +121,135 @@ AMLA_DEV void tile_body(const TileArgs &a) {
 #pragma unroll
   for (int g = 0; g < 2; ++g) srow[g] = (const __attribute__((address_space(4))) float *)(a.s[g]);
 
-  f32x16 acc[2][NJ];
 #pragma unroll
   for (int g = 0; g < 2; ++g)
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[g][j][r] = 0.f;
-  // The accumulators are kept in units of the current K block's scale, as in
-  // the 256 x 256 GEMM: acc *= s_prev / s_cur on entering a block, * s_last at
-  // the end (fp32 rounding of the ratios, ~1e-5 relative over 128 blocks).  A
-  // zero scale dequantises to zeros: the segment's fragments of that block are
-  // read from 16 zeroed bytes instead.
-  float s_run[2] = {0.f, 0.f};
-  bool skip[2] = {false, false};
-
+  // The accumulators are kept in units of the current K block's scale: acc *=
+  // s_prev / s_cur between two blocks, * s_last at the end (fp32 rounding of
+  // the ratios, ~1e-5 relative over 128 blocks).  A zero scale dequantises to
+  // zeros: the segment's fragments of that block are read from 16 zeroed bytes
+  // instead and the units stay.
+#pragma unroll
+  for (int g = 0; g < 2; ++g) s_run[g] = srow[g][a.kb0];
+  bool zero[2] = {s_run[0] == 0.f, s_run[1] == 0.f};
   if (tid < 4) *reinterpret_cast<uint32_t *>(tsm + T_ZERO + 4 * tid) = 0;  // visible after the first barrier
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
-  const int iters = 2 * KB;
+  const int it0 = 2 * a.kb0, iters = 2 * a.kb1;
 #pragma unroll
-  for (int i = 0; i < NST - 1; ++i) dma(i, i);  // iters >= 2 >= NST - 1
+  for (int i = 0; i < NST - 1; ++i) dma(it0 + i, i);  // a block is 2 >= NST - 1 stages
   int stg = 0;
-  for (int it = 0; it < iters; ++it) {
+  // One stage of 64: four sub-steps of 16 (K 32 pr + 16 hh + 8 s2 .. +7 of each
+  // half-wave).  While a sub-step multiplies, the fragments of the next are
+  // read and converted between its MFMAs.  The rescaling between two blocks
+  // (16 multiplies per 32 x 32 tile) runs between the last sub-step's MFMAs
+  // from the third on, while the next stage's first fragments are read, and
+  // between its first MFMAs.  Scheduling barriers keep the order: left to
+  // itself the compiler issues the multiplies and the LDS waits in runs.
+  constexpr int NT = 2 * NJ;           // tiles, in the order of their MFMAs
+  constexpr int LATE = NJ >= 3 ? 2 : 0;  // tiles rescaled between the next block's first MFMAs
+  auto rescale = [&](int half, const float *r) {  // half tiles in MFMA order
+    const int g = (half >> 1) / NJ, j = (half >> 1) % NJ;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[g][j][8 * (half & 1) + e] *= r[g];
+  };
+  auto stage = [&](int it, auto odd_c, const float *r) {
+    constexpr bool ODD = decltype(odd_c)::value;
     if (NST == 3 && it + 1 < iters) wait_vmcnt<COPIES>();
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (it + NST - 1 < iters) dma(it + NST - 1, stg == 0 ? NST - 1 : stg - 1);
-    if ((it & 1) == 0) {
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        const float sk = srow[g][it >> 1];
-        skip[g] = sk == 0.f;
-        if (!skip[g]) {
-          if (s_run[g] != 0.f) {
-            const float r = __fdiv_rn(s_run[g], sk);
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) acc[g][j] *= r;
-          }
-          s_run[g] = sk;
-        }
-      }
-    }
-    // Four sub-steps of 16 (K 32 pr + 16 hh + 8 s2 .. +7 of each half-wave);
-    // the fragments of the next one are read while the current one multiplies.
     const uint8_t *st = tsm + stg * STAGE;
     const uint8_t *sa[2];
 #pragma unroll
-    for (int g = 0; g < 2; ++g) sa[g] = skip[g] ? tsm + T_ZERO : st + g * 128 * T_BK;
+    for (int g = 0; g < 2; ++g) sa[g] = zero[g] ? tsm + T_ZERO : st + g * 128 * T_BK;
     u32x4 araw[2][2], bx[2][NJ];
+    bf16x8 av[2][2];
     auto read_a = [&](int pr) {
 #pragma unroll
-      for (int g = 0; g < 2; ++g) araw[pr][g] = *reinterpret_cast<const u32x4 *>(sa[g] + (skip[g] ? 0 : aoff[pr]));
+      for (int g = 0; g < 2; ++g) araw[pr][g] = *reinterpret_cast<const u32x4 *>(sa[g] + (zero[g] ? 0 : aoff[pr]));
     };
     auto read_b = [&](int q) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
         bx[q & 1][j] = *reinterpret_cast<const u32x4 *>(st + boff[q >> 1][q & 1] + j * 32 * T_XROW);
     };
+    auto cvt = [&](int q, int g) {
+      typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+      const uint32_t w0 = araw[q >> 1][g][2 * (q & 1)], w1 = araw[q >> 1][g][2 * (q & 1) + 1];
+      const bf16x2_t c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, false);
+      const bf16x2_t c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, true);
+      const bf16x2_t c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, false);
+      const bf16x2_t c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, true);
+      av[q & 1][g] = bf16x8{c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
+    };
     read_a(0);
     read_b(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!ODD) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (q < 3) read_b(q + 1);
-      if (q == 1) read_a(1);
-      __builtin_amdgcn_sched_barrier(0);
-      typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        const uint32_t w0 = araw[q >> 1][g][2 * (q & 1)], w1 = araw[q >> 1][g][2 * (q & 1) + 1];
-        const bf16x2_t c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, false);
-        const bf16x2_t c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, true);
-        const bf16x2_t c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, false);
-        const bf16x2_t c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, true);
-        const bf16x8 av = {c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-          acc[g][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, as_bf16x8(bx[q & 1][j]), acc[g][j], 0, 0, 0);
-      }
+      for (int h = NT - 2; h < 2 * (NT - LATE); ++h) rescale(h, r);
       __builtin_amdgcn_sched_barrier(0);
     }
+    cvt(0, 0);
+    cvt(0, 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const int i = g * NJ + j;
+          acc[g][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[q & 1][g], as_bf16x8(bx[q & 1][j]), acc[g][j], 0, 0, 0);
+          // (the reads go out behind the first MFMA: the wait before it covers
+          // every LDS read in flight)
+          if (i == 0 && q == 0) read_a(1);
+          if (i == 0 && q < 3) read_b(q + 1);
+          if (!ODD && q == 0 && i < 2 * LATE) rescale(2 * (NT - LATE) + i, r);
+          if (ODD && q == 3 && i >= 2) rescale(i - 2, r);
+          if (q < 3 && i == NT - 2) cvt(q + 1, 0);
+          if (q < 3 && i == NT - 1) cvt(q + 1, 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    }
     stg = stg == NST - 1 ? 0 : stg + 1;
+  };
+  float r[2] = {1.f, 1.f};
+  for (int kb = a.kb0; kb < a.kb1; ++kb) {
+    float sn[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) sn[g] = srow[g][min(kb + 1, a.kb1 - 1)];
+    stage(2 * kb, std::false_type{}, r);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) r[g] = s_run[g] == 0.f || sn[g] == 0.f ? 1.f : __fdiv_rn(s_run[g], sn[g]);
+    stage(2 * kb + 1, std::true_type{}, r);
+    if (kb + 1 < a.kb1) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        zero[g] = sn[g] == 0.f;
+        if (!zero[g]) s_run[g] = sn[g];
+      }
+    }
   }
+  // the tiles rescaled after the last block were so by s / s = 1
+}
+};
+
+// Stores a tile.  SILU: y = bf16(silu(segment 0)) * segment 1, 128 columns;
+// else y = both segments, 256 columns.
+template <int NJ, bool SILU>
+AMLA_DEV void tile_store(const TileArgs &a, const TileSums<NJ> &ts) {
+  extern __shared__ __align__(16) uint8_t tsm[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j32 = lane & 31, hh = lane >> 5;
+  auto &acc = ts.acc;
+  auto &s_run = ts.s_run;
 
   // Lane holds row 32 j + j32, columns 32 wave + 8 q + 4 hh .. +3 of each
   // segment.  The outputs go through LDS so that every store is 16 bytes of
@@ -231,6 +293,222 @@ AMLA_DEV void tile_body(const TileArgs &a) {
   }
 }
 
+// ---------------------------------------------------------------- linears of many rows
+
+// The GEMM of launch_gemm (GemvMode epilogues): tiles of 256 weight rows x 128
+// activation rows.  Workgroup i runs on XCD i % 8: each XCD takes a contiguous
+// run of the tiles in panels of 8 column tiles, row tiles within a panel, so
+// the 64 tiles it holds at a time share 8 + 8 tile operands through its L2.
+constexpr int TL_PANEL = 8;
+
+AMLA_DEV void tile_coords(int t, int n_tiles, int m_tiles, int &nt, int &mt) {
+  const int per = TL_PANEL * m_tiles, p = t / per, r = t - p * per;
+  const int width = min(TL_PANEL, n_tiles - p * TL_PANEL);
+  mt = r / width;
+  nt = p * TL_PANEL + r - mt * width;
+}
+// logical index of workgroup i of n (or -1): a contiguous run per XCD
+AMLA_DEV int xcd_run(int i, int n) {
+  const int run = (n + 7) >> 3, l = (i & 7) * run + (i >> 3);
+  return (i >> 3) < run && l < n ? l : -1;
+}
+
+template <int MODE, int NJ>
+AMLA_DEV void tile_linear_body(const GemvParams &p, const TileArgs &a, const int (&n0)[2], int m0, bool staged,
+                               float *partial) {
+  extern __shared__ __align__(16) uint8_t tsm[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j32 = lane & 31, hh = lane >> 5;
+  TileSums<NJ> ts;
+  TileMain<NJ>::run(a, ts);
+  auto &acc = ts.acc;
+  auto &s_run = ts.s_run;
+  auto sums = [&](int g, int j, int q) {
+    return f32x4{acc[g][j][4 * q], acc[g][j][4 * q + 1], acc[g][j][4 * q + 2], acc[g][j][4 * q + 3]} * s_run[g];
+  };
+  if (partial) {
+    // [g][j][wave][q][lane] f32x4: every store is 1 KB contiguous per wave
+    f32x4 *dst = reinterpret_cast<f32x4 *>(partial);
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) dst[(((g * 4 + j) * 4 + wave) * 4 + q) * 64 + lane] = sums(g, j, q);
+    return;
+  }
+  if (MODE == GEMV_F32 || (MODE != GEMV_SILU && !staged)) {
+    // fp32 rows, or rows without 16-byte alignment: four outputs per store straight from the accumulators
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int r = 32 * j + j32;
+      if (r >= a.rows) continue;
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int c = 32 * wave + 8 * q + 4 * hh;
+          if (c < a.wrows[g] && (g == 0 || a.two)) pstore4<MODE == GEMV_SILU ? GEMV_PLAIN : MODE>(p, m0 + r, n0[g] + c, sums(g, j, q));
+        }
+    }
+    return;
+  }
+  if constexpr (MODE == GEMV_SILU) {
+    tile_store<NJ, true>(a, ts);
+    return;
+  }
+  __builtin_amdgcn_s_barrier();  // every wave is past its last fragment read
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const f32x4 v = sums(g, j, q);
+        *reinterpret_cast<u32x2 *>(tsm + (32 * j + j32) * T_PITCH_Y + g * 256 + (32 * wave + 8 * q + 4 * hh) * 2) =
+            u32x2{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
+      }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  const int g = (tid >> 4) & 1, c = 8 * (tid & 15);
+  if (c < a.wrows[g] && (g == 0 || a.two))
+    for (int r = tid >> 5; r < a.rows; r += 8)
+      pstore8<MODE == GEMV_SILU ? GEMV_PLAIN : MODE>(p, m0 + r, n0[g] + c, *reinterpret_cast<const u32x4 *>(tsm + r * T_PITCH_Y + (tid & 31) * 16));
+}
+
+// Workgroups [0, full): whole tiles; then K part (i - full) % parts of tile full + (i - full) / parts.
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void tile_linear_kernel(GemvParams p, bool staged, GemmSplit sp) {
+  const int KB = p.K >> 7;
+  int t, kb0 = 0, kb1 = KB;
+  float *partial = nullptr;
+  if ((int)blockIdx.x < sp.full_blocks) {
+    t = xcd_run(blockIdx.x, sp.full);
+    if (t < 0) return;
+  } else {
+    const int l = xcd_run(blockIdx.x - sp.full_blocks, sp.rest * sp.parts);
+    if (l < 0) return;
+    const int st = l / sp.parts, q = l - st * sp.parts;
+    t = sp.full + st;
+    kb0 = q * KB / sp.parts;
+    kb1 = (q + 1) * KB / sp.parts;
+    partial = sp.partial + (size_t)l * TILE_PART_F32;
+  }
+  int nt, mt;
+  tile_coords(t, sp.n_tiles, sp.m_tiles, nt, mt);
+  TileArgs a;
+  const int m0 = mt * TILE_ROWS;
+  a.rows = min(TILE_ROWS, p.M - m0);
+  a.K = p.K;
+  a.ldx = p.ldx;
+  a.kb0 = kb0;
+  a.kb1 = kb1;
+  a.x = p.x + (size_t)m0 * p.ldx;
+  a.xrow = nullptr;
+  // segment = a run of up to 128 rows of one weight: the first weight's
+  // segments come before the second's (n_split % 128 == 0)
+  int n0[2];
+  a.two = true;
+  if constexpr (MODE == GEMV_SILU) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      n0[g] = nt * 128;
+      a.w[g] = (g ? p.w1 : p.w0) + (size_t)n0[g] * p.K;
+      a.s[g] = (g ? p.s1 : p.s0) + (size_t)nt * KB;
+      a.wrows[g] = 128;
+    }
+    a.y = p.y + (size_t)m0 * p.ldy + n0[0];
+    a.yrow = nullptr;
+    a.ldy = p.ldy;
+  } else
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    int n = nt * 256 + g * 128;
+    if (g == 1) {
+      a.two = n < p.N;
+      if (!a.two) n = nt * 256;  // no second segment: the first is multiplied twice
+    }
+    n0[g] = n;
+    const bool second = p.w1 && n >= p.n_split;
+    const int nl = second ? n - p.n_split : n;
+    a.w[g] = (second ? p.w1 : p.w0) + (size_t)nl * p.K;
+    a.s[g] = (second ? p.s1 : p.s0) + (size_t)(nl >> 7) * KB;
+    a.wrows[g] = min(128, (p.w1 && !second ? p.n_split : p.N) - n);
+  }
+  switch ((a.rows + 31) >> 5) {
+    case 1: tile_linear_body<MODE, 1>(p, a, n0, m0, staged, partial); break;
+    case 2: tile_linear_body<MODE, 2>(p, a, n0, m0, staged, partial); break;
+    case 3: tile_linear_body<MODE, 3>(p, a, n0, m0, staged, partial); break;
+    default: tile_linear_body<MODE, 4>(p, a, n0, m0, staged, partial); break;
+  }
+}
+
+// Sums the K parts of the split tiles in part order and applies the epilogue.
+// Workgroup = 32 rows x 128 columns (row group j of segment g, or of both for
+// SILU) of one split tile: the parts are read in the lane order they were
+// written, summed in part order, staged in LDS as rows, and stored 8 outputs
+// per thread through the same epilogue as the staged tiles.
+template <int MODE>
+__global__ __launch_bounds__(256) void tile_finish_kernel(GemvParams p, GemmSplit sp) {
+  constexpr bool SILU = MODE == GEMV_SILU;
+  constexpr int SEGS = SILU ? 2 : 1;
+  __shared__ float rows[32][128 + 4];
+  const int tid = threadIdx.x;
+  const int st = blockIdx.x >> (SILU ? 2 : 3), g = SILU ? 0 : (blockIdx.x >> 2) & 1, j = blockIdx.x & 3;
+  int nt, mt;
+  tile_coords(sp.full + st, sp.n_tiles, sp.m_tiles, nt, mt);
+  const int m0 = mt * TILE_ROWS + 32 * j, n0 = SILU ? nt * 128 : nt * 256 + g * 128;
+  if (m0 >= p.M || n0 >= p.N) return;
+  const f32x4 *src = reinterpret_cast<const f32x4 *>(sp.partial + (size_t)st * sp.parts * TILE_PART_F32) +
+                     (g * 4 + j) * 1024 + (tid >> 6) * 256 + (tid & 63);
+  f32x4 sum[SEGS][4];
+#pragma unroll
+  for (int s = 0; s < SEGS; ++s)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sum[s][q] = src[s * 4096 + q * 64];
+#pragma unroll 4
+  for (int k = 1; k < sp.parts; ++k)
+#pragma unroll
+    for (int s = 0; s < SEGS; ++s)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sum[s][q] += src[(size_t)k * (TILE_PART_F32 / 4) + s * 4096 + q * 64];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    f32x4 v = sum[0][q];
+    if constexpr (SILU)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = silu_bf16(round_bf16(v[i])) * round_bf16(sum[SEGS - 1][q][i]);
+    *reinterpret_cast<f32x4 *>(&rows[tid & 31][32 * (tid >> 6) + 8 * q + 4 * ((tid >> 5) & 1)]) = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int r = (tid >> 4) + 16 * k, c = (tid & 15) * 8;
+    if (m0 + r >= p.M || n0 + c >= p.N) continue;
+    const float *v = &rows[r][c];
+    if constexpr (MODE == GEMV_F32) {
+      pstore4<MODE>(p, m0 + r, n0 + c, f32x4{v[0], v[1], v[2], v[3]});
+      pstore4<MODE>(p, m0 + r, n0 + c + 4, f32x4{v[4], v[5], v[6], v[7]});
+    } else {
+      pstore8<SILU ? GEMV_PLAIN : MODE>(
+          p, m0 + r, n0 + c,
+          u32x4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])});
+    }
+  }
+}
+
+// ---------------------------------------------------------------- routed experts
+
+template <int NJ, bool SILU>
+AMLA_DEV void tile_body(const TileArgs &a) {
+  TileSums<NJ> ts;
+  TileMain<NJ>::run(a, ts);
+  tile_store<NJ, SILU>(a, ts);
+}
+
 template <bool SILU>
 AMLA_DEV void tile_dispatch(const TileArgs &a) {
   switch ((a.rows + 31) >> 5) {
@@ -257,6 +535,9 @@ AMLA_DEV void moe_tile(const MoeTileParams &p, const TileGroup &g, int nt, const
   a.xrow = xrow;
   a.y = (yrow ? p.y : p.y + (size_t)g.first * p.ldy) + nt * (GATEUP ? 128 : 256);
   a.yrow = yrow;
+  a.kb0 = 0;
+  a.kb1 = KB;
+  a.wrows[0] = a.wrows[1] = 128;
   a.two = GATEUP || nt * 256 + 128 < p.N;  // N % 256 == 128: the last tile multiplies its one segment twice
   a.w[0] = static_cast<const uint8_t *>(g.w0) + (size_t)nt * (GATEUP ? 128 : 256) * p.K;
   a.s[0] = g.s0 + (size_t)nt * (GATEUP ? 1 : 2) * KB;
@@ -338,6 +619,95 @@ int launch_tile_grouped(const MoeTileParams &p0, const TileGroups &gr, bool down
   if (down) tile_grouped_kernel<false><<<dim3((unsigned)blocks), 256, T_LDS, st>>>(p, gr);
   else tile_grouped_kernel<true><<<dim3((unsigned)blocks), 256, T_LDS, st>>>(p, gr);
   return check_launch("grouped fp8 tiles");
+}
+
+// Workgroups: 512 run at a time (two per CU).  Tiles past the last full round
+// are cut into K parts where that shortens the launch.  Measured on MI355X, a
+// 128-wide K block of a 128-row tile takes 3.9 us with two workgroups per CU
+// and 1.8 us with one; the partial sums (128 KB per part) cross memory twice
+// at ~4 TB/s, and the finishing pass costs about 5 us of its own.
+GemmSplit plan_gemm_split(int M, int N, int K, int mode) {
+  GemmSplit sp = {};
+  const int cols = mode == GEMV_SILU ? 128 : 256;
+  sp.n_tiles = (N + cols - 1) / cols;
+  sp.m_tiles = (M + TILE_ROWS - 1) / TILE_ROWS;
+  const int tiles = sp.n_tiles * sp.m_tiles;
+  const int KB = K / 128;
+  const int full = tiles / 512 * 512, rest = tiles - full;
+  const double nj = (std::min(M, TILE_ROWS) + 31) / 32;
+  const double one = 0.9 + 0.225 * nj, two = std::max(1.3, 0.975 * nj);  // us per K block
+  auto cost_of = [&](int parts) {
+    const int items = rest * parts, last = items % 512;
+    const double kb = (KB + parts - 1) / parts;
+    const double rounds = items / 512 * two + (last == 0 ? 0.0 : last <= 256 ? one : two);
+    return rounds * kb + (parts > 1 ? 5.0 + items * 0.064 * nj / 4 : 0.0);
+  };
+  int best = 1;
+  double best_cost = rest ? cost_of(1) : 0.0;
+  for (int s = 2; s <= std::min(GEMM_MAX_PARTS, KB) && rest; ++s) {
+    const double cost = cost_of(s);
+    if (cost < best_cost * 0.97) {
+      best_cost = cost;
+      best = s;
+    }
+  }
+  sp.full = best > 1 ? full : tiles;
+  sp.rest = tiles - sp.full;
+  sp.parts = best;
+  sp.full_blocks = (sp.full + 7) / 8 * 8;
+  sp.bytes = (size_t)sp.rest * (best > 1 ? best : 0) * TILE_PART_F32 * 4;
+  return sp;
+}
+
+size_t gemm_ws_bytes(int M, int N, int K, int mode) { return plan_gemm_split(M, N, K, mode).bytes; }
+
+template <int MODE>
+static int launch_tile_linear(const GemvParams &p, bool staged, const GemmSplit &sp, hipStream_t st) {
+  int rc = tile_lds((const void *)tile_linear_kernel<MODE>);
+  if (rc) return rc;
+  const unsigned blocks = (unsigned)(sp.full_blocks + (sp.rest * sp.parts + 7) / 8 * 8);
+  tile_linear_kernel<MODE><<<dim3(blocks), 256, T_LDS, st>>>(p, staged, sp);
+  if ((rc = check_launch("fp8 GEMM")) || !sp.rest) return rc;
+  tile_finish_kernel<MODE><<<dim3((unsigned)sp.rest * (MODE == GEMV_SILU ? 4 : 8)), 256, 0, st>>>(p, sp);
+  return check_launch("fp8 GEMM K-part finish");
+}
+
+int launch_gemm(const GemvParams &p, int mode, hipStream_t st, float *split_ws, size_t split_ws_bytes) {
+  if (p.K % 128 || p.N % 4) return fail(AMLA_EUNSUPPORTED, "fp8 GEMM needs K %% 128 == 0 and N %% 4 == 0");
+  if (p.ldx % 8) return fail(AMLA_EUNSUPPORTED, "fp8 GEMM needs 16-byte aligned activation rows");
+  if ((mode == GEMV_QKVA && p.max_rows <= 0) || (mode == GEMV_QROPE && p.rope_rows <= 0))
+    return fail(AMLA_EINVAL, "fp8 GEMM: cache rows / rope rows of the epilogue not set");
+  if (mode == GEMV_SILU && (p.N % 128 || p.ldy % 8 || !aligned16(p.y) || !p.w1))
+    return fail(AMLA_EUNSUPPORTED, "fp8 GEMM: silu * up needs two weights of N %% 128 == 0 rows and 16-byte aligned rows");
+  if (mode != GEMV_SILU && p.w1 && p.n_split % 128)
+    return fail(AMLA_EUNSUPPORTED, "fp8 GEMM: the first weight segment must be a multiple of 128 rows");
+  // 16-byte output stores need N, the row strides and the bases of every
+  // output (and of the residual) on 8-element boundaries
+  bool staged = p.N % 8 == 0 && p.ldy % 8 == 0 && aligned16(p.y);
+  if (mode == GEMV_RESID) staged = staged && p.ldr % 8 == 0 && aligned16(p.res);
+  if (mode == GEMV_QKVA)
+    staged = staged && aligned16(p.ckv) && aligned16(p.kpe) && p.kv_lora % 8 == 0 && p.rope % 8 == 0 &&
+             p.ckv_bstride % 8 == 0 && p.kpe_bstride % 8 == 0;
+  if (mode == GEMV_QROPE) staged = staged && p.head_dim % 8 == 0 && p.nope % 8 == 0;
+  if (mode == GEMV_F32) staged = p.N % 8 == 0 && p.ldy % 4 == 0 && aligned16(p.y);
+  GemmSplit sp = plan_gemm_split(p.M, p.N, p.K, mode);
+  if (sp.rest && (!staged || !split_ws || split_ws_bytes < sp.bytes || !aligned16(split_ws))) {
+    // no room for the partial sums (or outputs without 16-byte stores): whole tiles
+    sp.full = sp.n_tiles * sp.m_tiles;
+    sp.rest = 0;
+    sp.parts = 1;
+    sp.full_blocks = (sp.full + 7) / 8 * 8;
+  }
+  sp.partial = split_ws;
+  switch (mode) {
+    case GEMV_PLAIN: return launch_tile_linear<GEMV_PLAIN>(p, staged, sp, st);
+    case GEMV_RESID: return launch_tile_linear<GEMV_RESID>(p, staged, sp, st);
+    case GEMV_QKVA: return launch_tile_linear<GEMV_QKVA>(p, staged, sp, st);
+    case GEMV_QROPE: return launch_tile_linear<GEMV_QROPE>(p, staged, sp, st);
+    case GEMV_F32: return launch_tile_linear<GEMV_F32>(p, staged, sp, st);
+    case GEMV_SILU: return launch_tile_linear<GEMV_SILU>(p, staged, sp, st);
+    default: return fail(AMLA_EINVAL, "fp8 GEMM: unknown epilogue mode %d", mode);
+  }
 }
 
 }  // namespace amla

@@ -48,7 +48,9 @@ int amla_fp8_block_dequant(const void *weight, const float *scale_inv, int64_t n
  * stride ldy.  For m <= 64 a long K is split over workgroups whose fp32
  * partial sums need `workspace` (16-byte aligned) of
  * amla_fp8_linear_workspace_bytes(m, n, k) bytes; when that is 0, NULL is
- * accepted.  Scratch only: no contents carry between calls. */
+ * accepted.  For m > 64 it may always be NULL or smaller: the sums of a shape
+ * that would leave part of the device idle then stay unsplit, which is slower.
+ * Scratch only: no contents carry between calls. */
 int amla_fp8_linear(const void *x, int64_t m, int64_t k, int64_t ldx, const void *weight,
                     const float *scale_inv, int64_t n, void *y, int64_t ldy, void *workspace,
                     size_t workspace_bytes, void *stream);
