@@ -195,4 +195,12 @@ int check_mla_common(const amla_mla_args *a, const char *who);
 // (> 0), else max_seq.
 inline int mla_context_bound(const amla_mla_args &a) { return a.max_context > 0 ? a.max_context : a.max_seq; }
 
+
+// Prefill attention in latent space (mla_decode.hip): whether it is the faster
+// form for these sizes, its scratch, and the launches (q with the rope applied
+// and the new cache rows written before).
+bool prefill_absorbed(int batch, int seq_len, int context);
+size_t prefill_absorbed_ws_bytes(int batch, int seq_len, int context);
+int launch_prefill_absorbed(const amla_mla_args &a, const uint16_t *q, uint16_t *attn, char *ws, hipStream_t stream);
+
 }  // namespace amla

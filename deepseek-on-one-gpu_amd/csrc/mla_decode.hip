@@ -80,15 +80,32 @@ inline size_t plan_ints(int B, int slots) { return PLAN_HDR + 2 * (size_t)B + sl
 
 AMLA_DEV int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
+// The tokens of one launch sequence: token i is row first + i of the
+// (sequences, seq_len) new tokens.  In decode seq_len is 1 (token = sequence,
+// first = 0); the absorbed prefill runs the new tokens of a sequence as so
+// many decode tokens over the sequence's one cache, token s of it at position
+// pos[sequence] + s.
+struct TokenMap {
+  const int32_t *start;  // first new position per sequence
+  int seq_len, first;
+  AMLA_DEV int seq(int i) const { return seq_len == 1 ? first + i : (first + i) / seq_len; }
+  AMLA_DEV int pos(int i) const {
+    const int b = seq(i);
+    return start[b] + (first + i - b * seq_len);
+  }
+  // context of token i: cache rows [0, pos], clamped to the bound
+  AMLA_DEV int context(int i, int tmax) const { return min(pos(i) + 1, tmax); }
+};
+
 // Smallest and largest tile count of the batch (B <= 64), wave-uniform: lane
 // b loads sequence b's position (one vector load: a loop of scalar loads
 // waited for each one in turn, a round trip per sequence), then a butterfly
 // over the wave.  Every lane of the wave must call it.
-AMLA_DEV int2 batch_tile_range(const int32_t *pos, int tmax, int B) {
+AMLA_DEV int2 batch_tile_range(const TokenMap &map, int tmax, int B) {
   const int lane = threadIdx.x & 63;
   int lo = INT_MAX, hi = 0;
   if (lane < B) {
-    const int T = min(pos[lane] + 1, tmax);
+    const int T = map.context(lane, tmax);
     lo = hi = T > 0 ? ceil_div(T, TT) : 0;
   }
 #pragma unroll
@@ -137,14 +154,14 @@ AMLA_DEV int wave_max_int(int v) {
 // ceil(N_b / L) does not grow with L, and L = max N_b fits), then s_b and
 // first_b by a scan over its lanes; every thread then writes the sequence of
 // its slots (a binary search over first_b).
-AMLA_DEV void build_split_plan(const int32_t *__restrict__ pos, int tmax, int B, int units, int slots,
+AMLA_DEV void build_split_plan(const TokenMap &map, int tmax, int B, int units, int slots,
                                int32_t *__restrict__ plan, int *lds) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int *first = lds + B, *sh = lds + 2 * B;
   if (wave == 0) {
     int n = 0;
     if (lane < B) {
-      const int T = min(pos[lane] + 1, tmax);
+      const int T = map.context(lane, tmax);
       n = T > 0 ? ceil_div(T, TT) : 0;
     }
     const int N = wave_sum_int(n), most = wave_max_int(n);
@@ -220,7 +237,7 @@ __global__ __launch_bounds__(256) void absorb_kernel(const uint16_t *__restrict_
                                                      const float *__restrict__ skvb,
                                                      const uint16_t *__restrict__ gamma, int B,
                                                      uint16_t *__restrict__ qbuf,
-                                                     const int32_t *__restrict__ pos, int tmax, int units,
+                                                     TokenMap map, int tmax, int units,
                                                      int slots, int32_t *__restrict__ plan) {
   typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
   typedef int v2i __attribute__((ext_vector_type(2)));
@@ -238,8 +255,8 @@ __global__ __launch_bounds__(256) void absorb_kernel(const uint16_t *__restrict_
     // a batch with unequal tile counts (alongside the absorb workgroups, not
     // before one of them), the others have no work
     if (quarter == 0 && blockIdx.z == 0) {
-      const int2 r = batch_tile_range(pos, tmax, B);
-      if (r.x != r.y) build_split_plan(pos, tmax, B, units, slots, plan, reinterpret_cast<int *>(wsm));
+      const int2 r = batch_tile_range(map, tmax, B);
+      if (r.x != r.y) build_split_plan(map, tmax, B, units, slots, plan, reinterpret_cast<int *>(wsm));
     }
     return;
   }
@@ -341,7 +358,7 @@ struct AttnParams {
   const uint16_t *kpe;   // cache (B_alloc, max_seq, 64)
   int64_t ckv_bstride, kpe_bstride;  // elements per sequence
   const float *rope_table;           // (rows, 32, 2)
-  const int32_t *pos;                // decode position per sequence; context T = min(pos + 1, tmax)
+  TokenMap map;                      // tokens of the launch (b below: token); context T = min(pos + 1, tmax)
   int tmax;                          // context bound (rows of cache and rope table that may be read)
   int units;         // splits shared out over the batch (the grid has units + batch workgroups)
   int batch;
@@ -359,12 +376,12 @@ struct SeqSplits {
 };
 
 AMLA_DEV int seq_tiles(const AttnParams &p, int b) {
-  const int T = min(p.pos[b] + 1, p.tmax);
+  const int T = p.map.context(b, p.tmax);
   return T > 0 ? (T + TT - 1) / TT : 0;
 }
 
 AMLA_DEV SeqSplits seq_splits(const AttnParams &p, int b) {
-  const int2 r = batch_tile_range(p.pos, p.tmax, p.batch);
+  const int2 r = batch_tile_range(p.map, p.tmax, p.batch);
   if (r.x == r.y) {
     const int s = uniform_splits(r.x, p.units, p.batch);
     return SeqSplits{b * s, s, r.x};
@@ -576,7 +593,7 @@ __global__ __launch_bounds__(256, 1) void attn_kernel(AttnParams p) {
   // this workgroup's (sequence, split) from the batch's split plan; slots past
   // the plan have no work
   int b, split, ns;
-  const int2 range = batch_tile_range(p.pos, p.tmax, p.batch);
+  const int2 range = batch_tile_range(p.map, p.tmax, p.batch);
   if (range.x == range.y) {
     ns = uniform_splits(range.x, p.units, p.batch);
     b = slot / ns;
@@ -589,8 +606,9 @@ __global__ __launch_bounds__(256, 1) void attn_kernel(AttnParams p) {
     split = slot - __builtin_amdgcn_readfirstlane(fs.x);
     ns = __builtin_amdgcn_readfirstlane(fs.y);
   }
+  const int sq = __builtin_amdgcn_readfirstlane(p.map.seq(b));  // whose cache the token reads
   const int nb = seq_tiles(p, b);
-  const int T = min(p.pos[b] + 1, p.tmax);
+  const int T = p.map.context(b, p.tmax);
   const int tb = split_tile(nb, ns, split);
   const int te = split_tile(nb, ns, split + 1);
   extern __shared__ __align__(16) uint8_t smem[];
@@ -603,7 +621,7 @@ __global__ __launch_bounds__(256, 1) void attn_kernel(AttnParams p) {
   // once both have landed (the compiler's wait before the first fragment use
   // is for every load issued so far), the second tile's copies go out during
   // its score steps
-  if (tb < te) dma_tile(p, b, tb, T, smem, smem, wave, lane);
+  if (tb < te) dma_tile(p, sq, tb, T, smem, smem, wave, lane);
   __builtin_amdgcn_sched_barrier(0);
   constexpr int QLOADS = NTW * (QKD / 32);  // per wave, after the copies
   static_assert(TILE_DMA + QLOADS <= 63, "vmcnt range");
@@ -810,11 +828,11 @@ __global__ __launch_bounds__(256, 1) void attn_kernel(AttnParams p) {
           // the second tile's copies (steps 0 .. 10), then the third tile's
           // (steps 7 .. 17, after the second tile's piece of the same step)
           if (ks < TILE_DMA)
-            dma_piece(p, b, min(tile + 1, te - 1), tile + 1, T, smem, smem + STAGE_BYTES, wave, lane, lane16, ks);
+            dma_piece(p, sq, min(tile + 1, te - 1), tile + 1, T, smem, smem + STAGE_BYTES, wave, lane, lane16, ks);
           if (ks >= F3)
-            dma_piece(p, b, min(tile + 2, te - 1), tile + 2, T, smem, nst, wave, lane, lane16, ks - F3);
+            dma_piece(p, sq, min(tile + 2, te - 1), tile + 2, T, smem, nst, wave, lane, lane16, ks - F3);
         } else {
-          if (ks < TILE_DMA) dma_piece(p, b, min(tile + 2, te - 1), tile + 2, T, smem, nst, wave, lane, lane16, ks);
+          if (ks < TILE_DMA) dma_piece(p, sq, min(tile + 2, te - 1), tile + 2, T, smem, nst, wave, lane, lane16, ks);
         }
       }
       // the softmax reads sc: MFMA write -> VALU read wait states
@@ -1049,14 +1067,14 @@ AMLA_DEV void recompute_split(const AttnParams &p, int b, int h, const SeqSplits
                               float *ps, float *red, float &m_out, float &l_out, float &o0, float &o1) {
   const int tid = threadIdx.x;
   const bool act = tid < 256;
-  const int T = min(p.pos[b] + 1, p.tmax);
+  const int T = p.map.context(b, p.tmax);
   const int t0 = split_tile(sp.ntiles, sp.count, split) * TT;
   const int t1 = min(split_tile(sp.ntiles, sp.count, split + 1) * TT, T);
   __syncthreads();
   for (int c = tid; c < QKD; c += 512) qs[c] = bf2f(p.qbuf[qfrag_index(b, h, c)]);
   __syncthreads();
-  const uint16_t *cb = p.ckv + (size_t)b * p.ckv_bstride;
-  const uint16_t *kb = p.kpe + (size_t)b * p.kpe_bstride;
+  const uint16_t *cb = p.ckv + (size_t)p.map.seq(b) * p.ckv_bstride;
+  const uint16_t *kb = p.kpe + (size_t)p.map.seq(b) * p.kpe_bstride;
   float M = -INFINITY, L = 0.f, a0 = 0.f, a1 = 0.f;
   for (int c0 = t0; c0 < t1; c0 += 256) {
     const int t = c0 + tid;
@@ -1348,7 +1366,19 @@ constexpr int DECODE_MAX_BATCH = 64;
 // split slots fill at most half the CUs, so that a workgroup's fixed cost (the
 // query fragments in, the partial O out, both in proportion to its heads)
 // halves and twice the CUs share it; else one (all 128 heads).
-static int attn_head_groups(const DecodeLayout &L) { return L.slots <= 128 ? 2 : 1; }
+static int attn_head_groups(int slots) { return slots <= 128 ? 2 : 1; }
+
+// Split budget and partial slots of a launch sequence of `tokens` tokens with
+// contexts up to maxT: one split per CU, at least two tiles each for the
+// longest possible context, or one tile each while the tokens hold at most 64
+// tiles (a split's fixed cost then outweighs its second tile); the plan itself
+// is made on the device from the positions (build_split_plan).
+static void attn_units(int tokens, int maxT, int &units, int &slots) {
+  const int ntiles = (maxT + TT - 1) / TT;
+  const int64_t bt = (int64_t)tokens * ntiles;
+  units = (int)std::max<int64_t>(1, std::min<int64_t>(256, bt <= 64 ? bt : (int64_t)tokens * std::max(1, ntiles / 2)));
+  slots = units + tokens;
+}
 
 static DecodeLayout decode_layout(const amla_mla_args &a) {
   DecodeLayout L = {};
@@ -1357,15 +1387,7 @@ static DecodeLayout decode_layout(const amla_mla_args &a) {
   L.pa = plan_linear(B, a.q_lora + a.kv_lora + a.qk_rope, a.hidden);
   L.pb = plan_linear(B, a.heads * HD, a.q_lora);
   L.po = plan_linear(B, a.hidden, a.heads * a.v_dim);
-  // splits over the batch: one per CU, at least two tiles each for the
-  // longest possible context, or one tile each while the batch holds at most
-  // 64 tiles (a split's fixed cost then outweighs its second tile); the plan
-  // itself is made on the device from the positions (build_split_plan)
-  const int maxT = mla_context_bound(a);
-  const int ntiles = (maxT + TT - 1) / TT;
-  const int bt = B * ntiles;
-  L.units = std::max(1, std::min(256, bt <= 64 ? bt : B * std::max(1, ntiles / 2)));
-  L.slots = L.units + B;
+  attn_units(B, mla_context_bound(a), L.units, L.slots);
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
   L.plan = take(plan_ints(B, L.slots) * 4);  // first: a test reads the table back
@@ -1416,6 +1438,138 @@ constexpr int NSTAGE = 7;  // qkva, q_a norm, q_b, absorb, attention, combine, o
 static inline void mark(hipEvent_t const *ev, int i, hipStream_t st) {
   if (ev) (void)hipEventRecord(ev[i], st);
 }
+
+struct AbsorbedScratch {
+  int32_t *plan;      // plan_ints(tokens, slots)
+  uint16_t *qbuf;     // (tokens, H, 576)
+  float *part_ml;     // (slots, H, 2)
+  uint16_t *part_o;   // (slots, H, 512)
+};
+
+static void set_attn_attr();
+
+// Stages 4 - 6 for `tokens` <= DECODE_MAX_BATCH tokens: q (tokens, H, 192) with
+// the rope applied -> attn (tokens, H * 128), the cache rows already written.
+static int absorbed_attention(const amla_mla_args &a, const TokenMap &map, int tokens, int units, int slots,
+                              const uint16_t *q, const AbsorbedScratch &sc, uint16_t *attn, hipStream_t st,
+                              hipEvent_t const *ev = nullptr, int attn_repeat = 1) {
+  int rc;
+  const int B = tokens;
+  const uint8_t *wkvb = reinterpret_cast<const uint8_t *>(a.w_kv_b);
+  const uint16_t *gkv = reinterpret_cast<const uint16_t *>(a.gamma_kv);
+  set_attn_attr();
+  // 4. absorb W_UK into the query
+  mark(ev, 3, st);
+  const int tmax = mla_context_bound(a);
+  if (B <= AB_SEQ)
+    absorb_kernel<1><<<dim3(HEADS + 1, LORA / 128, 1), 256, 0, st>>>(q, wkvb, a.s_kv_b, gkv, B, sc.qbuf, map, tmax, units,
+                                                                     slots, sc.plan);
+  else
+    absorb_kernel<2><<<dim3(HEADS + 1, LORA / 128, (B + 2 * AB_SEQ - 1) / (2 * AB_SEQ)), 256, 0, st>>>(
+        q, wkvb, a.s_kv_b, gkv, B, sc.qbuf, map, tmax, units, slots, sc.plan);
+  if ((rc = check_launch("mla absorb"))) return rc;
+
+  // 5. attention over the latent cache, split over context
+  mark(ev, 4, st);
+  AttnParams ap = {};
+  ap.qbuf = sc.qbuf;
+  ap.ckv = reinterpret_cast<const uint16_t *>(a.ckv_cache);
+  ap.kpe = reinterpret_cast<const uint16_t *>(a.kpe_cache);
+  ap.ckv_bstride = (int64_t)a.max_seq * LORA; ap.kpe_bstride = (int64_t)a.max_seq * ROPE;
+  ap.rope_table = a.rope_table; ap.map = map; ap.tmax = tmax;
+  ap.units = units; ap.batch = B; ap.plan = sc.plan;
+  ap.scale_log2 = a.softmax_scale * 1.4426950408889634f;
+  ap.eps = a.eps;
+  ap.part_o = sc.part_o;
+  ap.part_ml = sc.part_ml;
+  for (int r = 0; r < attn_repeat; ++r) {
+    if (attn_head_groups(slots) == 2)
+      attn_kernel<1><<<dim3(slots, 2), 256, ATTN_LDS, st>>>(ap);
+    else
+      attn_kernel<2><<<dim3(slots), 256, ATTN_LDS, st>>>(ap);
+    if ((rc = check_launch("mla attention"))) return rc;
+  }
+
+  // 6. merge splits, W_UV
+  mark(ev, 5, st);
+  if (B <= 2)  // one sequence group: W_UV[h] split over two workgroups
+    combine_uv_kernel<4, 2, 2><<<dim3(2 * HEADS, 1), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
+  else if (B <= 8)
+    combine_uv_kernel<4, 2, 1><<<dim3(HEADS, (B + 3) / 4), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
+  else
+    combine_uv_kernel<16, 1, 1><<<dim3(HEADS, (B + 15) / 16), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
+  return check_launch("mla combine");
+}
+
+// ---- attention of a prefill over a long cache in latent space
+
+// Tokens per launch sequence: the new tokens of every sequence in as many
+// equal chunks as the limit of 64 needs.
+static int absorbed_chunk(int64_t tokens) {
+  const int64_t n = (tokens + DECODE_MAX_BATCH - 1) / DECODE_MAX_BATCH;
+  return (int)((tokens + n - 1) / n);
+}
+
+// Whether `batch` sequences of `seq_len` new tokens each over up to `context`
+// rows run in latent space (every new token reads the raw latent rows: work in
+// proportion to new tokens x rows) or decompressed (kv_b over every row, then
+// flash over 256-query blocks: in proportion to the rows alone while the
+// queries fit a block).  Times in us measured on MI355X: kv_b 0.041 per row,
+// flash 1.92 per 64-key tile and round of 256 workgroups, attn_kernel 2.25 per
+// 32-row tile of the longest split.  One sequence over 8192 rows: 50 new
+// tokens 170 against 620, about equal at 200; at 512 rows 8 new tokens.
+bool prefill_absorbed(int batch, int seq_len, int context) {
+  const double blocks = (seq_len + 255) / 256;
+  const double tiles = (context + 63) / 64, causal = 1.0 - 0.5 * seq_len / std::max(context, seq_len);
+  const double kvb = context <= 64 ? 8.0 : std::max(18.0, 0.041 * context);
+  const double flash = 8.0 + std::ceil(128 * blocks / 256) * 1.92 * tiles * (blocks > 1 ? causal : 1.0);
+  const double direct = batch * (10.0 + 0.0015 * context + kvb + flash);
+  const int64_t tokens = (int64_t)batch * seq_len;
+  const int n = absorbed_chunk(tokens);
+  int units, slots;
+  attn_units(n, context, units, slots);
+  const double split = std::ceil((double)n * ((context + TT - 1) / TT) / units);
+  const double chunk = (4.0 + 0.16 * n) + (10.0 + 2.25 * split) + (6.0 + units / 32.0 + 0.15 * n);
+  return (double)((tokens + n - 1) / n) * chunk < 0.9 * direct;
+}
+
+static size_t absorbed_scratch(int64_t tokens, int context, char *base, AbsorbedScratch *sc) {
+  const int chunk = absorbed_chunk(tokens), last = (int)(tokens - (tokens - 1) / chunk * chunk);
+  int units, slots, last_slots;  // a smaller last chunk may take more one-tile splits
+  attn_units(chunk, context, units, slots);
+  attn_units(last, context, units, last_slots);
+  slots = std::max(slots, last_slots);
+  size_t off = 0;
+  auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
+  const size_t plan = take(plan_ints(chunk, slots) * 4), qbuf = take((size_t)chunk * HEADS * QKD * 2),
+               ml = take((size_t)slots * HEADS * 2 * 4), po = take((size_t)slots * HEADS * LORA * 2);
+  if (sc)
+    *sc = AbsorbedScratch{reinterpret_cast<int32_t *>(base + plan), reinterpret_cast<uint16_t *>(base + qbuf),
+                          reinterpret_cast<float *>(base + ml), reinterpret_cast<uint16_t *>(base + po)};
+  return off;
+}
+
+size_t prefill_absorbed_ws_bytes(int batch, int seq_len, int context) {
+  return absorbed_scratch((int64_t)batch * seq_len, context, nullptr, nullptr);
+}
+
+int launch_prefill_absorbed(const amla_mla_args &a, const uint16_t *q, uint16_t *attn, char *ws, hipStream_t st) {
+  const int64_t tokens = (int64_t)a.batch * a.seq_len;
+  const int chunk = absorbed_chunk(tokens);
+  AbsorbedScratch sc;
+  absorbed_scratch(tokens, mla_context_bound(a), ws, &sc);
+  for (int64_t t0 = 0; t0 < tokens; t0 += chunk) {
+    const int n = (int)std::min<int64_t>(chunk, tokens - t0);
+    int units, slots;
+    attn_units(n, mla_context_bound(a), units, slots);
+    const int rc = absorbed_attention(a, TokenMap{a.positions, a.seq_len, (int)t0}, n, units, slots,
+                                      q + (size_t)t0 * HEADS * (NOPE + ROPE), sc, attn + (size_t)t0 * HEADS * VD, st);
+    if (rc) return rc;
+  }
+  return AMLA_OK;
+}
+
+// ---- decode
 
 static int decode_chunk(const amla_mla_args *a, hipStream_t st, hipEvent_t const *ev, int attn_repeat);
 
@@ -1518,57 +1672,15 @@ static int decode_chunk(const amla_mla_args *a, hipStream_t st, hipEvent_t const
   pb.part = reinterpret_cast<float *>(ws + L.lin);
   if ((rc = launch_gemv(pb, GEMV_QROPE, L.pb, st))) return rc;
 
-  // 4. absorb W_UK into the query
-  mark(ev, 3, st);
-  int32_t *plan = reinterpret_cast<int32_t *>(ws + L.plan);
-  const int tmax = mla_context_bound(*a);
-  if (B <= AB_SEQ)
-    absorb_kernel<1><<<dim3(HEADS + 1, LORA / 128, 1), 256, 0, st>>>(
-        q, reinterpret_cast<const uint8_t *>(a->w_kv_b), a->s_kv_b, reinterpret_cast<const uint16_t *>(a->gamma_kv), B,
-        qbuf, a->positions, tmax, L.units, L.slots, plan);
-  else
-    absorb_kernel<2><<<dim3(HEADS + 1, LORA / 128, (B + 2 * AB_SEQ - 1) / (2 * AB_SEQ)), 256, 0, st>>>(
-        q, reinterpret_cast<const uint8_t *>(a->w_kv_b), a->s_kv_b, reinterpret_cast<const uint16_t *>(a->gamma_kv), B,
-        qbuf, a->positions, tmax, L.units, L.slots, plan);
-  if ((rc = check_launch("mla absorb"))) return rc;
-
-  // 5. attention over the latent cache, split over context
-  mark(ev, 4, st);
-  AttnParams ap = {};
-  ap.qbuf = qbuf;
-  ap.ckv = reinterpret_cast<const uint16_t *>(a->ckv_cache);
-  ap.kpe = reinterpret_cast<const uint16_t *>(a->kpe_cache);
-  ap.ckv_bstride = (int64_t)a->max_seq * LORA; ap.kpe_bstride = (int64_t)a->max_seq * ROPE;
-  ap.rope_table = a->rope_table; ap.pos = a->positions; ap.tmax = tmax;
-  ap.units = L.units; ap.batch = B; ap.plan = plan;
-  ap.scale_log2 = a->softmax_scale * 1.4426950408889634f;
-  ap.eps = a->eps;
-  ap.part_o = reinterpret_cast<uint16_t *>(ws + L.part_o);
-  ap.part_ml = reinterpret_cast<float *>(ws + L.part_ml);
-  for (int r = 0; r < attn_repeat; ++r) {
-    if (attn_head_groups(L) == 2)
-      attn_kernel<1><<<dim3(L.slots, 2), 256, ATTN_LDS, st>>>(ap);
-    else
-      attn_kernel<2><<<dim3(L.slots), 256, ATTN_LDS, st>>>(ap);
-    if ((rc = check_launch("mla attention"))) return rc;
-  }
-
-  // 6. merge splits, W_UV
-  mark(ev, 5, st);
+  // 4. - 6. attention in latent space
+  AbsorbedScratch sc;
+  sc.plan = reinterpret_cast<int32_t *>(ws + L.plan);
+  sc.qbuf = qbuf;
+  sc.part_ml = reinterpret_cast<float *>(ws + L.part_ml);
+  sc.part_o = reinterpret_cast<uint16_t *>(ws + L.part_o);
   uint16_t *attn = reinterpret_cast<uint16_t *>(a->attn_out ? a->attn_out : ws + L.attn);
-  if (B <= 2)  // one sequence group: W_UV[h] split over two workgroups
-    combine_uv_kernel<4, 2, 2><<<dim3(2 * HEADS, 1), 512, 0, st>>>(
-        ap, reinterpret_cast<const uint8_t *>(a->w_kv_b), a->s_kv_b, reinterpret_cast<const uint16_t *>(a->gamma_kv), B,
-        attn);
-  else if (B <= 8)
-    combine_uv_kernel<4, 2, 1><<<dim3(HEADS, (B + 3) / 4), 512, 0, st>>>(
-        ap, reinterpret_cast<const uint8_t *>(a->w_kv_b), a->s_kv_b, reinterpret_cast<const uint16_t *>(a->gamma_kv), B,
-        attn);
-  else
-    combine_uv_kernel<16, 1, 1><<<dim3(HEADS, (B + 15) / 16), 512, 0, st>>>(
-        ap, reinterpret_cast<const uint8_t *>(a->w_kv_b), a->s_kv_b, reinterpret_cast<const uint16_t *>(a->gamma_kv), B,
-        attn);
-  if ((rc = check_launch("mla combine"))) return rc;
+  if ((rc = absorbed_attention(*a, TokenMap{a->positions, 1, 0}, B, L.units, L.slots, q, sc, attn, st, ev, attn_repeat)))
+    return rc;
 
   // 7. o_proj (+ residual in layer mode)
   mark(ev, 6, st);

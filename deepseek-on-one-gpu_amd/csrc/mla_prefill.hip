@@ -1,16 +1,12 @@
 // MLA prefill for gfx950: amla_mla_prefill replaces mla_attention for S >= 1
-// tokens per sequence with a causal mask (inference/ops.py:100-183, :172-177),
-// and the large-M block-FP8 GEMM that amla_fp8_linear uses for M > 64.
+// tokens per sequence with a causal mask (inference/ops.py:100-183, :172-177).
+// Its linears are those of fp8_linear.hip up to 64 rows and tile_gemm.hip above.
 //
-// Prefill keeps the reference's non-absorbed formulation (absorption would
-// cost more FLOPs at S = T): kv_b decompresses the RMS-normed latent rows once
-// per call (one GEMM), and causal flash attention runs per head with
-// d_qk = 128 + 64 (the rope key shared by all heads) and d_v = 128.
-//
-// GEMM (K3): C[m, n] = sum_k X[m, k] W[n, k] scale_inv[n/128, k/128], with
-//   256 x 256 workgroup tiles, LDS-DMA staging of fp8 weights and bf16
-//   activations, exact in-register fp8 -> bf16 conversion, 32x32x16 MFMAs and
-//   a running-scale accumulator for the 128 x 128 block scales.
+// Prefill keeps the reference's non-absorbed formulation while it is the
+// cheaper one (S comparable to T): kv_b decompresses the RMS-normed latent
+// rows once per call (one GEMM), and causal flash attention runs per head with
+// d_qk = 128 + 64 (the rope key shared by all heads) and d_v = 128.  A few new
+// tokens over a long cache run in latent space instead (mla_decode.hip).
 #include <math.h>
 
 #include <algorithm>
@@ -490,8 +486,9 @@ static int run_linear(const GemvParams &p, int mode, hipStream_t st, size_t lin_
 }
 
 struct PrefillLayout {
-  size_t xn, qa, qan, q, kvn, kpe, kvb, attn, lin, lin_bytes, total;
+  size_t xn, qa, qan, q, kvn, kpe, kvb, attn, lat, lin, lin_bytes, total;
   int Tmax;
+  bool absorbed;  // attention in latent space: no kv_b rows
 };
 
 static PrefillLayout prefill_layout(const amla_mla_args &a) {
@@ -505,9 +502,14 @@ static PrefillLayout prefill_layout(const amla_mla_args &a) {
   L.qa = take(M * a.q_lora * 2);
   L.qan = take(M * a.q_lora * 2);
   L.q = take(M * a.heads * HD * 2);
-  L.kvn = take((size_t)L.Tmax * a.kv_lora * 2);
-  L.kpe = take((size_t)L.Tmax * a.qk_rope * 2);
-  L.kvb = take((size_t)L.Tmax * a.heads * (a.qk_nope + a.v_dim) * 2);
+  L.absorbed = prefill_absorbed(a.batch, a.seq_len, L.Tmax);
+  if (L.absorbed) {
+    L.lat = take(prefill_absorbed_ws_bytes(a.batch, a.seq_len, L.Tmax));
+  } else {
+    L.kvn = take((size_t)L.Tmax * a.kv_lora * 2);
+    L.kpe = take((size_t)L.Tmax * a.qk_rope * 2);
+    L.kvb = take((size_t)L.Tmax * a.heads * (a.qk_nope + a.v_dim) * 2);
+  }
   L.attn = take(M * a.heads * a.v_dim * 2);
   // K-part sums of the skinny linears (M <= 64), or the K-split partial sums
   // of the large-M GEMMs
@@ -518,7 +520,7 @@ static PrefillLayout prefill_layout(const amla_mla_args &a) {
   };
   need((int)M, a.q_lora + a.kv_lora + a.qk_rope, a.hidden);
   need((int)M, a.heads * HD, a.q_lora);
-  need(L.Tmax, a.heads * HDv, a.kv_lora);
+  if (!L.absorbed) need(L.Tmax, a.heads * HDv, a.kv_lora);
   need((int)M, a.hidden, a.heads * a.v_dim);
   L.lin = take(lin);
   L.lin_bytes = lin;
@@ -599,11 +601,12 @@ int prefill_impl(const amla_mla_args *a, hipStream_t st) {
   pb.head_dim = HD; pb.nope = a->qk_nope;
   if ((rc = run_linear(pb, GEMV_QROPE, st, L.lin_bytes))) return rc;
 
+  if (L.absorbed && (rc = launch_prefill_absorbed(*a, q, attn, ws + L.lat, st))) return rc;
   const int T = L.Tmax;
   FlashParams fp = {};
   fp.q = q; fp.kvb = kvb; fp.kpe = kpe; fp.out = attn; fp.pos = a->positions; fp.S = S; fp.tmax = T;
   fp.scale_log2 = a->softmax_scale * 1.4426950408889634f;
-  for (int b = 0; b < B; ++b) {
+  for (int b = 0; b < (L.absorbed ? 0 : B); ++b) {
     const uint16_t *ckv_b = reinterpret_cast<const uint16_t *>(a->ckv_cache) + (size_t)b * a->max_seq * a->kv_lora;
     const uint16_t *kpe_b = reinterpret_cast<const uint16_t *>(a->kpe_cache) + (size_t)b * a->max_seq * a->qk_rope;
     // kv_a_layernorm of every cached row, then kv_b (inference/ops.py:148-151)

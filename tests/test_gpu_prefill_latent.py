@@ -1,0 +1,79 @@
+"""Prefill of a few new tokens over a filled cache, where the attention runs in latent space: one
+token and many, several sequences with their own start, more tokens than one launch holds, tile
+and split edges, chosen and not; against the oracle per sequence (its roundings), per head and
+after o_proj, with the cache rows written."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import ref_ops as R
+from amla import ops, synth
+from amla._lib import lib
+from amla.config import DeepSeekConfig
+from _tol import assert_bf16_ulps, assert_heads_parity, assert_parity
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+CFG = DeepSeekConfig()
+
+
+@pytest.fixture(scope="module")
+def layer():
+    return synth.make_layer(CFG, "latent-prefill")
+
+
+def _gpu(aw):
+    return {k: (tuple(t.to(DEV) for t in v) if isinstance(v, tuple) else v.to(DEV)) for k, v in aw.items()}
+
+
+@pytest.mark.parametrize("S,starts", [(2, [1023]), (7, [640]), (33, [1500]), (65, [1951]), (9, [513, 0, 1200, 70]),
+                                      (40, [900, 31])])
+def test_new_tokens_over_a_cache(layer, S, starts):
+    print(f"[case] latent prefill S={S} starts={starts}", flush=True)
+    B = len(starts)
+    rows = max(starts) + S + 5
+    hidden = synth.make_hidden(CFG, B, S, f"lp{S}")
+    ckv, kpe = synth.make_kv_cache(CFG, B, rows, starts, f"lp{S}")
+    tab = R.precompute_rope_freqs(CFG, rows)
+    cref, kref = ckv.clone(), kpe.clone()
+    want_h, want = R.mla_attention_per_sequence_parts(hidden, layer.attn_weights, (cref, kref), starts, tab, CFG)
+    cd, kd = ckv.to(DEV), kpe.to(DEV)
+    heads = torch.empty(B, S, CFG.num_attention_heads * CFG.v_head_dim, dtype=torch.bfloat16, device=DEV)
+    got = ops.mla_attention(hidden.to(DEV), _gpu(layer.attn_weights), (cd, kd), starts, tab.to(DEV), CFG, attn_out=heads)
+    torch.cuda.synchronize()
+    assert_heads_parity(heads, want_h, CFG.num_attention_heads, f"latent prefill S={S} heads")
+    assert_parity(got, want, f"latent prefill S={S}")
+    for b, p in enumerate(starts):
+        assert_bf16_ulps(cd[b, p:p + S], cref[b, p:p + S], 2, "new latent rows")
+        assert_bf16_ulps(kd[b, p:p + S], kref[b, p:p + S], 2, "new rope rows")
+        assert torch.equal(cd[b, :p].cpu(), ckv[b, :p]) and torch.equal(cd[b, p + S:].cpu(), ckv[b, p + S:])
+
+
+def test_prompt_and_token_by_token_agree(layer):
+    """The same 12 new tokens at once (latent attention over 1024 + 12 rows) and one decode step
+    each: the same rows in the cache and the same outputs to the bf16 bar."""
+    S, p, rows = 12, 1024, 1100
+    aw = _gpu(layer.attn_weights)
+    hidden = synth.make_hidden(CFG, 1, S, "lp-step").to(DEV)
+    ckv, kpe = (t.to(DEV) for t in synth.make_kv_cache(CFG, 1, rows, p, "lp-step"))
+    tab = R.precompute_rope_freqs(CFG, rows).to(DEV)
+    c2, k2 = ckv.clone(), kpe.clone()
+    at_once = ops.mla_attention(hidden, aw, (ckv, kpe), p, tab, CFG)
+    steps = torch.cat([ops.mla_attention(hidden[:, i:i + 1], aw, (c2, k2), p + i, tab, CFG) for i in range(S)], dim=1)
+    torch.cuda.synchronize()
+    assert_parity(at_once, steps, "prompt vs token by token")
+    assert_bf16_ulps(ckv, c2, 2, "cache rows")
+
+
+def test_scratch_covers_a_smaller_last_chunk():
+    """65 tokens run as 33 + 32: the smaller chunk may be cut into more one-tile splits."""
+    from amla._lib import MlaArgs
+    a = MlaArgs()
+    a.batch, a.seq_len, a.hidden, a.heads, a.q_lora, a.kv_lora = 1, 65, 7168, 128, 1536, 512
+    a.qk_nope, a.qk_rope, a.v_dim = 128, 64, 128
+    sizes = []
+    for ctx in (65, 128, 600, 4096, 32768):
+        a.max_seq = a.rope_rows = a.max_context = ctx
+        sizes.append(lib().amla_mla_prefill_workspace_bytes(ctypes.byref(a)))
+    assert all(s > 0 for s in sizes)
