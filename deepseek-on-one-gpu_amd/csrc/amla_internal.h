@@ -149,6 +149,7 @@ struct MoeTileParams {
   uint16_t *y;
   int ldx, ldy, K, N;
   int ntiles;  // column tiles (set by the launch)
+  bool wide;   // x (every row a row list may name) is 4 GB or more
 };
 int launch_tile_sched(const MoeTileParams &p, const MoeSched &s, int max_entries, hipStream_t stream);
 // The same tiles from a host list (amla_moe_experts): rows first .. first +

@@ -753,7 +753,7 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
     pd.seq_len = 1;
     const GemvPlan plan_g = plan_gemv_grouped(std::max(max_small, 1), 2 * n, D);
     const GemvPlan plan_d = plan_gemv_grouped(std::max(max_small, 1), D, n);
-    const MoeTileParams tg = {xs, hb, D, n, D, n, 0}, td = {hb, ys, n, D, n, D, 0};
+    const MoeTileParams tg = {xs, hb, D, n, D, n, 0, false}, td = {hb, ys, n, D, n, D, 0, false};
     for (int pass = 0; pass < 2; ++pass) {
       // groups of up to 16 rows: grouped skinny GEMMs, GEMV_MAX_GROUPS experts per launch
       const GemvPlan &pl = pass == 0 ? plan_g : plan_d;
@@ -1053,7 +1053,8 @@ int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, co
   // expert_out rows scatter[] = down(h)
   const MoeSched gu_s = {weight_table, ent, count, E, 0, gather}, dn_s = {weight_table, ent, count, E, 1, scatter};
   if (L.tiles) {
-    const MoeTileParams tg = {hid, hb, D, n, D, n, 0}, td = {hb, eout, n, D, n, D, 0};
+    const MoeTileParams tg = {hid, hb, D, n, D, n, 0, m * d * 2 > (int64_t)UINT32_MAX},
+                        td = {hb, eout, n, D, n, D, 0, false};
     if ((rc = launch_tile_sched(tg, gu_s, L.max_entries, st))) return rc;
     return launch_tile_sched(td, dn_s, L.max_entries, st);
   }

@@ -56,6 +56,7 @@ struct TileArgs {
   int ldx, ldy, K, rows;
   int kb0, kb1;          // 128-wide K blocks
   bool two;              // segment 1 is stored (always multiplied)
+  bool wide;             // byte offsets of x rows may not fit 32 bits
 };
 
 // A tile's sums: acc[segment][row group of 32], in units of s_run[segment].
@@ -79,34 +80,53 @@ struct TileMain {
   const int j32 = lane & 31, hh = lane >> 5;
 
   // copies: the wave's own 2 x 32 weight rows (16 rows of 64 B each) and its
-  // quarter of the activation rows (8 rows of 128 B each)
-  const uint8_t *wsrc[2][2];
+  // quarter of the activation rows (8 rows of 128 B each), as scalar bases that
+  // advance with the stage plus 32-bit lane offsets
+  uint32_t woff[2][2], xoff[NJ];
 #pragma unroll
   for (int g = 0; g < 2; ++g)
 #pragma unroll
     for (int c = 0; c < 2; ++c)
-      wsrc[g][c] = a.w[g] + (size_t)min(32 * wave + 16 * c + (lane >> 2), a.wrows[g] - 1) * a.K +
+      woff[g][c] = (uint32_t)min(32 * wave + 16 * c + (lane >> 2), a.wrows[g] - 1) * a.K +
                    16 * ((lane & 3) ^ ((lane >> 4) & 3));
-  const uint8_t *xsrc[NJ];
 #pragma unroll
   for (int c = 0; c < NJ; ++c) {
     const int r = 8 * (NJ * wave + c) + (lane >> 3);
     const int rc = min(r, a.rows - 1);  // rows past the tile repeat its last row (not stored)
-    const int64_t xr = a.xrow ? a.xrow[rc] : rc;
-    xsrc[c] = reinterpret_cast<const uint8_t *>(a.x + xr * a.ldx) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+    const uint32_t xr = a.xrow ? a.xrow[rc] : rc;
+    // a.wide: x is 4 GB or more, the offset does not fit and is formed per copy
+    xoff[c] = a.wide ? xr : xr * (uint32_t)(a.ldx * 2) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
   }
   auto dma = [&](int it, int stg) {
     uint8_t *st = tsm + stg * STAGE;
+    // (scalar base + 32-bit lane offset per copy: with the bases or the offsets'
+    // extension visible outside the loop, each copy costs a 64-bit vector add)
+    auto opaque = [](uint32_t v) {
+      asm volatile("" : "+v"(v));
+      return v;
+    };
+    typedef const __attribute__((address_space(1))) uint8_t *gptr;
+    gptr wb[2] = {(gptr)(a.w[0] + it * T_BK), (gptr)(a.w[1] + it * T_BK)};
+    gptr xb = (gptr)(reinterpret_cast<const uint8_t *>(a.x) + it * T_XROW);
+    asm volatile("" : "+s"(wb[0]));
+    asm volatile("" : "+s"(wb[1]));
+    asm volatile("" : "+s"(xb));
 #pragma unroll
     for (int g = 0; g < 2; ++g)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        __builtin_amdgcn_global_load_lds(wsrc[g][c] + it * T_BK,
-                                         LDS_PTR(st + (128 * g + 32 * wave + 16 * c) * T_BK), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(wb[g] + opaque(woff[g][c]), LDS_PTR(st + (128 * g + 32 * wave + 16 * c) * T_BK), 16, 0, 0);
+    if (!a.wide) {
 #pragma unroll
-    for (int c = 0; c < NJ; ++c)
-      __builtin_amdgcn_global_load_lds(xsrc[c] + it * T_XROW, LDS_PTR(st + T_WBYTES + 8 * (NJ * wave + c) * T_XROW),
-                                       16, 0, 0);
+      for (int c = 0; c < NJ; ++c)
+        __builtin_amdgcn_global_load_lds(xb + opaque(xoff[c]), LDS_PTR(st + T_WBYTES + 8 * (NJ * wave + c) * T_XROW), 16, 0, 0);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NJ; ++c)
+        __builtin_amdgcn_global_load_lds(
+            xb + (size_t)xoff[c] * a.ldx * 2 + 16 * ((lane & 7) ^ ((4 * (NJ * wave + c) + (lane >> 4)) & 7)),
+            LDS_PTR(st + T_WBYTES + 8 * (NJ * wave + c) * T_XROW), 16, 0, 0);
+    }
   };
 
   uint32_t aoff[2], boff[2][2];
@@ -141,7 +161,7 @@ struct TileMain {
   const int it0 = 2 * a.kb0, iters = 2 * a.kb1;
 #pragma unroll
   for (int i = 0; i < NST - 1; ++i) dma(it0 + i, i);  // a block is 2 >= NST - 1 stages
-  int stg = 0;
+  int ring = 0;
   // One stage of 64: four sub-steps of 16 (K 32 pr + 16 hh + 8 s2 .. +7 of each
   // half-wave).  While a sub-step multiplies, the fragments of the next are
   // read and converted between its MFMAs.  The rescaling between two blocks
@@ -158,6 +178,7 @@ struct TileMain {
   };
   auto stage = [&](int it, auto odd_c, const float *r) {
     constexpr bool ODD = decltype(odd_c)::value;
+    const int stg = NST == 2 ? (ODD ? 1 : 0) : ring;  // two stages: even blocks' halves in 0, odd ones in 1
     if (NST == 3 && it + 1 < iters) wait_vmcnt<COPIES>();
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
@@ -217,7 +238,7 @@ struct TileMain {
           __builtin_amdgcn_sched_barrier(0);
         }
     }
-    stg = stg == NST - 1 ? 0 : stg + 1;
+    if (NST == 3) ring = ring == NST - 1 ? 0 : ring + 1;
   };
   float r[2] = {1.f, 1.f};
   for (int kb = a.kb0; kb < a.kb1; ++kb) {
@@ -408,6 +429,7 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(GemvParams p, bool 
   a.kb1 = kb1;
   a.x = p.x + (size_t)m0 * p.ldx;
   a.xrow = nullptr;
+  a.wide = false;  // 128 rows from its base
   // segment = a run of up to 128 rows of one weight: the first weight's
   // segments come before the second's (n_split % 128 == 0)
   int n0[2];
@@ -532,6 +554,7 @@ AMLA_DEV void moe_tile(const MoeTileParams &p, const TileGroup &g, int nt, const
   a.ldy = p.ldy;
   const int KB = p.K >> 7;
   a.x = xrow ? p.x : p.x + (size_t)g.first * p.ldx;
+  a.wide = xrow && p.wide;
   a.xrow = xrow;
   a.y = (yrow ? p.y : p.y + (size_t)g.first * p.ldy) + nt * (GATEUP ? 128 : 256);
   a.yrow = yrow;

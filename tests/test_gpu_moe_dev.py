@@ -267,3 +267,29 @@ def test_moe_experts_dev_few_tokens_repeating_one_expert(m, K):
     got, hdr = _run_dev(h, idx, _stacked(table, E), E, i)
     assert hdr[0] == m * K and hdr[3] == 0
     assert_parity(got, _want(h, idx, table), f"moe_experts_dev repeated m={m} K={K}")
+
+
+def test_moe_experts_dev_hidden_of_4_gb():
+    """Hidden states of more than 4 GB: a gathered row's byte offset does not fit 32 bits.  Rows
+    from both ends and the middle equal the same rows in a small call bit for bit (a row's sums do
+    not depend on its tile)."""
+    m, d, i, E = 65536, 32896, 256, 2
+    print(f"[case] moe_experts_dev hidden {m * d * 2 / 2 ** 30:.2f} GiB", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(11)
+    h = torch.empty(m, d, dtype=torch.bfloat16, device=DEV)
+    for r in range(0, m, 8192):
+        h[r:r + 8192] = torch.randn(8192, d, generator=g, device=DEV, dtype=torch.bfloat16)
+    stacked = {}
+    for k, (n, kk) in (("gate_proj", (i, d)), ("up_proj", (i, d)), ("down_proj", (d, i))):
+        q = (torch.randn(E, n, kk, generator=g, device=DEV) * 60).clamp(-448, 448).to(torch.float8_e4m3fn)
+        stacked[k] = (q, torch.rand(E, n // 128, kk // 128, generator=g, device=DEV) * 1e-3)
+    idx = torch.arange(m, device=DEV).remainder(3).clamp(max=1).view(m, 1)
+    table, n_inter = ops._stacked_device_table(stacked, E, d, torch.device(DEV))
+    out = torch.empty(m, 1, d, dtype=torch.bfloat16, device=DEV)
+    ops._moe_experts_dev_call(h, idx, table, n_inter, E, out)
+    rows = torch.cat([torch.arange(0, 40), torch.arange(32750, 32790), torch.arange(m - 40, m)]).to(DEV)
+    few = torch.empty(rows.numel(), 1, d, dtype=torch.bfloat16, device=DEV)
+    ops._moe_experts_dev_call(h[rows].contiguous(), idx[rows].contiguous(), table, n_inter, E, few)
+    torch.cuda.synchronize()
+    assert torch.isfinite(few.float()).all() and few.float().abs().max() > 0
+    assert torch.equal(out[rows], few)
