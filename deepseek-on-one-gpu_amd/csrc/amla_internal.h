@@ -176,7 +176,8 @@ struct GemmSplit {
   int n_tiles, m_tiles;  // tiles of 256 columns (SILU: 128) x 128 rows
   int full;              // tiles with the whole K
   int rest;              // later tiles, cut into
-  int parts;             // K parts each
+  int parts;             // K parts each,
+  int group;             // in runs of this many tiles per part
   int full_blocks;       // workgroups before the parts
   float *partial;        // [split tile][part][TILE_PART_F32] in the lanes' own order
   size_t bytes;          // of partial

@@ -319,10 +319,17 @@ AMLA_DEV void tile_store(const TileArgs &a, const TileSums<NJ> &ts) {
 // The GEMM of launch_gemm (GemvMode epilogues): tiles of 256 weight rows x 128
 // activation rows.  Workgroup i runs on XCD i % 8: each XCD takes a contiguous
 // run of the tiles in panels of 8 column tiles, row tiles within a panel, so
-// the 64 tiles it holds at a time share 8 + 8 tile operands through its L2.
+// the 64 tiles it holds at a time share 8 + 8 tile operands through its L2;
+// with up to 8 row tiles the row tiles of a column tile come together (the
+// weights are then the larger operand).
 constexpr int TL_PANEL = 8;
 
 AMLA_DEV void tile_coords(int t, int n_tiles, int m_tiles, int &nt, int &mt) {
+  if (m_tiles <= TL_PANEL) {
+    nt = t / m_tiles;
+    mt = t - nt * m_tiles;
+    return;
+  }
   const int per = TL_PANEL * m_tiles, p = t / per, r = t - p * per;
   const int width = min(TL_PANEL, n_tiles - p * TL_PANEL);
   mt = r / width;
@@ -412,11 +419,14 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(GemvParams p, bool 
   } else {
     const int l = xcd_run(blockIdx.x - sp.full_blocks, sp.rest * sp.parts);
     if (l < 0) return;
-    const int st = l / sp.parts, q = l - st * sp.parts;
+    // K part q of `group` tiles at a time: the row tiles of a column tile read
+    // the same weights
+    const int per = sp.group * sp.parts, g = l / per, r = l - g * per;
+    const int q = r / sp.group, st = g * sp.group + r - q * sp.group;
     t = sp.full + st;
     kb0 = q * KB / sp.parts;
     kb1 = (q + 1) * KB / sp.parts;
-    partial = sp.partial + (size_t)l * TILE_PART_F32;
+    partial = sp.partial + (size_t)(st * sp.parts + q) * TILE_PART_F32;
   }
   int nt, mt;
   tile_coords(t, sp.n_tiles, sp.m_tiles, nt, mt);
@@ -646,9 +656,12 @@ int launch_tile_grouped(const MoeTileParams &p0, const TileGroups &gr, bool down
 
 // Workgroups: 512 run at a time (two per CU).  Tiles past the last full round
 // are cut into K parts where that shortens the launch.  Measured on MI355X, a
-// 128-wide K block of a 128-row tile takes 3.9 us with two workgroups per CU
-// and 1.8 us with one; the partial sums (128 KB per part) cross memory twice
-// at ~4 TB/s, and the finishing pass costs about 5 us of its own.
+// 128-wide K block of a 128-row tile takes 3.7 us with two workgroups per CU
+// and 2.1 us with one; writing and reading a part's sums (128 KB) adds about
+// 0.03 us each, the finishing pass 5 us of its own.  Against every part count
+// from 1 to 16 at N = 576, 4096, 7168, 24576 and 100-1000 rows the plan is
+// within 5 % of the best (7168 x 16384: 100 rows 50 us in 9 parts, 228 in one;
+// 333 rows 106 in 3; 1000 rows 242 in 2, 267 in one).
 GemmSplit plan_gemm_split(int M, int N, int K, int mode) {
   GemmSplit sp = {};
   const int cols = mode == GEMV_SILU ? 128 : 256;
@@ -658,12 +671,12 @@ GemmSplit plan_gemm_split(int M, int N, int K, int mode) {
   const int KB = K / 128;
   const int full = tiles / 512 * 512, rest = tiles - full;
   const double nj = (std::min(M, TILE_ROWS) + 31) / 32;
-  const double one = 0.9 + 0.225 * nj, two = std::max(1.3, 0.975 * nj);  // us per K block
+  const double one = 0.9 + 0.3 * nj, two = std::max(1.3, 0.925 * nj);  // us per K block
   auto cost_of = [&](int parts) {
     const int items = rest * parts, last = items % 512;
     const double kb = (KB + parts - 1) / parts;
     const double rounds = items / 512 * two + (last == 0 ? 0.0 : last <= 256 ? one : two);
-    return rounds * kb + (parts > 1 ? 5.0 + items * 0.064 * nj / 4 : 0.0);
+    return rounds * kb + (parts > 1 ? 5.0 + items * 0.03 * nj / 4 : 0.0);
   };
   int best = 1;
   double best_cost = rest ? cost_of(1) : 0.0;
@@ -677,6 +690,7 @@ GemmSplit plan_gemm_split(int M, int N, int K, int mode) {
   sp.full = best > 1 ? full : tiles;
   sp.rest = tiles - sp.full;
   sp.parts = best;
+  sp.group = sp.m_tiles <= TL_PANEL && sp.full % sp.m_tiles == 0 ? sp.m_tiles : 1;
   sp.full_blocks = (sp.full + 7) / 8 * 8;
   sp.bytes = (size_t)sp.rest * (best > 1 ? best : 0) * TILE_PART_F32 * 4;
   return sp;
