@@ -342,7 +342,7 @@ AMLA_DEV int xcd_run(int i, int n) {
 }
 
 template <int MODE, int NJ>
-AMLA_DEV void tile_linear_body(const GemvParams &p, const TileArgs &a, const int (&n0)[2], int m0, bool staged,
+AMLA_DEV void tile_linear_body(const GemvParams &p, const TileArgs &a, int n0, int n1, int m0, bool staged,
                                float *partial) {
   extern __shared__ __align__(16) uint8_t tsm[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -377,7 +377,7 @@ AMLA_DEV void tile_linear_body(const GemvParams &p, const TileArgs &a, const int
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int c = 32 * wave + 8 * q + 4 * hh;
-          if (c < a.wrows[g] && (g == 0 || a.two)) pstore4<MODE == GEMV_SILU ? GEMV_PLAIN : MODE>(p, m0 + r, n0[g] + c, sums(g, j, q));
+          if (c < a.wrows[g] && (g == 0 || a.two)) pstore4<MODE == GEMV_SILU ? GEMV_PLAIN : MODE>(p, m0 + r, (g ? n1 : n0) + c, sums(g, j, q));
         }
     }
     return;
@@ -402,9 +402,11 @@ AMLA_DEV void tile_linear_body(const GemvParams &p, const TileArgs &a, const int
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   const int g = (tid >> 4) & 1, c = 8 * (tid & 15);
-  if (c < a.wrows[g] && (g == 0 || a.two))
+  const int n = (g ? n1 : n0) + c;
+  if (c < (g ? a.wrows[1] : a.wrows[0]) && (g == 0 || a.two))
     for (int r = tid >> 5; r < a.rows; r += 8)
-      pstore8<MODE == GEMV_SILU ? GEMV_PLAIN : MODE>(p, m0 + r, n0[g] + c, *reinterpret_cast<const u32x4 *>(tsm + r * T_PITCH_Y + (tid & 31) * 16));
+      pstore8<MODE == GEMV_SILU ? GEMV_PLAIN : MODE>(
+          p, m0 + r, n, *reinterpret_cast<const u32x4 *>(tsm + r * T_PITCH_Y + (tid & 31) * 16));
 }
 
 // Workgroups [0, full): whole tiles; then K part (i - full) % parts of tile full + (i - full) / parts.
@@ -471,10 +473,10 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(GemvParams p, bool 
     a.wrows[g] = min(128, (p.w1 && !second ? p.n_split : p.N) - n);
   }
   switch ((a.rows + 31) >> 5) {
-    case 1: tile_linear_body<MODE, 1>(p, a, n0, m0, staged, partial); break;
-    case 2: tile_linear_body<MODE, 2>(p, a, n0, m0, staged, partial); break;
-    case 3: tile_linear_body<MODE, 3>(p, a, n0, m0, staged, partial); break;
-    default: tile_linear_body<MODE, 4>(p, a, n0, m0, staged, partial); break;
+    case 1: tile_linear_body<MODE, 1>(p, a, n0[0], n0[1], m0, staged, partial); break;
+    case 2: tile_linear_body<MODE, 2>(p, a, n0[0], n0[1], m0, staged, partial); break;
+    case 3: tile_linear_body<MODE, 3>(p, a, n0[0], n0[1], m0, staged, partial); break;
+    default: tile_linear_body<MODE, 4>(p, a, n0[0], n0[1], m0, staged, partial); break;
   }
 }
 
