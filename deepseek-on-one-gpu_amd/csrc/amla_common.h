@@ -79,6 +79,14 @@ AMLA_DEV f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 }
 
 AMLA_DEV u32x4 ldg16(const void *p) { return *reinterpret_cast<const u32x4 *>(p); }
+// eight bf16 values at any 2-byte alignment (the branch is uniform: `base` is)
+AMLA_DEV u32x4 ldg8_bf16(const uint16_t *base, int i) {
+  if ((reinterpret_cast<uintptr_t>(base) & 15) == 0) return ldg16(base + i);
+  u32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = (uint32_t)base[i + 2 * e] | (uint32_t)base[i + 2 * e + 1] << 16;
+  return v;
+}
 AMLA_DEV u32x2 ldg8(const void *p) { return *reinterpret_cast<const u32x2 *>(p); }
 
 AMLA_DEV u32x4 ldg16_nt(const void *p) {

@@ -93,6 +93,14 @@ struct TokenMap {
     const int b = seq(i);
     return start[b] + (first + i - b * seq_len);
   }
+  // decode: known at compile time (the division and the second position term
+  // in front of every workgroup's first loads are gone)
+  template <bool DECODE> AMLA_DEV void fix() {
+    if constexpr (DECODE) {
+      seq_len = 1;
+      first = 0;
+    }
+  }
   // context of token i: cache rows [0, pos], clamped to the bound
   AMLA_DEV int context(int i, int tmax) const { return min(pos(i) + 1, tmax); }
 };
@@ -231,7 +239,7 @@ constexpr int AB_OPITCH = 128 * 2 + 16;   // bytes per output row (bf16)
 
 // RT row tiles of 16 sequences per workgroup (2 above 16 sequences: each
 // W_UK fragment read feeds both, and the quarter is read once per 32)
-template <int RT>
+template <int RT, bool DECODE>
 __global__ __launch_bounds__(256) void absorb_kernel(const uint16_t *__restrict__ q,  // (B, H, 192)
                                                      const uint8_t *__restrict__ wkvb,
                                                      const float *__restrict__ skvb,
@@ -239,6 +247,7 @@ __global__ __launch_bounds__(256) void absorb_kernel(const uint16_t *__restrict_
                                                      uint16_t *__restrict__ qbuf,
                                                      TokenMap map, int tmax, int units,
                                                      int slots, int32_t *__restrict__ plan) {
+  map.template fix<DECODE>();
   typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
   typedef int v2i __attribute__((ext_vector_type(2)));
   constexpr int NS = RT * AB_SEQ;  // sequences of the workgroup
@@ -579,8 +588,9 @@ AMLA_DEV float max_lane_groups(float v) {
 // scheduled before it.  Counting only this code's own reads is safe: LDS
 // operations complete in order, so any other LDS operation issued in between
 // only makes a wait stricter; nothing in the loop uses scalar memory loads.
-template <int NTW>
+template <int NTW, bool DECODE>
 __global__ __launch_bounds__(256, 1) void attn_kernel(AttnParams p) {
+  p.map.template fix<DECODE>();
   static_assert(NTW == 1 || NTW == 2, "16 or 32 heads per wave");
   constexpr int HPW = 16 * NTW;  // heads per wave (scores)
   constexpr int HG = 4 * HPW;    // heads of the workgroup
@@ -1141,11 +1151,12 @@ AMLA_DEV void recompute_split(const AttnParams &p, int b, int h, const SeqSplits
 //   out[b][v] = W_UV[h][v] . lat[b] by 16x16x32 MFMAs: A = W_UV rows (fp8
 //     converted exactly), B = lat of the SQ sequences (columns past them
 //     zero); wave w produces rows v = 16w .. 16w+15.
-template <int SQ, int WPS, int VH>
+template <int SQ, int WPS, int VH, bool DECODE>
 __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const uint8_t *__restrict__ wkvb,
                                                          const float *__restrict__ skvb,
                                                          const uint16_t *__restrict__ gamma, int B,
                                                          uint16_t *__restrict__ attn) {
+  ap.map.template fix<DECODE>();
   constexpr int NU = SQ * WPS;    // merge units
   constexpr int XB = SQ > 4 ? 8 : 20;  // splits in flight per wave (a batch)
   constexpr int WMAX = 256;       // splits per sequence
@@ -1282,7 +1293,7 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
     }
     const float inv = 1.f / L;
     const float sc = bsc[(8 * lane) / 128];
-    const u32x4 gm = *reinterpret_cast<const u32x4 *>(gamma + 8 * lane);
+    const u32x4 gm = DECODE ? ldg16(gamma + 8 * lane) : ldg8_bf16(gamma, 8 * lane);
     u32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -1450,6 +1461,7 @@ static void set_attn_attr();
 
 // Stages 4 - 6 for `tokens` <= DECODE_MAX_BATCH tokens: q (tokens, H, 192) with
 // the rope applied -> attn (tokens, H * 128), the cache rows already written.
+template <bool DECODE>
 static int absorbed_attention(const amla_mla_args &a, const TokenMap &map, int tokens, int units, int slots,
                               const uint16_t *q, const AbsorbedScratch &sc, uint16_t *attn, hipStream_t st,
                               hipEvent_t const *ev = nullptr, int attn_repeat = 1) {
@@ -1462,10 +1474,10 @@ static int absorbed_attention(const amla_mla_args &a, const TokenMap &map, int t
   mark(ev, 3, st);
   const int tmax = mla_context_bound(a);
   if (B <= AB_SEQ)
-    absorb_kernel<1><<<dim3(HEADS + 1, LORA / 128, 1), 256, 0, st>>>(q, wkvb, a.s_kv_b, gkv, B, sc.qbuf, map, tmax, units,
+    absorb_kernel<1, DECODE><<<dim3(HEADS + 1, LORA / 128, 1), 256, 0, st>>>(q, wkvb, a.s_kv_b, gkv, B, sc.qbuf, map, tmax, units,
                                                                      slots, sc.plan);
   else
-    absorb_kernel<2><<<dim3(HEADS + 1, LORA / 128, (B + 2 * AB_SEQ - 1) / (2 * AB_SEQ)), 256, 0, st>>>(
+    absorb_kernel<2, DECODE><<<dim3(HEADS + 1, LORA / 128, (B + 2 * AB_SEQ - 1) / (2 * AB_SEQ)), 256, 0, st>>>(
         q, wkvb, a.s_kv_b, gkv, B, sc.qbuf, map, tmax, units, slots, sc.plan);
   if ((rc = check_launch("mla absorb"))) return rc;
 
@@ -1484,20 +1496,20 @@ static int absorbed_attention(const amla_mla_args &a, const TokenMap &map, int t
   ap.part_ml = sc.part_ml;
   for (int r = 0; r < attn_repeat; ++r) {
     if (attn_head_groups(slots) == 2)
-      attn_kernel<1><<<dim3(slots, 2), 256, ATTN_LDS, st>>>(ap);
+      attn_kernel<1, DECODE><<<dim3(slots, 2), 256, ATTN_LDS, st>>>(ap);
     else
-      attn_kernel<2><<<dim3(slots), 256, ATTN_LDS, st>>>(ap);
+      attn_kernel<2, DECODE><<<dim3(slots), 256, ATTN_LDS, st>>>(ap);
     if ((rc = check_launch("mla attention"))) return rc;
   }
 
   // 6. merge splits, W_UV
   mark(ev, 5, st);
   if (B <= 2)  // one sequence group: W_UV[h] split over two workgroups
-    combine_uv_kernel<4, 2, 2><<<dim3(2 * HEADS, 1), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
+    combine_uv_kernel<4, 2, 2, DECODE><<<dim3(2 * HEADS, 1), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
   else if (B <= 8)
-    combine_uv_kernel<4, 2, 1><<<dim3(HEADS, (B + 3) / 4), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
+    combine_uv_kernel<4, 2, 1, DECODE><<<dim3(HEADS, (B + 3) / 4), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
   else
-    combine_uv_kernel<16, 1, 1><<<dim3(HEADS, (B + 15) / 16), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
+    combine_uv_kernel<16, 1, 1, DECODE><<<dim3(HEADS, (B + 15) / 16), 512, 0, st>>>(ap, wkvb, a.s_kv_b, gkv, B, attn);
   return check_launch("mla combine");
 }
 
@@ -1562,7 +1574,7 @@ int launch_prefill_absorbed(const amla_mla_args &a, const uint16_t *q, uint16_t 
     const int n = (int)std::min<int64_t>(chunk, tokens - t0);
     int units, slots;
     attn_units(n, mla_context_bound(a), units, slots);
-    const int rc = absorbed_attention(a, TokenMap{a.positions, a.seq_len, (int)t0}, n, units, slots,
+    const int rc = absorbed_attention<false>(a, TokenMap{a.positions, a.seq_len, (int)t0}, n, units, slots,
                                       q + (size_t)t0 * HEADS * (NOPE + ROPE), sc, attn + (size_t)t0 * HEADS * VD, st);
     if (rc) return rc;
   }
@@ -1679,7 +1691,7 @@ static int decode_chunk(const amla_mla_args *a, hipStream_t st, hipEvent_t const
   sc.part_ml = reinterpret_cast<float *>(ws + L.part_ml);
   sc.part_o = reinterpret_cast<uint16_t *>(ws + L.part_o);
   uint16_t *attn = reinterpret_cast<uint16_t *>(a->attn_out ? a->attn_out : ws + L.attn);
-  if ((rc = absorbed_attention(*a, TokenMap{a->positions, 1, 0}, B, L.units, L.slots, q, sc, attn, st, ev, attn_repeat)))
+  if ((rc = absorbed_attention<true>(*a, TokenMap{a->positions, 1, 0}, B, L.units, L.slots, q, sc, attn, st, ev, attn_repeat)))
     return rc;
 
   // 7. o_proj (+ residual in layer mode)
@@ -1702,10 +1714,9 @@ static bool g_attr_set = false;
 static void set_attn_attr() {
   if (!g_attr_set) {
     // Opt in to more than 64 KB of dynamic LDS (gfx950 has 160 KB per CU).
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_kernel<1>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)ATTN_LDS);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_kernel<2>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)ATTN_LDS);
+    for (const void *fn : {reinterpret_cast<const void *>(attn_kernel<1, true>), reinterpret_cast<const void *>(attn_kernel<2, true>),
+                           reinterpret_cast<const void *>(attn_kernel<1, false>), reinterpret_cast<const void *>(attn_kernel<2, false>)})
+      (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ATTN_LDS);
     (void)hipGetLastError();
     g_attr_set = true;
   }
