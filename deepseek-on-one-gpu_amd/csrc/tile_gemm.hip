@@ -664,6 +664,14 @@ int launch_tile_grouped(const MoeTileParams &p0, const TileGroups &gr, bool down
 // from 1 to 16 at N = 576, 4096, 7168, 24576 and 100-1000 rows the plan is
 // within 5 % of the best (7168 x 16384: 100 rows 50 us in 9 parts, 228 in one;
 // 333 rows 106 in 3; 1000 rows 242 in 2, 267 in one).
+//
+// More than 256 tiles past the last full round: 256 of them run whole, one per
+// CU, and the K parts of the others share the CUs with them at first (two per
+// CU for `kb` blocks, then one).  The parts end long before the launch does,
+// but their finish is not hidden (8 us with the disturbance measured).
+// 7168 x 16384 at 1400 rows 381 -> 350 us; q_a | kv_a at 4096 rows (288 tiles)
+// 177 -> 159, finish included; o_proj at 4096 rows 882 -> 838; 24576 x 1536 at 333 rows (288 tiles of 12 blocks) 47 either way,
+// left whole.
 GemmSplit plan_gemm_split(int M, int N, int K, int mode) {
   GemmSplit sp = {};
   const int cols = mode == GEMV_SILU ? 128 : 256;
@@ -690,6 +698,18 @@ GemmSplit plan_gemm_split(int M, int N, int K, int mode) {
     }
   }
   sp.full = best > 1 ? full : tiles;
+  if (rest > 256) {
+    const int whole = sp.m_tiles <= TL_PANEL ? (full + 256) / sp.m_tiles * sp.m_tiles : full + 256;
+    const int over = tiles - whole, s = std::min({256 / std::max(1, over), GEMM_MAX_PARTS, KB});
+    if (s > 1) {
+      const int kb = (KB + s - 1) / s;
+      const double cost = kb * two + (KB - kb) * one + 8.0 + over * s * 0.03 * nj / 4;
+      if (cost < best_cost * 0.97) {
+        best = s;
+        sp.full = whole;
+      }
+    }
+  }
   sp.rest = tiles - sp.full;
   sp.parts = best;
   sp.group = sp.m_tiles <= TL_PANEL && sp.full % sp.m_tiles == 0 ? sp.m_tiles : 1;

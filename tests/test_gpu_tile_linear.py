@@ -71,6 +71,16 @@ def test_many_tiles_end_in_parts():
     _check(ops.fp8_linear(x, w, s), want, bound, True)
 
 
+@pytest.mark.parametrize("m,n,k", [(130, 256 * 130, 2304), (1200, 256 * 27, 2304)])
+def test_one_tile_per_cu_and_parts_beside_it(m, n, k):
+    """A little more than 256 tiles: 256 (or the row tiles of as many whole column tiles) run whole,
+    the rest in K parts beside them."""
+    print(f"[case] tile linear m={m} n={n} k={k}", flush=True)
+    x, w, s, want, bound = _case(m, n, k, "beside")
+    assert lib().amla_fp8_linear_workspace_bytes(m, n, k) > 0
+    _check(ops.fp8_linear(x, w, s), want, bound, True)
+
+
 @pytest.mark.parametrize("m,n,k", [(65, 128, 256), (100, 384, 1152), (129, 256, 128), (333, 640, 768)])
 def test_swiglu_tiles(m, n, k):
     """silu(gate) * up in the tile's epilogue and in the K-part finish, intermediate sizes that are
