@@ -187,6 +187,20 @@ size_t gemm_ws_bytes(int M, int N, int K, int mode = GEMV_PLAIN);
 int launch_gemm(const GemvParams &p, int mode, hipStream_t stream, float *split_ws = nullptr,
                 size_t split_ws_bytes = 0);
 
+// Row passes between the projections of a prefill (q_rows or T may be 0): the
+// q_a norm of every new row; kv_a_layernorm and the rotated rope key of the
+// cached rows [0, T) of one sequence.
+struct PrefillRows {
+  const uint16_t *qa, *gamma_q;
+  uint16_t *qan;
+  const uint16_t *ckv, *kpe, *gamma_kv;  // (T, 512), (T, 64)
+  const float *table;                    // (T, 32, 2)
+  uint16_t *kvn, *kpe_out;
+  int q_rows, q_lora, T;
+  float eps;
+};
+int launch_prefill_rows(PrefillRows p, hipStream_t st);
+
 int launch_rms_norm(const uint16_t *x, int64_t rows, int64_t dim, int64_t ldx, const uint16_t *gamma,
                     float eps, uint16_t *y, int64_t ldy, hipStream_t stream);
 

@@ -528,19 +528,6 @@ static PrefillLayout prefill_layout(const amla_mla_args &a) {
   return L;
 }
 
-// rope of the cached rope-key rows [0, T) of one sequence with table rows [0, T)
-__global__ __launch_bounds__(256) void kpe_rope_kernel(const uint16_t *__restrict__ kpe, const float *__restrict__ tab,
-                                                       int T, uint16_t *__restrict__ out) {
-  const int e = blockIdx.x * 256 + threadIdx.x;  // one pair
-  if (e >= T * (P_ROPE / 2)) return;
-  const int t = e / (P_ROPE / 2), i = e % (P_ROPE / 2);
-  const uint32_t x = reinterpret_cast<const uint32_t *>(kpe)[e];
-  const float a = lo_bf(x), b = hi_bf(x);
-  const float c = tab[((size_t)t * (P_ROPE / 2) + i) * 2], s = tab[((size_t)t * (P_ROPE / 2) + i) * 2 + 1];
-  reinterpret_cast<uint32_t *>(out)[e] =
-      pack_bf16(__fsub_rn(__fmul_rn(a, c), __fmul_rn(b, s)), __fadd_rn(__fmul_rn(a, s), __fmul_rn(b, c)));
-}
-
 int prefill_impl(const amla_mla_args *a, hipStream_t st);
 
 }  // namespace amla
@@ -586,9 +573,17 @@ int prefill_impl(const amla_mla_args *a, hipStream_t st) {
   pa.kv_lora = a->kv_lora; pa.rope = a->qk_rope; pa.pos = a->positions; pa.seq_len = S; pa.max_rows = a->max_seq;
   if ((rc = run_linear(pa, GEMV_QKVA, st, L.lin_bytes))) return rc;
 
-  if ((rc = launch_rms_norm(qa, M, a->q_lora, a->q_lora, reinterpret_cast<const uint16_t *>(a->gamma_q), a->eps,
-                            qan, a->q_lora, st)))
-    return rc;
+  // q_a_layernorm of the new rows; with the first sequence's kv_a_layernorm of
+  // every cached row and its rotated rope keys (inference/ops.py:148-151)
+  const int T = L.Tmax;
+  PrefillRows rows = {};
+  rows.qa = qa; rows.gamma_q = reinterpret_cast<const uint16_t *>(a->gamma_q); rows.qan = qan;
+  rows.ckv = reinterpret_cast<const uint16_t *>(a->ckv_cache); rows.kpe = reinterpret_cast<const uint16_t *>(a->kpe_cache);
+  rows.gamma_kv = reinterpret_cast<const uint16_t *>(a->gamma_kv); rows.table = a->rope_table;
+  rows.kvn = kvn; rows.kpe_out = kpe;
+  rows.q_rows = M; rows.q_lora = a->q_lora; rows.T = L.absorbed ? 0 : T; rows.eps = a->eps;
+  if ((rc = launch_prefill_rows(rows, st))) return rc;
+  rows.q_rows = 0;
 
   GemvParams pb = {};
   pb.part = reinterpret_cast<float *>(ws + L.lin);
@@ -602,19 +597,15 @@ int prefill_impl(const amla_mla_args *a, hipStream_t st) {
   if ((rc = run_linear(pb, GEMV_QROPE, st, L.lin_bytes))) return rc;
 
   if (L.absorbed && (rc = launch_prefill_absorbed(*a, q, attn, ws + L.lat, st))) return rc;
-  const int T = L.Tmax;
   FlashParams fp = {};
   fp.q = q; fp.kvb = kvb; fp.kpe = kpe; fp.out = attn; fp.pos = a->positions; fp.S = S; fp.tmax = T;
   fp.scale_log2 = a->softmax_scale * 1.4426950408889634f;
   for (int b = 0; b < (L.absorbed ? 0 : B); ++b) {
-    const uint16_t *ckv_b = reinterpret_cast<const uint16_t *>(a->ckv_cache) + (size_t)b * a->max_seq * a->kv_lora;
-    const uint16_t *kpe_b = reinterpret_cast<const uint16_t *>(a->kpe_cache) + (size_t)b * a->max_seq * a->qk_rope;
-    // kv_a_layernorm of every cached row, then kv_b (inference/ops.py:148-151)
-    if ((rc = launch_rms_norm(ckv_b, T, a->kv_lora, a->kv_lora, reinterpret_cast<const uint16_t *>(a->gamma_kv),
-                              a->eps, kvn, a->kv_lora, st)))
-      return rc;
-    kpe_rope_kernel<<<dim3((T * (P_ROPE / 2) + 255) / 256), 256, 0, st>>>(kpe_b, a->rope_table, T, kpe);
-    if ((rc = check_launch("kpe rope"))) return rc;
+    if (b) {
+      rows.ckv += (size_t)a->max_seq * a->kv_lora;
+      rows.kpe += (size_t)a->max_seq * a->qk_rope;
+      if ((rc = launch_prefill_rows(rows, st))) return rc;
+    }
     GemvParams pk = {};
     pk.part = reinterpret_cast<float *>(ws + L.lin);
     pk.x = kvn; pk.M = T; pk.ldx = a->kv_lora;

@@ -66,6 +66,33 @@ def test_prompt_and_token_by_token_agree(layer):
     assert_bf16_ulps(ckv, c2, 2, "cache rows")
 
 
+@pytest.mark.parametrize("S,starts", [(5, [700]), (66, [3, 0, 30]), (130, [1])])
+def test_norm_weights_at_any_alignment(layer, S, starts):
+    """The row passes between the projections and the latent merge read the norm weights 16 bytes at
+    a time where these are aligned: weights two bytes off give the same result."""
+    print(f"[case] prefill norm weights S={S} starts={starts}", flush=True)
+    B, rows = len(starts), max(starts) + S + 2
+    aw = _gpu(layer.attn_weights)
+    hidden = synth.make_hidden(CFG, B, S, "lp-gamma").to(DEV)
+    kv = [t.to(DEV) for t in synth.make_kv_cache(CFG, B, rows, starts, "lp-gamma")]
+    tab = R.precompute_rope_freqs(CFG, rows).to(DEV)
+
+    def off(g):
+        buf = torch.empty(g.numel() + 1, dtype=g.dtype, device=DEV)
+        buf[1:] = g
+        return buf[1:]
+
+    c2, c3 = [t.clone() for t in kv], [t.clone() for t in kv]
+    want = ops.mla_attention(hidden, aw, tuple(kv), starts, tab, CFG)
+    got = ops.mla_attention(hidden, dict(aw, kv_a_layernorm=off(aw["kv_a_layernorm"])), tuple(c2), starts, tab, CFG)
+    both = ops.mla_attention(hidden, dict(aw, kv_a_layernorm=off(aw["kv_a_layernorm"]),
+                                          q_a_layernorm=off(aw["q_a_layernorm"])), tuple(c3), starts, tab, CFG)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(kv, c2))
+    # the q_a norm sums an unaligned row in another order
+    assert_parity(both, want, f"both weights off S={S}")
+
+
 def test_scratch_covers_a_smaller_last_chunk():
     """65 tokens run as 33 + 32: the smaller chunk may be cut into more one-tile splits."""
     from amla._lib import MlaArgs
