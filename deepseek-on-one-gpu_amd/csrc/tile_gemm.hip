@@ -1,5 +1,5 @@
 // Block-FP8 GEMM tiles of 256 weight rows x up to 128 activation rows for gfx950:
-// the routed experts' groups of more than 16 rows (amla_moe_experts_dev).
+// the linears above 64 rows and the routed experts' larger groups.
 //
 // y[m, n] = sum_k x[m, k] w[n, k] scale_inv[n/128, k/128], w e4m3fn converted
 // exactly to bf16 in registers, 32x32x16 bf16 MFMAs, fp32 sums.
@@ -29,10 +29,10 @@ namespace amla {
 // 8000 tokens (250 rows) 4.8 + 2.4 ms against 5.6 + 2.9.  Gathering and
 // scattering the rows here saved two more passes (0.14 ms at 2000 tokens).
 //
-// K stages of 64 in LDS: fp8 weight rows (64 B, chunk c of row r at
-// c ^ ((r >> 2) & 3)), bf16 activation rows (128 B, chunk c of row r at
-// c ^ ((r >> 1) & 7)): the 16 lanes of each fragment-read pass hit distinct
-// banks.  Three stages for up to 64 rows, two above (80 KB).
+// Above 64 rows (TileHalves): two K stages of 64 in LDS, fp8 weight rows (64 B,
+// chunk c of row r at c ^ ((r >> 2) & 3)) and bf16 activation rows (128 B,
+// chunk c of row r at c ^ ((r >> 1) & 7)): the 16 lanes of each fragment-read
+// pass hit distinct banks.  Up to 64 rows: TileLines below.
 constexpr int T_BK = 64;
 constexpr int T_WBYTES = 256 * T_BK;             // weight part of a stage
 constexpr int T_XROW = T_BK * 2;                 // activation row of a stage
@@ -41,9 +41,7 @@ constexpr int T_ZERO = T_LDS - 16;               // weight fragments of a block 
 constexpr int T_PITCH_H = 128 * 2 + 16;          // epilogue rows in LDS: 128 or 256 bf16 outputs
 constexpr int T_PITCH_Y = 256 * 2 + 16;
 static_assert(128 * T_PITCH_Y <= T_ZERO, "staged output tile exceeds LDS");
-constexpr int tile_stages(int nj) { return nj <= 2 ? 3 : 2; }
-static_assert(tile_stages(2) * (T_WBYTES + 64 * T_XROW) <= T_ZERO && tile_stages(4) * (T_WBYTES + 128 * T_XROW) <= T_ZERO,
-              "stages exceed LDS");
+static_assert(2 * (T_WBYTES + 128 * T_XROW) <= T_ZERO, "stages exceed LDS");
 
 struct TileArgs {
   const uint8_t *w[2];   // first row of each segment
@@ -67,14 +65,12 @@ struct TileSums {
 };
 
 template <int NJ>
-struct TileMain {
+struct TileHalves {
   static AMLA_DEV void run(const TileArgs &a, TileSums<NJ> &sums) {
   auto &acc = sums.acc;
   auto &s_run = sums.s_run;
   extern __shared__ __align__(16) uint8_t tsm[];
-  constexpr int NST = tile_stages(NJ);
   constexpr int STAGE = T_WBYTES + 32 * NJ * T_XROW;
-  constexpr int COPIES = 4 + NJ;  // per wave and stage
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j32 = lane & 31, hh = lane >> 5;
@@ -159,9 +155,7 @@ struct TileMain {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
   const int it0 = 2 * a.kb0, iters = 2 * a.kb1;
-#pragma unroll
-  for (int i = 0; i < NST - 1; ++i) dma(it0 + i, i);  // a block is 2 >= NST - 1 stages
-  int ring = 0;
+  dma(it0, 0);
   // One stage of 64: four sub-steps of 16 (K 32 pr + 16 hh + 8 s2 .. +7 of each
   // half-wave).  While a sub-step multiplies, the fragments of the next are
   // read and converted between its MFMAs.  The rescaling between two blocks
@@ -170,7 +164,7 @@ struct TileMain {
   // between its first MFMAs.  Scheduling barriers keep the order: left to
   // itself the compiler issues the multiplies and the LDS waits in runs.
   constexpr int NT = 2 * NJ;           // tiles, in the order of their MFMAs
-  constexpr int LATE = NJ >= 3 ? 2 : 0;  // tiles rescaled between the next block's first MFMAs
+  constexpr int LATE = 2;              // tiles rescaled between the next block's first MFMAs
   auto rescale = [&](int half, const float *r) {  // half tiles in MFMA order
     const int g = (half >> 1) / NJ, j = (half >> 1) % NJ;
 #pragma unroll
@@ -178,12 +172,11 @@ struct TileMain {
   };
   auto stage = [&](int it, auto odd_c, const float *r) {
     constexpr bool ODD = decltype(odd_c)::value;
-    const int stg = NST == 2 ? (ODD ? 1 : 0) : ring;  // two stages: even blocks' halves in 0, odd ones in 1
-    if (NST == 3 && it + 1 < iters) wait_vmcnt<COPIES>();
-    else wait_vmcnt<0>();
+    constexpr int stg = ODD ? 1 : 0;
+    wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (it + NST - 1 < iters) dma(it + NST - 1, stg == 0 ? NST - 1 : stg - 1);
+    if (it + 1 < iters) dma(it + 1, 1 - stg);
     const uint8_t *st = tsm + stg * STAGE;
     const uint8_t *sa[2];
 #pragma unroll
@@ -238,7 +231,6 @@ struct TileMain {
           __builtin_amdgcn_sched_barrier(0);
         }
     }
-    if (NST == 3) ring = ring == NST - 1 ? 0 : ring + 1;
   };
   float r[2] = {1.f, 1.f};
   for (int kb = a.kb0; kb < a.kb1; ++kb) {
@@ -260,6 +252,166 @@ struct TileMain {
   // the tiles rescaled after the last block were so by s / s = 1
 }
 };
+
+// Up to 64 rows, where the weight stream is the bound: the stages are whole 128 B
+// lines of the weights, one segment of a K block at a time (16 KB: 128 rows x 128 B,
+// three in the ring, two ahead), the activation rows a K block at a time (two
+// buffers).  With stages of 64 K values of both segments every line was fetched
+// in two halves: LINES_FIG.
+//
+// LDS: weight row 128 B, chunk c of row r at c ^ ((r >> 1) & 7); activation row
+// 256 B, chunk c of row r at c ^ (r & 15): the 16 lanes of a fragment-read pass
+// hit distinct banks.  At 64 rows this is all of the 80 KB: the fragments of a
+// block whose scale is zero are masked in registers.
+constexpr int T_WSEG = 128 * 128;  // one segment of a K block
+constexpr int T_XBLK = 256;        // activation row of a K block
+static_assert(3 * T_WSEG + 2 * 64 * T_XBLK <= T_LDS, "stages exceed LDS");
+
+template <int NJ>
+struct TileLines {
+  static AMLA_DEV void run(const TileArgs &a, TileSums<NJ> &sums) {
+  auto &acc = sums.acc;
+  auto &s_run = sums.s_run;
+  extern __shared__ __align__(16) uint8_t tsm[];
+  constexpr int WC = 4, XC = 2 * NJ;  // copies per wave: a segment, the activation rows of a block
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j32 = lane & 31, hh = lane >> 5;
+
+  // copies: the wave's own 32 weight rows (8 rows of 128 B each) and its quarter
+  // of the activation rows (4 rows of 256 B each), scalar bases plus lane offsets
+  uint32_t woff[2][WC], xoff[XC];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int c = 0; c < WC; ++c)
+      woff[g][c] = (uint32_t)min(32 * wave + 8 * c + (lane >> 3), a.wrows[g] - 1) * a.K +
+                   16 * ((lane & 7) ^ ((4 * c + (lane >> 4)) & 7));
+  auto xchunk = [&](int c) { return 16 * ((lane & 15) ^ ((8 * NJ * wave + 4 * c + (lane >> 4)) & 15)); };
+#pragma unroll
+  for (int c = 0; c < XC; ++c) {
+    const int rc = min(8 * NJ * wave + 4 * c + (lane >> 4), a.rows - 1);  // rows past the tile repeat its last row (not stored)
+    const uint32_t xr = a.xrow ? a.xrow[rc] : rc;
+    // a.wide: x is 4 GB or more, the offset does not fit and is formed per copy
+    xoff[c] = a.wide ? xr : xr * (uint32_t)(a.ldx * 2) + xchunk(c);
+  }
+  typedef const __attribute__((address_space(1))) uint8_t *gptr;
+  auto opaque = [](uint32_t v) {  // (keeps the copies on scalar bases, as above)
+    asm volatile("" : "+v"(v));
+    return v;
+  };
+  auto dma_w = [&](int kb, int g, int slot) {
+    gptr wb = (gptr)(a.w[g] + (size_t)kb * 128);
+    asm volatile("" : "+s"(wb));
+#pragma unroll
+    for (int c = 0; c < WC; ++c)
+      __builtin_amdgcn_global_load_lds(wb + opaque(woff[g][c]), LDS_PTR(tsm + slot * T_WSEG + (32 * wave + 8 * c) * 128), 16, 0, 0);
+  };
+  auto dma_x = [&](int kb, int buf) {
+    gptr xb = (gptr)(reinterpret_cast<const uint8_t *>(a.x) + (size_t)kb * T_XBLK);
+    asm volatile("" : "+s"(xb));
+    uint8_t *dst = tsm + 3 * T_WSEG + (buf * 32 * NJ + 8 * NJ * wave) * T_XBLK;
+    if (!a.wide) {
+#pragma unroll
+      for (int c = 0; c < XC; ++c)
+        __builtin_amdgcn_global_load_lds(xb + opaque(xoff[c]), LDS_PTR(dst + 4 * c * T_XBLK), 16, 0, 0);
+    } else {
+#pragma unroll
+      for (int c = 0; c < XC; ++c)
+        __builtin_amdgcn_global_load_lds(xb + (size_t)xoff[c] * a.ldx * 2 + xchunk(c), LDS_PTR(dst + 4 * c * T_XBLK), 16, 0, 0);
+    }
+  };
+
+  const __attribute__((address_space(4))) float *srow[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) srow[g] = (const __attribute__((address_space(4))) float *)(a.s[g]);
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[g][j][r] = 0.f;
+  // (units of the accumulators: as in TileHalves)
+#pragma unroll
+  for (int g = 0; g < 2; ++g) s_run[g] = srow[g][a.kb0];
+  uint32_t keep[2] = {s_run[0] == 0.f ? 0u : ~0u, s_run[1] == 0.f ? 0u : ~0u};
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+
+  dma_w(a.kb0, 0, 0);
+  dma_x(a.kb0, 0);
+  dma_w(a.kb0, 1, 1);
+  int slot = 0, buf = 0;
+  // One segment of a K block: eight sub-steps of 16 (K 32 pr + 16 hh + 8 s2 ..
+  // +7 of each half-wave).  `other`: the other segment's sums change their units
+  // by r meanwhile (segment 0's to the next block, segment 1's to this one).
+  auto stage = [&](int kb, auto g_c, float r) {
+    constexpr int G = decltype(g_c)::value;
+    const bool more = kb + 1 < a.kb1;
+    // issued after what this stage reads: segment 1 of this block; then, of the
+    // next block, segment 0 and the activation rows
+    if (G == 0) wait_vmcnt<WC>();
+    else if (more) wait_vmcnt<WC + XC>();
+    else wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (more) {
+      dma_w(kb + 1, G, slot == 0 ? 2 : slot - 1);
+      if (G == 0) dma_x(kb + 1, buf ^ 1);
+    }
+    const uint8_t *sw = tsm + slot * T_WSEG + (32 * wave + j32) * 128;
+    const uint8_t *sx = tsm + 3 * T_WSEG + (buf * 32 * NJ + j32) * T_XBLK;
+    u32x4 aw[4], bx[8][NJ];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if ((q & 1) == 0) aw[q >> 1] = *reinterpret_cast<const u32x4 *>(sw + 16 * ((q + hh) ^ ((j32 >> 1) & 7)));
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        bx[q][j] = *reinterpret_cast<const u32x4 *>(sx + j * 32 * T_XBLK + 16 * ((4 * (q >> 1) + 2 * hh + (q & 1)) ^ (j32 & 15)));
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+      const uint32_t w0 = aw[q >> 1][2 * (q & 1)] & keep[G], w1 = aw[q >> 1][2 * (q & 1) + 1] & keep[G];
+      const bf16x2_t c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, false);
+      const bf16x2_t c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.f, true);
+      const bf16x2_t c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, false);
+      const bf16x2_t c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.f, true);
+      const bf16x8 av = bf16x8{c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        acc[G][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, as_bf16x8(bx[q][j]), acc[G][j], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) acc[1 - G][j][2 * q + e] *= r;
+      }
+    }
+    slot = slot == 2 ? 0 : slot + 1;
+  };
+  float r1 = 1.f;
+  for (int kb = a.kb0; kb < a.kb1; ++kb) {
+    float sn[2], r[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) sn[g] = srow[g][min(kb + 1, a.kb1 - 1)];
+    stage(kb, std::integral_constant<int, 0>{}, r1);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) r[g] = s_run[g] == 0.f || sn[g] == 0.f ? 1.f : __fdiv_rn(s_run[g], sn[g]);
+    stage(kb, std::integral_constant<int, 1>{}, r[0]);
+    r1 = r[1];
+    buf ^= 1;
+    if (kb + 1 < a.kb1) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        keep[g] = sn[g] == 0.f ? 0u : ~0u;
+        if (sn[g] != 0.f) s_run[g] = sn[g];
+      }
+    }
+  }
+  // segment 0's sums were rescaled after the last block by s / s = 1
+  asm volatile("" ::: "memory");
+}
+};
+
+template <int NJ>
+using TileMain = std::conditional_t<(NJ <= 2), TileLines<NJ>, TileHalves<NJ>>;
 
 // Stores a tile.  SILU: y = bf16(silu(segment 0)) * segment 1, 128 columns;
 // else y = both segments, 256 columns.
@@ -670,8 +822,8 @@ int launch_tile_grouped(const MoeTileParams &p0, const TileGroups &gr, bool down
 // CU for `kb` blocks, then one).  The parts end long before the launch does,
 // but their finish is not hidden (8 us with the disturbance measured).
 // 7168 x 16384 at 1400 rows 381 -> 350 us; q_a | kv_a at 4096 rows (288 tiles)
-// 177 -> 159, finish included; o_proj at 4096 rows 882 -> 838; 24576 x 1536 at 333 rows (288 tiles of 12 blocks) 47 either way,
-// left whole.
+// 177 -> 159, finish included; o_proj at 4096 rows 882 -> 838; 24576 x 1536 at
+// 333 rows (288 tiles of 12 blocks) 47 either way, left whole.
 GemmSplit plan_gemm_split(int M, int N, int K, int mode) {
   GemmSplit sp = {};
   const int cols = mode == GEMV_SILU ? 128 : 256;
