@@ -18,7 +18,7 @@
 // finish) adds them in part order.  Results are deterministic, and no
 // workgroup waits on another: an in-kernel finish would need device-scope
 // release fences, which write back the per-XCD L2s and cost more than the
-// separate pass.  M > 64 takes the tiled GEMM (gemm_kernel, mla_prefill.hip).
+// separate pass.  M > 64 takes the GEMM tiles (tile_gemm.hip).
 #include <stdarg.h>
 #include <stdio.h>
 
