@@ -25,7 +25,8 @@
 //   absorb     : qt = gamma_kv * W_UK^T q_nope -> qbuf (B, H, 576) with q_pe,
 //                stored in attn_kernel's fragment order; one more workgroup
 //                makes the split plan from the positions
-//   attn       : split over context, fixed-reference softmax, bf16 partial O, (m, l)
+//   attn       : split over context, fixed-reference softmax, partial O (bf16; fp32 in a
+//                latent prefill), (m, l)
 //   combine_uv : merge splits, gamma_kv, W_UV -> (B, H*128) bf16
 //   gemv  PLAIN/RESID : wo (+ residual), then its K-part finish
 #include <limits.h>
@@ -374,7 +375,7 @@ struct AttnParams {
   const int32_t *plan;  // split plan (build_split_plan)
   float scale_log2;  // softmax scale * log2(e)
   float eps;
-  uint16_t *part_o;  // (units + B, H, 512) bf16 by split slot: sum_t p_t r_t c_t, p relative to the split's reference max
+  void *part_o;      // (units + B, H, 512) PartialO elements by split slot: sum_t p_t r_t c_t, p relative to the split's reference max
   float *part_ml;  // (units + B, H, 2) reference max (log2 units) and sum of p; sum < 0 marks a
                    // (split, head) whose scores overflowed the reference (recomputed by the combine)
 };
@@ -1029,11 +1030,22 @@ __global__ __launch_bounds__(256, 1) void attn_kernel(AttnParams p) {
       p.part_ml[row * 2 + 1] = bad ? -1.f : l;
     }
   }
+  wait_vmcnt<0>();
+  if constexpr (!DECODE) {
+    // fp32 partials (PartialO), four columns of a head row per store
+    float *dst = static_cast<float *>(p.part_o) + ((size_t)slot * HEADS + blockIdx.y * HG) * LORA;
+#pragma unroll
+    for (int nt = 0; nt < NH; ++nt)
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+        *reinterpret_cast<f32x4 *>(dst + (size_t)((((NTW * wave + nt) % NH) * 16) + li) * LORA + wave * 128 + mt * 16 +
+                                   4 * lg) = o[mt][nt];
+    return;
+  }
   // O goes out through LDS, over the stages and table blocks: the copies the
   // last iterations issued (into stages nothing reads) must have landed in
   // every wave before any wave writes there; then head rows of 512 bf16, and
   // 1 KB contiguous per wave-wide store
-  wait_vmcnt<0>();
   __syncthreads();
 #pragma unroll
   for (int nt = 0; nt < NH; ++nt)
@@ -1043,7 +1055,7 @@ __global__ __launch_bounds__(256, 1) void attn_kernel(AttnParams p) {
                                  (wave * 128 + mt * 16 + 4 * lg) * 2) =
           u32x2{pack_bf16(o[mt][nt].x, o[mt][nt].y), pack_bf16(o[mt][nt].z, o[mt][nt].w)};
   __syncthreads();
-  uint8_t *const dst = reinterpret_cast<uint8_t *>(p.part_o + ((size_t)slot * HEADS + blockIdx.y * HG) * LORA);
+  uint8_t *const dst = reinterpret_cast<uint8_t *>(static_cast<uint16_t *>(p.part_o) + ((size_t)slot * HEADS + blockIdx.y * HG) * LORA);
 #pragma unroll 8
   for (int i = 0; i < HG * LORA * 2 / (256 * 16); ++i) {
     const int chunk = i * 256 + tid, head = chunk >> 6, c16 = chunk & 63;
@@ -1052,6 +1064,40 @@ __global__ __launch_bounds__(256, 1) void attn_kernel(AttnParams p) {
 }
 
 constexpr size_t ATTN_LDS = ATTN_LDS_BYTES;
+
+// Eight columns of a split's partial O as the combine loads them: bf16 in
+// decode; fp32 in the latent prefill, whose counterpart for longer prompts
+// (flash_kernel) keeps O in fp32 over the whole context.
+template <bool DECODE> struct PartialO;
+template <> struct PartialO<true> {
+  typedef uint16_t elem;
+  u32x4 v;
+  AMLA_DEV void load(const elem *p) { v = ldg16(p); }
+  AMLA_DEV void add(float w, float (&acc)[8]) const {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      acc[2 * e] += w * lo_bf(v[e]);
+      acc[2 * e + 1] += w * hi_bf(v[e]);
+    }
+  }
+  static AMLA_DEV float2 pair(const elem *row, int i) {
+    const uint32_t v = reinterpret_cast<const uint32_t *>(row)[i];
+    return float2{lo_bf(v), hi_bf(v)};
+  }
+};
+template <> struct PartialO<false> {
+  typedef float elem;
+  f32x4 v[2];
+  AMLA_DEV void load(const elem *p) {
+    v[0] = *reinterpret_cast<const f32x4 *>(p);
+    v[1] = *reinterpret_cast<const f32x4 *>(p + 4);
+  }
+  AMLA_DEV void add(float w, float (&acc)[8]) const {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] += w * v[e >> 2][e & 3];
+  }
+  static AMLA_DEV float2 pair(const elem *row, int i) { return reinterpret_cast<const float2 *>(row)[i]; }
+};
 
 // ---------------------------------------------------------------- combine + W_UV
 
@@ -1147,7 +1193,11 @@ AMLA_DEV void recompute_split(const AttnParams &p, int b, int h, const SeqSplits
 //     own with exp2(m_s - M); the parts' sums meet in LDS in part order;
 //   a sequence with a flagged split is merged by the whole workgroup with
 //     exact recomputation of the flagged splits (rare);
-//   lat = O / l times kv_a_layernorm gamma and W_UV's block scale, as bf16;
+//   lat = O / l times kv_a_layernorm gamma and W_UV's block scale, as bf16
+//     (latent prefill: as two, the second what the first rounds off, and two
+//     MFMAs: against 64 bits the heads of 8150 rows are then off by 0.0022 -
+//     0.0028 of their norm, flash_kernel's by 0.0029 - 0.0057, a single bf16
+//     latent and bf16 partial O by 0.0032 - 0.0036);
 //   out[b][v] = W_UV[h][v] . lat[b] by 16x16x32 MFMAs: A = W_UV rows (fp8
 //     converted exactly), B = lat of the SQ sequences (columns past them
 //     zero); wave w produces rows v = 16w .. 16w+15.
@@ -1158,7 +1208,7 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
                                                          uint16_t *__restrict__ attn) {
   ap.map.template fix<DECODE>();
   constexpr int NU = SQ * WPS;    // merge units
-  constexpr int XB = SQ > 4 ? 8 : 20;  // splits in flight per wave (a batch)
+  constexpr int XB = (SQ > 4 ? 8 : 20) / (DECODE ? 1 : 2);  // splits in flight per wave (a batch)
   constexpr int WMAX = 256;       // splits per sequence
   constexpr int MLR = WMAX / 64;  // (m, l) loads per lane
   constexpr int LROW = LORA + 8;  // bf16 per lat row in LDS (16 B pad)
@@ -1172,7 +1222,7 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   __shared__ __align__(16) uint16_t latb[SQ][LROW];
   __shared__ float wsp[8][WMAX + XB];  // weight of split s, zero past the last split
-  __shared__ float xacc[NU][8][64];  // each unit's sums, [column e][lane]
+  __shared__ __align__(16) float xacc[NU][8][64];  // each unit's sums, [column e][lane]
   __shared__ float xl[NU];
   __shared__ float qs[QKD];
   __shared__ float ps[256];
@@ -1200,6 +1250,13 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
     }
   }
 
+  typedef PartialO<DECODE> Part;
+  typedef typename Part::elem part_t;
+  const part_t *const part_o = static_cast<const part_t *>(ap.part_o);
+  // latent prefill: the low half of sequence sq's latent lies over its own sums
+  // (read by the wave that writes it), 16-byte chunk c at c ^ sq
+  auto lat_lo = [&](int sq, int c) { return reinterpret_cast<uint8_t *>(&xacc[sq * WPS][0][0]) + 16 * (c ^ sq); };
+
   // ---- fast merge: unit u = (sequence b0 + u / WPS, part u % WPS).  A
   // unit's first batch of partial rows and every split's (m, l) are loaded
   // together (lane l: splits l, l + 64, ..); the max and the weights are
@@ -1212,14 +1269,14 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
     }
     const SeqSplits sp = seq_splits(ap, b0 + su);
     const size_t base = (size_t)sp.first * HEADS + h;
-    const u32x4 *po = reinterpret_cast<const u32x4 *>(ap.part_o + base * LORA) + lane;
-    const size_t stride = (size_t)HEADS * LORA / 8;
+    const part_t *po = part_o + base * LORA + 8 * lane;
+    const size_t stride = (size_t)HEADS * LORA;
     const int nsp = sp.count;
     const int chunk = (nsp + WPS - 1) / WPS;
     const int s0 = min(pu * chunk, nsp), s1 = min(s0 + chunk, nsp);  // this unit's splits [s0, s1)
-    u32x4 v[XB];
+    Part v[XB];
 #pragma unroll
-    for (int j = 0; j < XB; ++j) v[j] = po[(size_t)min(s0 + j, nsp - 1) * stride];
+    for (int j = 0; j < XB; ++j) v[j].load(po + (size_t)min(s0 + j, nsp - 1) * stride);
     float2 ml[MLR];
 #pragma unroll
     for (int r = 0; r < MLR; ++r) {
@@ -1261,17 +1318,10 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int k = 0; k < s1 - s0; k += XB) {
 #pragma unroll
-      for (int j = 0; j < XB; ++j) {
-        const float w = wsp[wave][s0 + k + j];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          acc[2 * e] += w * lo_bf(v[j][e]);
-          acc[2 * e + 1] += w * hi_bf(v[j][e]);
-        }
-      }
+      for (int j = 0; j < XB; ++j) v[j].add(wsp[wave][s0 + k + j], acc);
       if (k + XB < s1 - s0) {
 #pragma unroll
-        for (int j = 0; j < XB; ++j) v[j] = po[(size_t)min(s0 + k + XB + j, nsp - 1) * stride];
+        for (int j = 0; j < XB; ++j) v[j].load(po + (size_t)min(s0 + k + XB + j, nsp - 1) * stride);
       }
     }
 #pragma unroll
@@ -1294,11 +1344,15 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
     const float inv = 1.f / L;
     const float sc = bsc[(8 * lane) / 128];
     const u32x4 gm = DECODE ? ldg16(gamma + 8 * lane) : ldg8_bf16(gamma, 8 * lane);
-    u32x4 o;
+    u32x4 o, lo;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      o[e] = pack_bf16(acc[2 * e] * inv * lo_bf(gm[e]) * sc, acc[2 * e + 1] * inv * hi_bf(gm[e]) * sc);
+    for (int e = 0; e < 4; ++e) {
+      const float a0 = acc[2 * e] * inv * lo_bf(gm[e]) * sc, a1 = acc[2 * e + 1] * inv * hi_bf(gm[e]) * sc;
+      o[e] = pack_bf16(a0, a1);
+      if constexpr (!DECODE) lo[e] = pack_bf16(a0 - lo_bf(o[e]), a1 - hi_bf(o[e]));
+    }
     *reinterpret_cast<u32x4 *>(&latb[sq][8 * lane]) = o;
+    if constexpr (!DECODE) *reinterpret_cast<u32x4 *>(lat_lo(sq, lane)) = lo;
   }
   __syncthreads();
 
@@ -1316,9 +1370,9 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
       if (l1 < 0.f) {
         recompute_split(ap, b, h, sp, s, qs, ps, red, m1, l1, o0, o1);
       } else if (tid < 256) {
-        const uint32_t v = reinterpret_cast<const uint32_t *>(ap.part_o + row * LORA)[tid];
-        o0 = lo_bf(v);
-        o1 = hi_bf(v);
+        const float2 v = Part::pair(part_o + row * LORA, tid);
+        o0 = v.x;
+        o1 = v.y;
       }
       if (m1 == -INFINITY) continue;  // split past this sequence's context
       const float Mn = fmaxf(M, m1);
@@ -1333,7 +1387,11 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
       const float inv = 1.f / Ls;
       const float sc = bsc[(2 * tid) / 128];
       const uint32_t gm = reinterpret_cast<const uint32_t *>(gamma)[tid];
-      reinterpret_cast<uint32_t *>(&latb[bb][0])[tid] = pack_bf16(a0 * inv * lo_bf(gm) * sc, a1 * inv * hi_bf(gm) * sc);
+      const float l0 = a0 * inv * lo_bf(gm) * sc, l1 = a1 * inv * hi_bf(gm) * sc;
+      const uint32_t o = pack_bf16(l0, l1);
+      reinterpret_cast<uint32_t *>(&latb[bb][0])[tid] = o;
+      if constexpr (!DECODE)
+        reinterpret_cast<uint32_t *>(lat_lo(bb, tid >> 2))[tid & 3] = pack_bf16(l0 - lo_bf(o), l1 - hi_bf(o));
     }
     __syncthreads();
   }
@@ -1353,6 +1411,10 @@ __global__ __launch_bounds__(512) void combine_uv_kernel(AttnParams ap, const ui
     const bf16x2_t c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(wa[ks].y, 1.f, true);
     const bf16x8 a = {c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
     c = mfma16(a, as_bf16x8(bl), c);
+    if constexpr (!DECODE) {
+      const u32x4 bo = bvalid ? *reinterpret_cast<const u32x4 *>(lat_lo(li, lg + 4 * ks)) : u32x4{0, 0, 0, 0};
+      c = mfma16(a, as_bf16x8(bo), c);
+    }
   }
   // C: lane holds sequence b0 + li, rows v = 16w + 4 lg .. +3
   if (bvalid) {
@@ -1454,7 +1516,7 @@ struct AbsorbedScratch {
   int32_t *plan;      // plan_ints(tokens, slots)
   uint16_t *qbuf;     // (tokens, H, 576)
   float *part_ml;     // (slots, H, 2)
-  uint16_t *part_o;   // (slots, H, 512)
+  void *part_o;       // (slots, H, 512) PartialO elements
 };
 
 static void set_attn_attr();
@@ -1528,8 +1590,12 @@ static int absorbed_chunk(int64_t tokens) {
 // flash over 256-query blocks: in proportion to the rows alone while the
 // queries fit a block).  Times in us measured on MI355X: kv_b 0.041 per row,
 // flash 1.92 per 64-key tile and round of 256 workgroups, attn_kernel 2.25 per
-// 32-row tile of the longest split.  One sequence over 8192 rows: 50 new
-// tokens 170 against 620, about equal at 200; at 512 rows 8 new tokens.
+// 32-row tile of the longest split, the fp32 partials 0.07 per split to store
+// and merge (followup of 50 tokens over 8150 rows, whole layer: 231 with bf16
+// partials, 241 with fp32).  Whole call, decompressed against latent: 2 new
+// tokens over none 62 / 71, over 200 rows 87 / 74; 32 over 200 89 / 101, over
+// 900 146 / 118; 64 over 900 165 / 155; 50 over 8192 680 / 240, about equal
+// at 200.
 bool prefill_absorbed(int batch, int seq_len, int context) {
   const double blocks = (seq_len + 255) / 256;
   const double tiles = (context + 63) / 64, causal = 1.0 - 0.5 * seq_len / std::max(context, seq_len);
@@ -1541,8 +1607,8 @@ bool prefill_absorbed(int batch, int seq_len, int context) {
   int units, slots;
   attn_units(n, context, units, slots);
   const double split = std::ceil((double)n * ((context + TT - 1) / TT) / units);
-  const double chunk = (4.0 + 0.16 * n) + (10.0 + 2.25 * split) + (6.0 + units / 32.0 + 0.15 * n);
-  return (double)((tokens + n - 1) / n) * chunk < 0.9 * direct;
+  const double chunk = (4.0 + 0.16 * n) + (15.0 + 2.25 * split) + (6.0 + units / 14.0 + 0.15 * n);
+  return (double)((tokens + n - 1) / n) * chunk < 0.95 * direct;
 }
 
 static size_t absorbed_scratch(int64_t tokens, int context, char *base, AbsorbedScratch *sc) {
@@ -1554,10 +1620,10 @@ static size_t absorbed_scratch(int64_t tokens, int context, char *base, Absorbed
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
   const size_t plan = take(plan_ints(chunk, slots) * 4), qbuf = take((size_t)chunk * HEADS * QKD * 2),
-               ml = take((size_t)slots * HEADS * 2 * 4), po = take((size_t)slots * HEADS * LORA * 2);
+               ml = take((size_t)slots * HEADS * 2 * 4), po = take((size_t)slots * HEADS * LORA * sizeof(PartialO<false>::elem));
   if (sc)
     *sc = AbsorbedScratch{reinterpret_cast<int32_t *>(base + plan), reinterpret_cast<uint16_t *>(base + qbuf),
-                          reinterpret_cast<float *>(base + ml), reinterpret_cast<uint16_t *>(base + po)};
+                          reinterpret_cast<float *>(base + ml), base + po};
   return off;
 }
 

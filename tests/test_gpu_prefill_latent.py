@@ -9,7 +9,7 @@ import torch
 
 from oracle import ref_ops as R
 from amla import ops, synth
-from amla._lib import lib
+from amla._lib import MlaArgs, lib
 from amla.config import DeepSeekConfig
 from _tol import assert_bf16_ulps, assert_heads_parity, assert_parity
 
@@ -91,6 +91,44 @@ def test_norm_weights_at_any_alignment(layer, S, starts):
     assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(kv, c2))
     # the q_a norm sums an unaligned row in another order
     assert_parity(both, want, f"both weights off S={S}")
+
+
+def _sizes(B, S, context):
+    a = MlaArgs()
+    a.batch, a.seq_len, a.hidden, a.heads, a.q_lora, a.kv_lora = B, S, 7168, 128, 1536, 512
+    a.qk_nope, a.qk_rope, a.v_dim, a.max_seq, a.rope_rows, a.max_context = 128, 64, 128, context, context, context
+    return lib().amla_mla_prefill_workspace_bytes(ctypes.byref(a))
+
+
+@pytest.mark.parametrize("S,p", [(12, 1500), (70, 4000)])
+def test_heads_lose_nothing_to_16_bit_sums(layer, S, p):
+    """Rows about one latent vector under equal scores, where the roundings of a split's sums and of
+    the merged latent do not average out: the heads against 64 bits.  Left are their own rounding to
+    bf16 (taken from the 64-bit values) and the one of p r_t, 2^-9 at most on each weight and, the
+    row norms spread over several bf16 steps, under 2^-11 on a sum of them."""
+    T = p + S
+    assert _sizes(1, S, T) < T * 128 * 256 * 2, "the decompressed form was chosen"
+    print(f"[case] latent prefill precision S={S} T={T}", flush=True)
+    aw = _gpu(layer.attn_weights)
+    aw["q_b_proj"] = (aw["q_b_proj"][0], aw["q_b_proj"][1] * 1e-12)
+    hidden = synth.make_hidden(CFG, 1, S, "lp-flat").to(DEV)
+    g = torch.Generator().manual_seed(S)
+    ckv = (torch.randn(1, 1, 512, generator=g) + 0.5 * torch.randn(1, T, 512, generator=g)).to(torch.bfloat16).to(DEV)
+    kpe = torch.randn(1, T, 64, generator=g).to(torch.bfloat16).to(DEV)
+    tab = R.precompute_rope_freqs(CFG, T).to(DEV)
+    heads = torch.empty(1, S, 128 * 128, dtype=torch.bfloat16, device=DEV)
+    ops.mla_attention(hidden, aw, (ckv, kpe), p, tab, CFG, attn_out=heads)
+    torch.cuda.synchronize()
+    c = ckv[0].double().cpu()
+    c = c * torch.rsqrt(c.pow(2).mean(1, keepdim=True) + CFG.rms_norm_eps) * layer.attn_weights["kv_a_layernorm"].double()
+    lat = (c.cumsum(0) / torch.arange(1, T + 1, dtype=torch.float64)[:, None])[p:]
+    w, s = layer.attn_weights["kv_b_proj"]
+    w = (w.double() * s.double().repeat_interleave(128, 0).repeat_interleave(128, 1)).view(128, 256, 512)[:, 128:]
+    want = torch.einsum("sl,hvl->shv", lat, w).reshape(S, 128 * 128)
+    n = want.norm()
+    err, own = (heads[0].double().cpu() - want).norm() / n, (want.to(torch.bfloat16).double() - want).norm() / n
+    print(f"    error {err:.6f}, rounding of the result {own:.6f}", flush=True)
+    assert err ** 2 <= own ** 2 + 2.0 ** -22
 
 
 def test_scratch_covers_a_smaller_last_chunk():
