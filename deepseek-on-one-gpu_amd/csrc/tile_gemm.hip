@@ -43,6 +43,10 @@ constexpr int T_PITCH_Y = 256 * 2 + 16;
 static_assert(128 * T_PITCH_Y <= T_ZERO, "staged output tile exceeds LDS");
 static_assert(2 * (T_WBYTES + 128 * T_XROW) <= T_ZERO, "stages exceed LDS");
 
+// x row strides (bf16) up to which the byte offsets of 128 rows fit 32 bits;
+// weight rows are half as far apart
+constexpr int T_MAX_LD = (int)((UINT32_MAX - T_XROW) / (2 * 127));
+
 struct TileArgs {
   const uint8_t *w[2];   // first row of each segment
   const float *s[2];     // scale row (K / 128) of each segment
@@ -54,7 +58,7 @@ struct TileArgs {
   int ldx, ldy, K, rows;
   int kb0, kb1;          // 128-wide K blocks
   bool two;              // segment 1 is stored (always multiplied)
-  bool wide;             // byte offsets of x rows may not fit 32 bits
+  bool wide, wwide;      // byte offsets of the tile's x / weight rows may not fit 32 bits
 };
 
 // A tile's sums: acc[segment][row group of 32], in units of s_run[segment].
@@ -83,15 +87,17 @@ struct TileHalves {
   for (int g = 0; g < 2; ++g)
 #pragma unroll
     for (int c = 0; c < 2; ++c)
-      woff[g][c] = (uint32_t)min(32 * wave + 16 * c + (lane >> 2), a.wrows[g] - 1) * a.K +
-                   16 * ((lane & 3) ^ ((lane >> 4) & 3));
+    {
+      const uint32_t wr = min(32 * wave + 16 * c + (lane >> 2), a.wrows[g] - 1);
+      // a.wide, a.wwide: the row index only, the offset is formed per copy
+      woff[g][c] = a.wwide ? wr : wr * (uint32_t)a.K + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
+    }
 #pragma unroll
   for (int c = 0; c < NJ; ++c) {
     const int r = 8 * (NJ * wave + c) + (lane >> 3);
     const int rc = min(r, a.rows - 1);  // rows past the tile repeat its last row (not stored)
     const uint32_t xr = a.xrow ? a.xrow[rc] : rc;
-    // a.wide: x is 4 GB or more, the offset does not fit and is formed per copy
-    xoff[c] = a.wide ? xr : xr * (uint32_t)(a.ldx * 2) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+    xoff[c] = a.wide ? xr : xr * ((uint32_t)a.ldx * 2) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
   }
   auto dma = [&](int it, int stg) {
     uint8_t *st = tsm + stg * STAGE;
@@ -111,7 +117,9 @@ struct TileHalves {
     for (int g = 0; g < 2; ++g)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        __builtin_amdgcn_global_load_lds(wb[g] + opaque(woff[g][c]), LDS_PTR(st + (128 * g + 32 * wave + 16 * c) * T_BK), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(
+            wb[g] + (a.wwide ? (size_t)woff[g][c] * a.K + 16 * ((lane & 3) ^ ((lane >> 4) & 3)) : opaque(woff[g][c])),
+            LDS_PTR(st + (128 * g + 32 * wave + 16 * c) * T_BK), 16, 0, 0);
     if (!a.wide) {
 #pragma unroll
       for (int c = 0; c < NJ; ++c)
@@ -281,19 +289,22 @@ struct TileLines {
   // copies: the wave's own 32 weight rows (8 rows of 128 B each) and its quarter
   // of the activation rows (4 rows of 256 B each), scalar bases plus lane offsets
   uint32_t woff[2][WC], xoff[XC];
+  auto wchunk = [&](int c) { return 16 * ((lane & 7) ^ ((4 * c + (lane >> 4)) & 7)); };
 #pragma unroll
   for (int g = 0; g < 2; ++g)
 #pragma unroll
     for (int c = 0; c < WC; ++c)
-      woff[g][c] = (uint32_t)min(32 * wave + 8 * c + (lane >> 3), a.wrows[g] - 1) * a.K +
-                   16 * ((lane & 7) ^ ((4 * c + (lane >> 4)) & 7));
+    {
+      const uint32_t wr = min(32 * wave + 8 * c + (lane >> 3), a.wrows[g] - 1);
+      // a.wide, a.wwide: the row index only, the offset is formed per copy
+      woff[g][c] = a.wwide ? wr : wr * (uint32_t)a.K + wchunk(c);
+    }
   auto xchunk = [&](int c) { return 16 * ((lane & 15) ^ ((8 * NJ * wave + 4 * c + (lane >> 4)) & 15)); };
 #pragma unroll
   for (int c = 0; c < XC; ++c) {
     const int rc = min(8 * NJ * wave + 4 * c + (lane >> 4), a.rows - 1);  // rows past the tile repeat its last row (not stored)
     const uint32_t xr = a.xrow ? a.xrow[rc] : rc;
-    // a.wide: x is 4 GB or more, the offset does not fit and is formed per copy
-    xoff[c] = a.wide ? xr : xr * (uint32_t)(a.ldx * 2) + xchunk(c);
+    xoff[c] = a.wide ? xr : xr * ((uint32_t)a.ldx * 2) + xchunk(c);
   }
   typedef const __attribute__((address_space(1))) uint8_t *gptr;
   auto opaque = [](uint32_t v) {  // (keeps the copies on scalar bases, as above)
@@ -305,7 +316,8 @@ struct TileLines {
     asm volatile("" : "+s"(wb));
 #pragma unroll
     for (int c = 0; c < WC; ++c)
-      __builtin_amdgcn_global_load_lds(wb + opaque(woff[g][c]), LDS_PTR(tsm + slot * T_WSEG + (32 * wave + 8 * c) * 128), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(wb + (a.wwide ? (size_t)woff[g][c] * a.K + wchunk(c) : opaque(woff[g][c])),
+                                       LDS_PTR(tsm + slot * T_WSEG + (32 * wave + 8 * c) * 128), 16, 0, 0);
   };
   auto dma_x = [&](int kb, int buf) {
     gptr xb = (gptr)(reinterpret_cast<const uint8_t *>(a.x) + (size_t)kb * T_XBLK);
@@ -562,7 +574,10 @@ AMLA_DEV void tile_linear_body(const GemvParams &p, const TileArgs &a, int n0, i
 }
 
 // Workgroups [0, full): whole tiles; then K part (i - full) % parts of tile full + (i - full) / parts.
-template <int MODE>
+// WIDE: x or weight rows whose byte offsets from the tile's first row do not
+// fit 32 bits, each formed in 64 per copy (a kernel of its own: with the choice
+// made inside, 4096 x 7168 x 18432 took 4 % longer).
+template <int MODE, bool WIDE>
 __global__ __launch_bounds__(256, 2) void tile_linear_kernel(GemvParams p, bool staged, GemmSplit sp) {
   const int KB = p.K >> 7;
   int t, kb0 = 0, kb1 = KB;
@@ -593,7 +608,7 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(GemvParams p, bool 
   a.kb1 = kb1;
   a.x = p.x + (size_t)m0 * p.ldx;
   a.xrow = nullptr;
-  a.wide = false;  // 128 rows from its base
+  a.wide = a.wwide = WIDE;
   // segment = a run of up to 128 rows of one weight: the first weight's
   // segments come before the second's (n_split % 128 == 0)
   int n0[2];
@@ -719,6 +734,7 @@ AMLA_DEV void moe_tile(const MoeTileParams &p, const TileGroup &g, int nt, const
   const int KB = p.K >> 7;
   a.x = xrow ? p.x : p.x + (size_t)g.first * p.ldx;
   a.wide = xrow && p.wide;
+  a.wwide = false;
   a.xrow = xrow;
   a.y = (yrow ? p.y : p.y + (size_t)g.first * p.ldy) + nt * (GATEUP ? 128 : 256);
   a.yrow = yrow;
@@ -770,8 +786,10 @@ __global__ __launch_bounds__(256, 2) void tile_grouped_kernel(MoeTileParams p, T
 }
 
 static int check_tiles(const MoeTileParams &p) {
-  if (p.K % 128 || p.N % 128 || p.ldx % 8 || p.ldy % 8 || !aligned16(p.x) || !aligned16(p.y))
-    return fail(AMLA_EUNSUPPORTED, "expert fp8 tiles need K %% 128 == 0, N %% 128 == 0 and 16-byte aligned rows");
+  if (p.K % 128 || p.N % 128 || p.ldx % 8 || p.ldy % 8 || !aligned16(p.x) || !aligned16(p.y) || p.K > T_MAX_LD ||
+      p.ldx > T_MAX_LD)
+    return fail(AMLA_EUNSUPPORTED,
+                "expert fp8 tiles need K %% 128 == 0, N %% 128 == 0, 16-byte aligned rows and K, ldx <= %d", T_MAX_LD);
   return AMLA_OK;
 }
 
@@ -874,10 +892,15 @@ size_t gemm_ws_bytes(int M, int N, int K, int mode) { return plan_gemm_split(M, 
 
 template <int MODE>
 static int launch_tile_linear(const GemvParams &p, bool staged, const GemmSplit &sp, hipStream_t st) {
-  int rc = tile_lds((const void *)tile_linear_kernel<MODE>);
+  // the epilogue modes' rows are packed: only x of the plain ones has a stride of its own
+  constexpr bool STRIDED = MODE == GEMV_PLAIN || MODE == GEMV_F32;
+  const bool wide = p.ldx > T_MAX_LD || p.K > T_MAX_LD;
+  if (wide && !STRIDED) return fail(AMLA_EUNSUPPORTED, "fp8 GEMM: rows of %d elements in epilogue mode %d", p.ldx, MODE);
+  const auto kernel = wide ? tile_linear_kernel<MODE, STRIDED> : tile_linear_kernel<MODE, false>;
+  int rc = tile_lds((const void *)kernel);
   if (rc) return rc;
   const unsigned blocks = (unsigned)(sp.full_blocks + (sp.rest * sp.parts + 7) / 8 * 8);
-  tile_linear_kernel<MODE><<<dim3(blocks), 256, T_LDS, st>>>(p, staged, sp);
+  kernel<<<dim3(blocks), 256, T_LDS, st>>>(p, staged, sp);
   if ((rc = check_launch("fp8 GEMM")) || !sp.rest) return rc;
   tile_finish_kernel<MODE><<<dim3((unsigned)sp.rest * (MODE == GEMV_SILU ? 4 : 8)), 256, 0, st>>>(p, sp);
   return check_launch("fp8 GEMM K-part finish");

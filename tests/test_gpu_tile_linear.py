@@ -101,3 +101,20 @@ def test_swiglu_tiles(m, n, k):
     # an fp32 sum next to a rounding boundary may move g or u by one bf16 ulp: h then differs by 2^-7 in few entries
     # (one K block of zero scales in either weight makes the whole output zero at k = 128: it must be so)
     assert (got - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("m,stride", [(130, 4096 * 7168), (192, 36000000)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_rows_four_gb_apart(m, stride, f32):
+    """x rows so far apart that a row's byte offset in its tile does not fit 32 bits (130 rows: the
+    last positions of sequences of 4096 tokens; 192: in the tile of 64 rows too): the same bits as
+    packed rows."""
+    k, n = 640, 272
+    print(f"[case] tile linear m={m} row stride {stride}", flush=True)
+    x, w, s, want, bound = _case(m, n, k, "far")
+    far = torch.empty(m, stride, dtype=torch.bfloat16, device=DEV)[:, :k]
+    far.copy_(x)
+    out = torch.float32 if f32 else torch.bfloat16
+    got = ops.fp8_linear(far, w, s, out)
+    assert torch.equal(got, ops.fp8_linear(x, w, s, out))
+    _check(got, want, bound, not f32)
