@@ -58,7 +58,7 @@ struct TileArgs {
   int ldx, ldy, K, rows;
   int kb0, kb1;          // 128-wide K blocks
   bool two;              // segment 1 is stored (always multiplied)
-  bool wide, wwide;      // byte offsets of the tile's x / weight rows may not fit 32 bits
+  bool wide;             // byte offsets of the tile's x rows may not fit 32 bits
 };
 
 // A tile's sums: acc[segment][row group of 32], in units of s_run[segment].
@@ -68,7 +68,8 @@ struct TileSums {
   float s_run[2];
 };
 
-template <int NJ>
+// WIDE: nor do those of its weight rows
+template <int NJ, bool WIDE>
 struct TileHalves {
   static AMLA_DEV void run(const TileArgs &a, TileSums<NJ> &sums) {
   auto &acc = sums.acc;
@@ -89,8 +90,8 @@ struct TileHalves {
     for (int c = 0; c < 2; ++c)
     {
       const uint32_t wr = min(32 * wave + 16 * c + (lane >> 2), a.wrows[g] - 1);
-      // a.wide, a.wwide: the row index only, the offset is formed per copy
-      woff[g][c] = a.wwide ? wr : wr * (uint32_t)a.K + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
+      // a.wide, WIDE: the row index only, the offset is formed per copy
+      woff[g][c] = WIDE ? wr : wr * (uint32_t)a.K + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
     }
 #pragma unroll
   for (int c = 0; c < NJ; ++c) {
@@ -113,13 +114,20 @@ struct TileHalves {
     asm volatile("" : "+s"(wb[0]));
     asm volatile("" : "+s"(wb[1]));
     asm volatile("" : "+s"(xb));
+    if constexpr (!WIDE) {
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
+      for (int g = 0; g < 2; ++g)
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
-        __builtin_amdgcn_global_load_lds(
-            wb[g] + (a.wwide ? (size_t)woff[g][c] * a.K + 16 * ((lane & 3) ^ ((lane >> 4) & 3)) : opaque(woff[g][c])),
-            LDS_PTR(st + (128 * g + 32 * wave + 16 * c) * T_BK), 16, 0, 0);
+        for (int c = 0; c < 2; ++c)
+          __builtin_amdgcn_global_load_lds(wb[g] + opaque(woff[g][c]), LDS_PTR(st + (128 * g + 32 * wave + 16 * c) * T_BK), 16, 0, 0);
+    } else {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          __builtin_amdgcn_global_load_lds(wb[g] + (size_t)woff[g][c] * a.K + 16 * ((lane & 3) ^ ((lane >> 4) & 3)),
+                                           LDS_PTR(st + (128 * g + 32 * wave + 16 * c) * T_BK), 16, 0, 0);
+    }
     if (!a.wide) {
 #pragma unroll
       for (int c = 0; c < NJ; ++c)
@@ -275,7 +283,7 @@ constexpr int T_WSEG = 128 * 128;  // one segment of a K block
 constexpr int T_XBLK = 256;        // activation row of a K block
 static_assert(3 * T_WSEG + 2 * 64 * T_XBLK <= T_LDS, "stages exceed LDS");
 
-template <int NJ>
+template <int NJ, bool WIDE>
 struct TileLines {
   static AMLA_DEV void run(const TileArgs &a, TileSums<NJ> &sums) {
   auto &acc = sums.acc;
@@ -296,8 +304,8 @@ struct TileLines {
     for (int c = 0; c < WC; ++c)
     {
       const uint32_t wr = min(32 * wave + 8 * c + (lane >> 3), a.wrows[g] - 1);
-      // a.wide, a.wwide: the row index only, the offset is formed per copy
-      woff[g][c] = a.wwide ? wr : wr * (uint32_t)a.K + wchunk(c);
+      // a.wide, WIDE: the row index only, the offset is formed per copy
+      woff[g][c] = WIDE ? wr : wr * (uint32_t)a.K + wchunk(c);
     }
   auto xchunk = [&](int c) { return 16 * ((lane & 15) ^ ((8 * NJ * wave + 4 * c + (lane >> 4)) & 15)); };
 #pragma unroll
@@ -314,10 +322,16 @@ struct TileLines {
   auto dma_w = [&](int kb, int g, int slot) {
     gptr wb = (gptr)(a.w[g] + (size_t)kb * 128);
     asm volatile("" : "+s"(wb));
+    if constexpr (!WIDE) {
 #pragma unroll
-    for (int c = 0; c < WC; ++c)
-      __builtin_amdgcn_global_load_lds(wb + (a.wwide ? (size_t)woff[g][c] * a.K + wchunk(c) : opaque(woff[g][c])),
-                                       LDS_PTR(tsm + slot * T_WSEG + (32 * wave + 8 * c) * 128), 16, 0, 0);
+      for (int c = 0; c < WC; ++c)
+        __builtin_amdgcn_global_load_lds(wb + opaque(woff[g][c]), LDS_PTR(tsm + slot * T_WSEG + (32 * wave + 8 * c) * 128), 16, 0, 0);
+    } else {
+#pragma unroll
+      for (int c = 0; c < WC; ++c)
+        __builtin_amdgcn_global_load_lds(wb + (size_t)woff[g][c] * a.K + wchunk(c),
+                                         LDS_PTR(tsm + slot * T_WSEG + (32 * wave + 8 * c) * 128), 16, 0, 0);
+    }
   };
   auto dma_x = [&](int kb, int buf) {
     gptr xb = (gptr)(reinterpret_cast<const uint8_t *>(a.x) + (size_t)kb * T_XBLK);
@@ -422,8 +436,8 @@ struct TileLines {
 }
 };
 
-template <int NJ>
-using TileMain = std::conditional_t<(NJ <= 2), TileLines<NJ>, TileHalves<NJ>>;
+template <int NJ, bool WIDE>
+using TileMain = std::conditional_t<(NJ <= 2), TileLines<NJ, WIDE>, TileHalves<NJ, WIDE>>;
 
 // Stores a tile.  SILU: y = bf16(silu(segment 0)) * segment 1, 128 columns;
 // else y = both segments, 256 columns.
@@ -505,7 +519,7 @@ AMLA_DEV int xcd_run(int i, int n) {
   return (i >> 3) < run && l < n ? l : -1;
 }
 
-template <int MODE, int NJ>
+template <int MODE, int NJ, bool WIDE>
 AMLA_DEV void tile_linear_body(const GemvParams &p, const TileArgs &a, int n0, int n1, int m0, bool staged,
                                float *partial) {
   extern __shared__ __align__(16) uint8_t tsm[];
@@ -513,7 +527,7 @@ AMLA_DEV void tile_linear_body(const GemvParams &p, const TileArgs &a, int n0, i
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j32 = lane & 31, hh = lane >> 5;
   TileSums<NJ> ts;
-  TileMain<NJ>::run(a, ts);
+  TileMain<NJ, WIDE>::run(a, ts);
   auto &acc = ts.acc;
   auto &s_run = ts.s_run;
   auto sums = [&](int g, int j, int q) {
@@ -608,7 +622,7 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(GemvParams p, bool 
   a.kb1 = kb1;
   a.x = p.x + (size_t)m0 * p.ldx;
   a.xrow = nullptr;
-  a.wide = a.wwide = WIDE;
+  a.wide = WIDE;
   // segment = a run of up to 128 rows of one weight: the first weight's
   // segments come before the second's (n_split % 128 == 0)
   int n0[2];
@@ -640,10 +654,10 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(GemvParams p, bool 
     a.wrows[g] = min(128, (p.w1 && !second ? p.n_split : p.N) - n);
   }
   switch ((a.rows + 31) >> 5) {
-    case 1: tile_linear_body<MODE, 1>(p, a, n0[0], n0[1], m0, staged, partial); break;
-    case 2: tile_linear_body<MODE, 2>(p, a, n0[0], n0[1], m0, staged, partial); break;
-    case 3: tile_linear_body<MODE, 3>(p, a, n0[0], n0[1], m0, staged, partial); break;
-    default: tile_linear_body<MODE, 4>(p, a, n0[0], n0[1], m0, staged, partial); break;
+    case 1: tile_linear_body<MODE, 1, WIDE>(p, a, n0[0], n0[1], m0, staged, partial); break;
+    case 2: tile_linear_body<MODE, 2, WIDE>(p, a, n0[0], n0[1], m0, staged, partial); break;
+    case 3: tile_linear_body<MODE, 3, WIDE>(p, a, n0[0], n0[1], m0, staged, partial); break;
+    default: tile_linear_body<MODE, 4, WIDE>(p, a, n0[0], n0[1], m0, staged, partial); break;
   }
 }
 
@@ -706,7 +720,7 @@ __global__ __launch_bounds__(256) void tile_finish_kernel(GemvParams p, GemmSpli
 template <int NJ, bool SILU>
 AMLA_DEV void tile_body(const TileArgs &a) {
   TileSums<NJ> ts;
-  TileMain<NJ>::run(a, ts);
+  TileMain<NJ, false>::run(a, ts);
   tile_store<NJ, SILU>(a, ts);
 }
 
@@ -734,7 +748,6 @@ AMLA_DEV void moe_tile(const MoeTileParams &p, const TileGroup &g, int nt, const
   const int KB = p.K >> 7;
   a.x = xrow ? p.x : p.x + (size_t)g.first * p.ldx;
   a.wide = xrow && p.wide;
-  a.wwide = false;
   a.xrow = xrow;
   a.y = (yrow ? p.y : p.y + (size_t)g.first * p.ldy) + nt * (GATEUP ? 128 : 256);
   a.yrow = yrow;
