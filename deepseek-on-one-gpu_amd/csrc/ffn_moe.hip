@@ -127,9 +127,11 @@ static int fp8_linear_into(const uint16_t *x, int m, int k, const uint8_t *w, co
 
 struct SwigluLayout {
   size_t gu, h, part, part_bytes, total;
+  size_t need;  // without the K-part sums of the large-M GEMM: less than this is refused
 };
 
 // [gate | up] rows (m, 2n) (skinny path), then h (m, n), then the K-part sums
+// (above 64 rows the GEMM runs without them, on whole tiles)
 static SwigluLayout swiglu_layout(int64_t m, int64_t k, int64_t n) {
   SwigluLayout L;
   size_t off = 0;
@@ -145,6 +147,7 @@ static SwigluLayout swiglu_layout(int64_t m, int64_t k, int64_t n) {
   L.part = off;
   off = align_up(off + L.part_bytes, 256);
   L.total = off;
+  L.need = m <= 64 ? L.total : L.part;
   return L;
 }
 
@@ -164,7 +167,12 @@ int amla_silu_mul(const void *gate, const void *up, int64_t numel, void *out, vo
 
 size_t amla_swiglu_workspace_bytes(int64_t m, int64_t k, int64_t n) {
   if (m <= 0 || k <= 0 || n <= 0 || m > INT32_MAX || k > INT32_MAX || n > INT32_MAX) return 0;
-  return swiglu_layout(m, k, n).total;
+  // one buffer serves every smaller m too: the K-part counts of the skinny path
+  // change at 16 and 32 rows, those of the GEMM are not needed
+  size_t total = swiglu_layout(m, k, n).total;
+  for (int64_t t : {8, 16, 32, 64})
+    if (t < m) total = std::max(total, swiglu_layout(t, k, n).total);
+  return total;
 }
 
 int amla_swiglu(const void *x, int64_t m, int64_t k, const void *gate_w, const float *gate_s, const void *up_w,
@@ -183,9 +191,10 @@ int amla_swiglu(const void *x, int64_t m, int64_t k, const void *gate_w, const f
                 (long long)k, (long long)n);
   if (m > INT32_MAX || k > INT32_MAX || n > INT32_MAX) return fail(AMLA_EUNSUPPORTED, "swiglu: sizes above 2^31");
   const SwigluLayout L = swiglu_layout(m, k, n);
-  if (!workspace || workspace_bytes < L.total || !aligned16(workspace))
-    return fail(AMLA_EWORKSPACE, "swiglu: needs %zu bytes of 16-byte aligned workspace (got %zu)", L.total,
+  if (!workspace || workspace_bytes < L.need || !aligned16(workspace))
+    return fail(AMLA_EWORKSPACE, "swiglu: needs %zu bytes of 16-byte aligned workspace (got %zu)", L.need,
                 workspace ? workspace_bytes : (size_t)0);
+  const size_t part_bytes = std::min(L.part_bytes, workspace_bytes - L.part);
   uint8_t *ws = static_cast<uint8_t *>(workspace);
   uint16_t *gu = reinterpret_cast<uint16_t *>(ws + L.gu);
   uint16_t *h = reinterpret_cast<uint16_t *>(ws + L.h);
@@ -207,9 +216,9 @@ int amla_swiglu(const void *x, int64_t m, int64_t k, const void *gate_w, const f
     p.y = h;
     p.ldy = (int)n;
     p.seq_len = 1;
-    if ((rc = launch_gemm(p, GEMV_SILU, st, part, L.part_bytes))) return rc;
+    if ((rc = launch_gemm(p, GEMV_SILU, st, part, part_bytes))) return rc;
     return fp8_linear_into(h, (int)m, (int)n, static_cast<const uint8_t *>(down_w), down_s, (int)k,
-                           static_cast<uint16_t *>(y), part, L.part_bytes, st);
+                           static_cast<uint16_t *>(y), part, part_bytes, st);
   }
   // gate and up as one GEMM over the two stacked weights: rows (m, [gate | up])
   GemvParams p = {};
@@ -235,7 +244,7 @@ int amla_swiglu(const void *x, int64_t m, int64_t k, const void *gate_w, const f
     gu_finish_silu_kernel<<<(unsigned)((items + 63) / 64), 64, 0, st>>>(part, (int)m, (int)n, pl.kparts, h);
     if ((rc = check_launch("swiglu gate|up finish + silu_mul"))) return rc;
     return fp8_linear_into(h, (int)m, (int)n, static_cast<const uint8_t *>(down_w), down_s, (int)k,
-                           static_cast<uint16_t *>(y), part, L.part_bytes, st);
+                           static_cast<uint16_t *>(y), part, part_bytes, st);
   }
   rc = launch_gemv(p, GEMV_PLAIN, pl, st);
   if (rc) return rc;
@@ -244,7 +253,7 @@ int amla_swiglu(const void *x, int64_t m, int64_t k, const void *gate_w, const f
                          256, 0, st>>>(gu, (int)m, (int)n, h);
   if ((rc = check_launch("swiglu silu_mul"))) return rc;
   return fp8_linear_into(h, (int)m, (int)n, static_cast<const uint8_t *>(down_w), down_s, (int)k,
-                         static_cast<uint16_t *>(y), part, L.part_bytes, st);
+                         static_cast<uint16_t *>(y), part, part_bytes, st);
 }
 
 }  // extern "C"
@@ -542,12 +551,16 @@ int amla_moe_route(const void *hidden, int64_t m, int64_t d, const void *gate_we
   if (top_k > 64) return fail(AMLA_EUNSUPPORTED, "moe_route: top_k > 64");
   if (d % 32 || !aligned16(hidden) || !aligned16(gate_weight) || m > (int64_t)65535 * 16 || d > INT32_MAX)
     return fail(AMLA_EUNSUPPORTED, "moe_route: needs hidden size %% 32 == 0 and 16-byte aligned inputs");
-  const size_t need = amla_moe_route_workspace_bytes(m, n_experts);
+  // above ROUTE_WIDE_M tokens the K splits are for speed alone: as many as there is room for
+  const size_t one = (size_t)m * n_experts * 4;
+  int ks = route_ksplit(m, n_experts);
+  const size_t need = m > ROUTE_WIDE_M ? one : amla_moe_route_workspace_bytes(m, n_experts);
   if (!workspace || workspace_bytes < need || !aligned16(workspace))
-    return fail(AMLA_EWORKSPACE, "moe_route: needs %zu bytes of 16-byte aligned workspace", need);
+    return fail(AMLA_EWORKSPACE, "moe_route: needs %zu bytes of 16-byte aligned workspace (got %zu)", need,
+                workspace ? workspace_bytes : (size_t)0);
+  if (m > ROUTE_WIDE_M) ks = (int)std::min<size_t>(ks, workspace_bytes / one);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   float *part = static_cast<float *>(workspace);
-  const int ks = route_ksplit(m, n_experts);
   const uint16_t *hid = static_cast<const uint16_t *>(hidden), *gw = static_cast<const uint16_t *>(gate_weight);
   if (m > ROUTE_WIDE_M)
     route_logits_wide_kernel<<<dim3((unsigned)((n_experts + 63) / 64), (unsigned)((m + 63) / 64), (unsigned)ks), 256, 0,

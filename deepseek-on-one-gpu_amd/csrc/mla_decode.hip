@@ -1611,12 +1611,16 @@ bool prefill_absorbed(int batch, int seq_len, int context) {
   return (double)((tokens + n - 1) / n) * chunk < 0.95 * direct;
 }
 
+// Sized for every launch sequence of up to min(tokens, 64) tokens, so that a
+// buffer for more tokens holds any smaller call: the slots grow with the tokens
+// but for one step, where the splits go from one tile each to two.
 static size_t absorbed_scratch(int64_t tokens, int context, char *base, AbsorbedScratch *sc) {
-  const int chunk = absorbed_chunk(tokens), last = (int)(tokens - (tokens - 1) / chunk * chunk);
-  int units, slots, last_slots;  // a smaller last chunk may take more one-tile splits
+  const int chunk = (int)std::min<int64_t>(tokens, DECODE_MAX_BATCH);
+  const int one_tile = std::min(chunk, 64 / std::max(1, (context + TT - 1) / TT));
+  int units, slots, slots1 = 0;
   attn_units(chunk, context, units, slots);
-  attn_units(last, context, units, last_slots);
-  slots = std::max(slots, last_slots);
+  if (one_tile > 0) attn_units(one_tile, context, units, slots1);
+  slots = std::max(slots, slots1);
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
   const size_t plan = take(plan_ints(chunk, slots) * 4), qbuf = take((size_t)chunk * HEADS * QKD * 2),

@@ -487,22 +487,23 @@ static int run_linear(const GemvParams &p, int mode, hipStream_t st, size_t lin_
 
 struct PrefillLayout {
   size_t xn, qa, qan, q, kvn, kpe, kvb, attn, lat, lin, lin_bytes, total;
+  size_t need;  // without the K-part sums of the GEMMs above 64 rows: less than this is refused
   int Tmax;
   bool absorbed;  // attention in latent space: no kv_b rows
 };
 
-static PrefillLayout prefill_layout(const amla_mla_args &a) {
+static PrefillLayout prefill_layout(const amla_mla_args &a, bool absorbed) {
   PrefillLayout L = {};
   const size_t M = (size_t)a.batch * a.seq_len;
   const int HD = a.qk_nope + a.qk_rope;
   L.Tmax = std::min(mla_context_bound(a), a.max_seq);
+  L.absorbed = absorbed;
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
   L.xn = take(M * a.hidden * 2);
   L.qa = take(M * a.q_lora * 2);
   L.qan = take(M * a.q_lora * 2);
   L.q = take(M * a.heads * HD * 2);
-  L.absorbed = prefill_absorbed(a.batch, a.seq_len, L.Tmax);
   if (L.absorbed) {
     L.lat = take(prefill_absorbed_ws_bytes(a.batch, a.seq_len, L.Tmax));
   } else {
@@ -511,21 +512,61 @@ static PrefillLayout prefill_layout(const amla_mla_args &a) {
     L.kvb = take((size_t)L.Tmax * a.heads * (a.qk_nope + a.v_dim) * 2);
   }
   L.attn = take(M * a.heads * a.v_dim * 2);
-  // K-part sums of the skinny linears (M <= 64), or the K-split partial sums
-  // of the large-M GEMMs
-  size_t lin = 0;
+  // K-part sums of the skinny linears (M <= 64), which those need, or of the
+  // large-M GEMMs, which run without them on whole tiles
+  size_t skinny = 0, lin = 0;
   const int HDv = a.qk_nope + a.v_dim;
-  auto need = [&](int m, int n, int k) {
-    lin = std::max(lin, m <= 64 ? plan_linear(m, n, k).part_bytes : gemm_ws_bytes(m, n, k));
+  auto sums = [&](int m, int n, int k) {
+    if (m <= 64) skinny = std::max(skinny, plan_linear(m, n, k).part_bytes);
+    else lin = std::max(lin, gemm_ws_bytes(m, n, k));
   };
-  need((int)M, a.q_lora + a.kv_lora + a.qk_rope, a.hidden);
-  need((int)M, a.heads * HD, a.q_lora);
-  if (!L.absorbed) need(L.Tmax, a.heads * HDv, a.kv_lora);
-  need((int)M, a.hidden, a.heads * a.v_dim);
-  L.lin = take(lin);
-  L.lin_bytes = lin;
-  L.total = off;
+  sums((int)M, a.q_lora + a.kv_lora + a.qk_rope, a.hidden);
+  sums((int)M, a.heads * HD, a.q_lora);
+  if (!L.absorbed) sums(L.Tmax, a.heads * HDv, a.kv_lora);
+  sums((int)M, a.hidden, a.heads * a.v_dim);
+  L.lin = off;
+  L.lin_bytes = std::max(skinny, lin);
+  L.need = off + align_up(skinny, 256);
+  L.total = off + align_up(L.lin_bytes, 256);
   return L;
+}
+
+static bool prefers_absorbed(const amla_mla_args &a) {
+  return prefill_absorbed(a.batch, a.seq_len, std::min(mla_context_bound(a), a.max_seq));
+}
+
+// The size to ask for: the faster form with every K part, and enough for any
+// smaller call over as many rows (the skinny linears' K-part counts change at
+// 16 and 32 rows; the form that fits runs, choose_prefill).
+static size_t prefill_ws_bytes(const amla_mla_args &a) {
+  PrefillLayout L = prefill_layout(a, prefers_absorbed(a));
+  size_t total = L.total;
+  const int64_t M = (int64_t)a.batch * a.seq_len;
+  const int HD = a.qk_nope + a.qk_rope, HDv = a.qk_nope + a.v_dim;
+  for (int t : {8, 16, 32, 64}) {
+    if (t >= M) break;
+    size_t part = plan_linear(t, a.q_lora + a.kv_lora + a.qk_rope, a.hidden).part_bytes;
+    part = std::max(part, plan_linear(t, a.heads * HD, a.q_lora).part_bytes);
+    part = std::max(part, plan_linear(t, a.hidden, a.heads * a.v_dim).part_bytes);
+    if (!L.absorbed && L.Tmax <= 64) part = std::max(part, plan_linear(L.Tmax, a.heads * HDv, a.kv_lora).part_bytes);
+    total = std::max(total, L.lin + align_up(part, 256));
+  }
+  return total;
+}
+
+// The faster form of the attention if its scratch fits in the workspace, else
+// the other one if that fits.
+static int choose_prefill(const amla_mla_args &a, PrefillLayout *out) {
+  const bool first = prefers_absorbed(a);
+  size_t least = SIZE_MAX;
+  for (bool absorbed : {first, !first}) {
+    *out = prefill_layout(a, absorbed);
+    least = std::min(least, out->need);
+    if (a.workspace_bytes < out->need) continue;
+    out->lin_bytes = std::min(out->lin_bytes, a.workspace_bytes - out->lin);
+    return AMLA_OK;
+  }
+  return fail(AMLA_EWORKSPACE, "mla_prefill: workspace %zu bytes < %zu needed", a.workspace_bytes, least);
 }
 
 int prefill_impl(const amla_mla_args *a, hipStream_t st);
@@ -537,9 +578,8 @@ namespace amla {
 int prefill_impl(const amla_mla_args *a, hipStream_t st) {
   int rc = check_mla_common(a, "mla_prefill");
   if (rc) return rc;
-  const PrefillLayout L = prefill_layout(*a);
-  if (a->workspace_bytes < L.total)
-    return fail(AMLA_EWORKSPACE, "mla_prefill: workspace %zu bytes < %zu needed", a->workspace_bytes, L.total);
+  PrefillLayout L;
+  if ((rc = choose_prefill(*a, &L))) return rc;
   char *ws = reinterpret_cast<char *>(a->workspace);
   const int B = a->batch, S = a->seq_len, M = B * S;
   const int HD = a->qk_nope + a->qk_rope;
@@ -640,7 +680,7 @@ extern "C" {
 
 size_t amla_mla_prefill_workspace_bytes(const amla_mla_args *a) {
   if (!a || a->batch <= 0 || a->seq_len <= 0) return 0;
-  return amla::prefill_layout(*a).total;
+  return amla::prefill_ws_bytes(*a);
 }
 
 int amla_mla_prefill(const amla_mla_args *a, void *stream) {

@@ -176,7 +176,10 @@ int amla_mla_decode_noalloc(const amla_mla_args *args, void *stream);
 int amla_mla_prefill(const amla_mla_args *args, void *stream);
 
 /* Workspace bytes amla_mla_decode / amla_mla_prefill need for these args
- * (pointer fields are ignored).  Scratch only: no contents carry between calls. */
+ * (pointer fields are ignored).  Scratch only: no contents carry between calls.
+ * A prefill's size also holds one of fewer tokens over as many rows, which may
+ * then run slower than with its own: the form of the attention whose scratch
+ * fits, the K-part sums of its larger GEMMs in what room there is. */
 size_t amla_mla_decode_workspace_bytes(const amla_mla_args *args);
 size_t amla_mla_prefill_workspace_bytes(const amla_mla_args *args);
 
@@ -193,7 +196,9 @@ int amla_silu_mul(const void *gate, const void *up, int64_t numel, void *out, vo
  * x (m, k) bf16; gate_w, up_w (n, k) e4m3fn with (ceil(n/128), ceil(k/128))
  * fp32 scales; down_w (k, n) with (ceil(k/128), ceil(n/128)) scales; y (m, k)
  * bf16.  k and n multiples of 128.  Workspace (16-byte aligned) of
- * amla_swiglu_workspace_bytes(m, k, n) bytes; scratch only. */
+ * amla_swiglu_workspace_bytes(m, k, n) bytes; scratch only.  That size also
+ * holds any call with fewer rows, which may then run slower than with its own:
+ * above 64 rows the K-part sums are optional and take what room there is. */
 int amla_swiglu(const void *x, int64_t m, int64_t k, const void *gate_w, const float *gate_s, const void *up_w,
                 const float *up_s, int64_t n, const void *down_w, const float *down_s, void *y, void *workspace,
                 size_t workspace_bytes, void *stream);
@@ -207,7 +212,9 @@ size_t amla_swiglu_workspace_bytes(int64_t m, int64_t k, int64_t n);
  *   norm_topk_prob.
  * hidden (m, d) bf16 (d % 32 == 0); gate_weight (n_experts, d) bf16;
  * indices (m, top_k) int64, weights (m, top_k) fp32.  Workspace of
- * amla_moe_route_workspace_bytes(m, n_experts) bytes (the fp32 logits). */
+ * amla_moe_route_workspace_bytes(m, n_experts) bytes (the fp32 logits of every
+ * K split); above 64 tokens m * n_experts * 4 bytes are enough, with fewer
+ * splits. */
 int amla_moe_route(const void *hidden, int64_t m, int64_t d, const void *gate_weight, int64_t n_experts,
                    int n_group, int topk_group, int top_k, int norm_topk_prob, int64_t *indices, float *weights,
                    void *workspace, size_t workspace_bytes, void *stream);

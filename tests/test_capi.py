@@ -191,6 +191,56 @@ def test_moe_experts_dev_checks_sizes_on_the_host():
     assert L.amla_moe_experts_dev(p, 0, d, top_k, p, n, E, p, p, p, 0, None) == 0  # nothing to do
 
 
+def _least(call):
+    """The workspace a call with none asks for before it launches anything."""
+    assert call() == -2
+    m = re.search(rb"needs (\d+) bytes|< (\d+) needed", _lib.lib().amla_last_error())
+    return int(m.group(1) or m.group(2))
+
+
+def _largest_smaller_call(ms, size, least):
+    """Every m: the size asked for holds each call of the list with at most m rows."""
+    worst = 0
+    for m in ms:
+        worst = max(worst, least(m))
+        assert size(m) >= worst, f"a buffer for {m} rows is refused by a smaller call ({size(m)} < {worst})"
+
+
+ROWS = [*range(1, 70), 80, 96, 100, 128, 129, *range(150, 700, 37), 1000, 1472, 1536, 1920, 2048, 3713, 3840, 4096]
+
+
+@pytest.mark.parametrize("n,k", [(18432, 7168), (2048, 7168), (512, 1024)])
+def test_swiglu_workspace_for_more_rows_holds_fewer(n, k):
+    L, p = _lib.lib(), 1 << 12  # an aligned address, never read
+    _largest_smaller_call(ROWS, lambda m: L.amla_swiglu_workspace_bytes(m, k, n),
+                          lambda m: _least(lambda: L.amla_swiglu(p, m, k, p, p, p, p, n, p, p, p, None, 0, None)))
+
+
+@pytest.mark.parametrize("E", [16, 64, 256])
+def test_route_workspace_for_more_tokens_holds_fewer(E):
+    L, p = _lib.lib(), 1 << 12
+    _largest_smaller_call([m for m in ROWS if m > 64], lambda m: L.amla_moe_route_workspace_bytes(m, E),
+                          lambda m: _least(lambda: L.amla_moe_route(p, m, 7168, p, E, 4, 2, 4, 1, p, p, None, 0, None)))
+
+
+@pytest.mark.parametrize("batch,rows", [(1, 333), (1, 8192), (1, 32768), (4, 256), (4, 1024), (13, 64), (13, 4096)])
+def test_prefill_workspace_for_more_tokens_holds_fewer(batch, rows):
+    L, a = _lib.lib(), _lib.MlaArgs()
+    for name, kind in a._fields_:
+        if kind is ctypes.c_void_p:
+            setattr(a, name, 1 << 12)
+    a.hidden, a.heads, a.q_lora, a.kv_lora, a.qk_nope, a.qk_rope, a.v_dim = 7168, 128, 1536, 512, 128, 64, 128
+    a.batch, a.max_seq, a.rope_rows, a.eps, a.softmax_scale, a.workspace_bytes = batch, rows, rows, 1e-6, 0.1, 0
+
+    def at(s, call):
+        a.seq_len = s
+        return call()
+
+    _largest_smaller_call([s for s in ROWS if s <= rows and s * batch <= 4096],
+                          lambda s: at(s, lambda: L.amla_mla_prefill_workspace_bytes(ctypes.byref(a))),
+                          lambda s: at(s, lambda: _least(lambda: L.amla_mla_prefill(ctypes.byref(a), None))))
+
+
 def test_sample_checks_sizes_on_the_host():
     """amla_sample: the workspace it asks for (three level histograms per row, chunk maxima and
     kept masses), and the arguments it rejects before any launch."""
