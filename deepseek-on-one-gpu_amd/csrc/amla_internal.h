@@ -132,8 +132,8 @@ AMLA_DEV void moe_sched_weights(GemvParams &p, const MoeSched &s, int e) {
   p.w1 = s.down ? nullptr : static_cast<const uint8_t *>(t[2 * s.E + e]);
   p.s1 = s.down ? nullptr : static_cast<const float *>(t[3 * s.E + e]);
 }
-// Skinny GEMMs of the scheduled entries, each with at most 16 rows; grid
-// max_entries x plan.groups.  plan: plan_gemv_grouped(16 or less, N, K);
+// Skinny GEMMs of the scheduled entries, each with at most max_m <= 64 rows; grid
+// max_entries x plan.groups.  plan: plan_gemv_grouped(max_m, N, K);
 // p.part holds plan.kparts * positions * N fp32 when kparts > 1 (an entry at
 // position r0 uses part + kparts * r0 * N).  down = 0: p.x hidden, p.y the
 // [gate | up] rows by position (used with one K part only), h the silu(gate) *

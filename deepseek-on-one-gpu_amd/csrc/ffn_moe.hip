@@ -608,7 +608,37 @@ namespace amla {
 // copy their lists into the workspace
 constexpr int MOE_ARG_SLOTS = 512;
 constexpr int MOE_MAX_SLOTS = 65536;  // slots per chunk
-constexpr int MOE_SKINNY_ROWS = 16;   // largest group on the skinny path (one MFMA row tile)
+constexpr int MOE_SKINNY_ROWS = 64;   // most rows of an entry on the skinny GEMM
+
+// Which kernels a set of groups takes.  The tiles walk the whole K in each
+// workgroup, so with few experts most of the machine idles where the skinny GEMM
+// cuts K into parts; with many both are weight streams and the tiles, which read
+// whole lines, are the faster one unless the groups are a row or two each.
+// Measured on MI355X, hidden 7168 x intermediate 2048, top 2 of E experts (host
+// lists; us, skinny / tiles): E = 1 32 rows each 55 / 94, 64 rows 72 / 124;
+// E = 4 24 rows 69 / 95, 50 rows 88 / 125; E = 8 8 rows 86 / 99, 25 rows 103 /
+// 104; top 8 of 16 16 rows 184 / 146; of 64 12 rows 626 / 520; 2048 x 1536 E = 4
+// 24 rows 53 / 44.  Model of both projections in us (entries: groups, cut to the
+// rows a workgroup takes; K block times as in plan_gemm_split):
+static double moe_skinny_us(double entries, double slots, int rows_max, int64_t d, int64_t n) {
+  const double bytes = 3.0 * n * d * entries;
+  return std::max(rows_max > 32 ? 63.0 : 45.0, bytes * (1.0 + 0.025 * slots / std::max(entries, 1.0)) / 6.1e6);
+}
+static double moe_tiles_us(double entries, double rows_max, int64_t d, int64_t n) {
+  const double nj = std::ceil(std::min<double>(rows_max, TILE_ROWS) / 32), one = 0.9 + 0.3 * nj,
+               two = std::max(1.3, 0.925 * nj);
+  auto pass = [&](double blocks, int64_t k) {
+    return k / 128 * (blocks <= 256 ? one : std::ceil(blocks / 512) * two);
+  };
+  return std::max(8.0 + pass(entries * (n / 128), d) + pass(entries * ((d + 255) / 256), n),
+                  3.0 * n * d * entries / 5.8e6);
+}
+// K parts within what the skinny GEMM's finishing passes add up (hidden sizes
+// above 32768 are past it)
+static bool moe_skinny_fits(int rows, int64_t d, int64_t n) {
+  return plan_gemv_grouped(rows, (int)(2 * n), (int)d).kparts <= GEMV_MAX_PARTS &&
+         plan_gemv_grouped(rows, (int)d, (int)n).kparts <= GEMV_MAX_PARTS;
+}
 
 struct RowList {
   int32_t row[MOE_ARG_SLOTS];
@@ -638,7 +668,6 @@ static MoeLayout moe_layout(int64_t m, int64_t d, int top_k, int64_t n) {
   MoeLayout L;
   L.chunk_tokens = (int)std::min<int64_t>(m, (m * top_k <= MOE_ARG_SLOTS ? MOE_ARG_SLOTS : MOE_MAX_SLOTS) / top_k);
   const size_t slots = (size_t)L.chunk_tokens * top_k;
-  const int mg = (int)std::min<size_t>(slots, MOE_SKINNY_ROWS);  // largest expert group on the skinny path
   size_t off = 0;
   L.lists = off;
   off = align_up(off + (slots > MOE_ARG_SLOTS ? 2 * slots * 4 : 0), 256);
@@ -651,11 +680,14 @@ static MoeLayout moe_layout(int64_t m, int64_t d, int top_k, int64_t n) {
   L.h = off;
   off = align_up(off + slots * n * 2, 256);
   L.part = off;
-  // partial sums of every group of one grouped launch, each sized for its own rows
-  const GemvPlan a = plan_gemv(mg, (int)(2 * n), (int)d), b = plan_gemv(mg, (int)d, (int)n);
-  const size_t pa = a.kparts > 1 ? (size_t)a.kparts * slots * 2 * n * 4 : 0;
-  const size_t pb = b.kparts > 1 ? (size_t)b.kparts * slots * d * 4 : 0;
-  L.part_bytes = std::max(pa, pb);
+  // partial sums of every group of one grouped launch, each sized for its own
+  // rows (the K parts of the largest group's plan: 16, 32 or 64 rows)
+  L.part_bytes = 0;
+  for (int mg : {16, 32, 64}) {
+    const GemvPlan a = plan_gemv(mg, (int)(2 * n), (int)d), b = plan_gemv(mg, (int)d, (int)n);
+    if (a.kparts > 1) L.part_bytes = std::max(L.part_bytes, (size_t)a.kparts * slots * 2 * n * 4);
+    if (b.kparts > 1) L.part_bytes = std::max(L.part_bytes, (size_t)b.kparts * slots * d * 4);
+  }
   off = align_up(off + L.part_bytes, 256);
   L.total = off;
   return L;
@@ -746,10 +778,10 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
       if (i == 0 || ix[order[i]] != ix[order[i - 1]]) run_begin.push_back(i);
     run_begin.push_back(ns);
     const int nruns = (int)run_begin.size() - 1;
-    int max_small = 0;
-    for (int r = 0; r < nruns; ++r)
-      if (run_begin[r + 1] - run_begin[r] <= MOE_SKINNY_ROWS)
-        max_small = std::max(max_small, run_begin[r + 1] - run_begin[r]);
+    int max_run = 0;
+    for (int r = 0; r < nruns; ++r) max_run = std::max(max_run, run_begin[r + 1] - run_begin[r]);
+    const bool tiles = max_run > MOE_SKINNY_ROWS || !moe_skinny_fits(max_run, d, n) ||
+                       moe_tiles_us(nruns, max_run, d, n) < 0.95 * moe_skinny_us(nruns, ns, max_run, d, n);
     GemvParams pg = {};  // [gate | up] x (cnt, D) -> gu (cnt, 2n)
     pg.ldx = D;
     pg.N = 2 * n;
@@ -764,11 +796,35 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
     pd.n_split = D;
     pd.ldy = D;
     pd.seq_len = 1;
-    const GemvPlan plan_g = plan_gemv_grouped(std::max(max_small, 1), 2 * n, D);
-    const GemvPlan plan_d = plan_gemv_grouped(std::max(max_small, 1), D, n);
+    const GemvPlan plan_g = plan_gemv_grouped(std::min(max_run, MOE_SKINNY_ROWS), 2 * n, D);
+    const GemvPlan plan_d = plan_gemv_grouped(std::min(max_run, MOE_SKINNY_ROWS), D, n);
     const MoeTileParams tg = {xs, hb, D, n, D, n, 0, false}, td = {hb, ys, n, D, n, D, 0, false};
     for (int pass = 0; pass < 2; ++pass) {
-      // groups of up to 16 rows: grouped skinny GEMMs, GEMV_MAX_GROUPS experts per launch
+      if (tiles) {
+        // tiles of up to 128 rows, silu * up in their epilogue
+        TileGroups tl;
+        tl.n = 0;
+        for (int r = 0; r < nruns; ++r) {
+          const int i0 = run_begin[r], cnt = run_begin[r + 1] - i0;
+          const int64_t e = ix[order[i0]];
+          for (int c = 0; c < cnt; c += TILE_ROWS) {
+            TileGroup &g = tl.g[tl.n++];
+            g.w0 = pass == 0 ? gate_w[e] : down_w[e];
+            g.s0 = pass == 0 ? gate_s[e] : down_s[e];
+            g.w1 = pass == 0 ? up_w[e] : nullptr;
+            g.s1 = pass == 0 ? up_s[e] : nullptr;
+            g.first = i0 + c;
+            g.rows = std::min(TILE_ROWS, cnt - c);
+            if (tl.n == TILE_MAX_GROUPS) {
+              if ((rc = launch_tile_grouped(pass == 0 ? tg : td, tl, pass == 1, st))) return rc;
+              tl.n = 0;
+            }
+          }
+        }
+        if (tl.n && (rc = launch_tile_grouped(pass == 0 ? tg : td, tl, pass == 1, st))) return rc;
+        continue;
+      }
+      // grouped skinny GEMMs, GEMV_MAX_GROUPS experts per launch
       const GemvPlan &pl = pass == 0 ? plan_g : plan_d;
       const GemvParams &base = pass == 0 ? pg : pd;
       if (pl.kparts > 1 && (size_t)pl.kparts * ns * base.N * 4 > L.part_bytes)
@@ -777,18 +833,11 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
       GemvGroups gr;
       gr.n = 0;
       gr.units = 0;
-      for (int r = 0; r <= nruns; ++r) {
-        const bool flush = r == nruns || gr.n == GEMV_MAX_GROUPS;
-        if (flush && gr.n) {
-          if ((rc = launch_gemv_grouped(base, gr, pl, st))) return rc;
-          gr.n = 0;
-        }
-        if (r == nruns) break;
-        const int i0 = run_begin[r], cnt = run_begin[r + 1] - i0;
-        if (cnt > MOE_SKINNY_ROWS) continue;
+      for (int r = 0; r < nruns; ++r) {
+        const int i0 = run_begin[r];
         const int64_t e = ix[order[i0]];
         GemvGroup &g = gr.g[gr.n++];
-        g.M = cnt;
+        g.M = run_begin[r + 1] - i0;
         g.pad = 0;
         if (pass == 0) {
           g.x = xs + (size_t)i0 * D;
@@ -807,35 +856,16 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
           g.y = ys + (size_t)i0 * D;
           g.part = pl.kparts > 1 ? part + (size_t)pl.kparts * i0 * D : nullptr;
         }
+        if (gr.n == GEMV_MAX_GROUPS || r + 1 == nruns) {
+          if ((rc = launch_gemv_grouped(base, gr, pl, st))) return rc;
+          gr.n = 0;
+        }
       }
-      if (pass == 0 && max_small) {
-        // silu * up over every row of [gate | up] (the tiles below write the larger groups' rows of h)
+      if (pass == 0) {
         silu_mul_rows_kernel<<<dim3((unsigned)std::max(1, std::min(n / 8 / 256, 16)), (unsigned)std::min(ns, 65535)),
                                256, 0, st>>>(gu, ns, n, hb);
         if ((rc = check_launch("moe_experts silu_mul"))) return rc;
       }
-      // larger groups: tiles of up to 128 rows, silu * up in their epilogue
-      TileGroups tl;
-      tl.n = 0;
-      for (int r = 0; r <= nruns; ++r) {
-        const int i0 = r < nruns ? run_begin[r] : 0, cnt = r < nruns ? run_begin[r + 1] - i0 : 0;
-        if (r < nruns && cnt <= MOE_SKINNY_ROWS) continue;
-        const int64_t e = r < nruns ? ix[order[i0]] : 0;
-        for (int c = 0; c < cnt; c += TILE_ROWS) {
-          TileGroup &g = tl.g[tl.n++];
-          g.w0 = pass == 0 ? gate_w[e] : down_w[e];
-          g.s0 = pass == 0 ? gate_s[e] : down_s[e];
-          g.w1 = pass == 0 ? up_w[e] : nullptr;
-          g.s1 = pass == 0 ? up_s[e] : nullptr;
-          g.first = i0 + c;
-          g.rows = std::min(TILE_ROWS, cnt - c);
-          if (tl.n == TILE_MAX_GROUPS) {
-            if ((rc = launch_tile_grouped(pass == 0 ? tg : td, tl, pass == 1, st))) return rc;
-            tl.n = 0;
-          }
-        }
-      }
-      if (tl.n && (rc = launch_tile_grouped(pass == 0 ? tg : td, tl, pass == 1, st))) return rc;
     }
     move_rows_kernel<true><<<ns, 256, 0, st>>>(ys, d, ns, scatter, dsc, eout);
     if ((rc = check_launch("moe_experts scatter"))) return rc;
@@ -865,16 +895,34 @@ struct MoeDevLayout {
   size_t hdr, count, gather, scatter, ent, gu, h, part, total;
 };
 
-static MoeDevLayout moe_dev_layout(int64_t m, int64_t d, int top_k, int64_t n, int64_t E) {
+// Rows of an entry on the skinny GEMM, or 0: the tiles.  Up to 32 tokens the
+// groups (1-2 rows per expert) stream through the skinny GEMM.  [gate | up] +
+// down with their passes at R1 shapes, skinny against tiles: 3 tokens 185 / 214
+// us, 8 tokens 443 / 472, 16 tokens 754 / 788, 40 tokens 1376 / 1377, 128 tokens
+// 2091 / 1885, 300 tokens 2343 / 1936.  Entries of 16 rows there, of 32 where
+// cutting the groups would read many weights twice (top 8 of 8, 24 tokens 118 us
+// against 146; top 4 of 4 of 2048 x 1536, where the machine idles, 54 / 48).  Above 32 tokens
+// only a few experts do, as the groups a random routing gives (the sizes are
+// known to the device alone) of up to 64 rows on average: top 2 of 4, 64 tokens
+// 93 us against 125, 100 tokens 99 / 125, 200 tokens 172 / 168; of 8, 64 tokens
+// 98 / 99; one expert, 64 tokens 58 / 125.
+static int moe_dev_skinny_rows(int64_t m, int64_t d, int top_k, int64_t n, int64_t E) {
+  const double S = (double)m * top_k;
+  const double present = E * (1.0 - std::pow(1.0 - std::min(1.0, (double)top_k / E), (double)m)), c = S / present;
+  if (!moe_skinny_fits(32, d, n)) return 0;
+  if (m <= 32) return c > 14 && S / 16 * 3 * n * d > 60 * 4.8e6 ? 32 : (int)std::min<int64_t>(m, 16);
+  if (c > MOE_SKINNY_ROWS) return 0;
+  const double entries = present * std::max(1.0, std::min(c / 32 + 0.5, std::ceil(m / 32.0)));
+  const double skinny = 25.0 + std::max(27.0, entries * 3 * n * d / 4.8e6);
+  const double tiles = moe_tiles_us(present, std::min((double)m, c + 2 * std::sqrt(c)), d, n);
+  return skinny < 0.85 * tiles ? 32 : 0;
+}
+
+static MoeDevLayout moe_dev_layout(int64_t m, int64_t d, int top_k, int64_t n, int64_t E, int skinny_rows) {
   MoeDevLayout L;
   const int64_t S = m * top_k;
-  // Up to 32 tokens the groups (1-2 rows per expert) stream through the skinny
-  // GEMM, above that through the large tiles.  [gate | up] + down with their
-  // passes at R1 shapes, skinny against tiles: 3 tokens 185 / 214 us, 8 tokens
-  // 443 / 472, 16 tokens 754 / 788, 40 tokens 1376 / 1377, 128 tokens 2091 /
-  // 1885, 300 tokens 2343 / 1936.  Longer groups are cut into entries.
-  L.tiles = m > 32;
-  L.rows = L.tiles ? TILE_ROWS : (int)std::min<int64_t>(m, MOE_SKINNY_ROWS);
+  L.tiles = skinny_rows == 0;
+  L.rows = L.tiles ? TILE_ROWS : skinny_rows;
   L.max_entries = (int)std::min<int64_t>(S, std::min<int64_t>(E, S) + S / L.rows);
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align_up(off + bytes, 256); return o; };
@@ -1027,7 +1075,7 @@ size_t amla_moe_experts_dev_workspace_bytes(int64_t m, int64_t d, int top_k, int
   if (m <= 0 || d <= 0 || top_k <= 0 || top_k > 64 || n_inter <= 0 || n_experts <= 0 ||
       n_experts > MSORT_MAXE || m * top_k > MOE_DEV_MAX_SLOTS)
     return 0;
-  return moe_dev_layout(m, d, top_k, n_inter, n_experts).total;
+  return moe_dev_layout(m, d, top_k, n_inter, n_experts, moe_dev_skinny_rows(m, d, top_k, n_inter, n_experts)).total;
 }
 
 int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, const int64_t *indices,
@@ -1044,7 +1092,8 @@ int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, co
       !aligned16(expert_out))
     return fail(AMLA_EUNSUPPORTED,
                 "moe_experts_dev: needs hidden %% 128 == 0, intermediate %% 256 == 0 and 16-byte aligned rows");
-  const MoeDevLayout L = moe_dev_layout(m, d, top_k, n_inter, n_experts);
+  const MoeDevLayout L =
+      moe_dev_layout(m, d, top_k, n_inter, n_experts, moe_dev_skinny_rows(m, d, top_k, n_inter, n_experts));
   if (!workspace || workspace_bytes < L.total || !aligned16(workspace))
     return fail(AMLA_EWORKSPACE, "moe_experts_dev: needs %zu bytes of 16-byte aligned workspace (got %zu)", L.total,
                 workspace ? workspace_bytes : (size_t)0);

@@ -464,9 +464,10 @@ __global__ __launch_bounds__(64) void gemv_finish_grouped(GemvParams p, GemvGrou
   gemv_finish_body<GEMV_PLAIN>(q, (int64_t)(blockIdx.x % gr.units) * 64 + threadIdx.x, kparts);
 }
 
-// Skinny GEMMs of a device schedule (routed experts, up to 16 rows each):
+// Skinny GEMMs of a device schedule (routed experts, up to 16 MT rows each):
 // entry g = blockIdx.x / units; entries past the device count return at once
 // (uniform per workgroup).
+template <int MT>
 __global__ __launch_bounds__(256, 2) void gemv_sched_kernel(GemvParams p, MoeSched s, int units, int rg, int kparts,
                                                          int kpb) {
   const int g = blockIdx.x / units;
@@ -478,7 +479,7 @@ __global__ __launch_bounds__(256, 2) void gemv_sched_kernel(GemvParams p, MoeSch
   else p.y += (size_t)r0 * p.ldy;
   p.part += (size_t)kparts * r0 * p.N;
   moe_sched_weights(p, s, e);
-  gemv_body<1, GEMV_PLAIN, true>(p, blockIdx.x % units, rg, kparts, kpb, s.down ? nullptr : s.rowmap + r0,
+  gemv_body<MT, GEMV_PLAIN, true>(p, blockIdx.x % units, rg, kparts, kpb, s.down ? nullptr : s.rowmap + r0,
                                  s.down ? s.rowmap + r0 : nullptr);
 }
 
@@ -1922,25 +1923,35 @@ int launch_gemv_grouped(const GemvParams &p, GemvGroups gr, const GemvPlan &pl, 
   return check_launch("grouped fp8 skinny GEMM");
 }
 
+template <int MT>
+static void launch_sched_mt(const GemvParams &p, const MoeSched &s, int max_entries, const GemvPlan &pl,
+                            hipStream_t st) {
+  static bool attr_set = false;  // raise the dynamic LDS limit once per process
+  if (!attr_set) {
+    (void)hipFuncSetAttribute((const void *)gemv_sched_kernel<MT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              160 * 1024);
+    attr_set = true;
+  }
+  gemv_sched_kernel<MT><<<dim3((unsigned)(max_entries * pl.groups)), 256, pl.lds, st>>>(p, s, pl.groups, pl.rg,
+                                                                                      pl.kparts, pl.kpb);
+}
+
 int launch_gemv_sched(const GemvParams &p, const MoeSched &s, int max_entries, int max_m, const GemvPlan &pl,
                       uint16_t *h, hipStream_t st) {
   if (max_entries <= 0) return AMLA_OK;
-  if (max_m < 1 || max_m > 16) return fail(AMLA_EINVAL, "scheduled skinny GEMM: max rows %d", max_m);
+  if (max_m < 1 || max_m > 64) return fail(AMLA_EINVAL, "scheduled skinny GEMM: max rows %d", max_m);
   if (p.N % 16 || p.K % 128 || pl.kparts > GEMV_MAX_PARTS || (!s.down && (p.n_split % 128 || p.N != 2 * p.n_split)))
     return fail(AMLA_EUNSUPPORTED, "scheduled skinny GEMM: unsupported shape N=%d K=%d", p.N, p.K);
   if (pl.kparts > 1 && !p.part) return fail(AMLA_EWORKSPACE, "scheduled skinny GEMM: missing partial sums");
-  if (gemv_lds_bytes(1, pl.kpb, pl.rg, pl.kparts) > pl.lds || pl.kpb > gemv_kpb_max(1))
+  const int MT = max_m <= 16 ? 1 : (max_m <= 32 ? 2 : 4);
+  if (gemv_lds_bytes(MT, pl.kpb, pl.rg, pl.kparts) > pl.lds || pl.kpb > gemv_kpb_max(MT))
     return fail(AMLA_EINVAL, "scheduled skinny GEMM: plan for a smaller M");
   const int64_t units = ((int64_t)max_m * ((s.down ? p.N : p.n_split) / 4) + 63) / 64;
   if ((int64_t)max_entries * pl.groups > INT32_MAX || max_entries * units > INT32_MAX)
     return fail(AMLA_EUNSUPPORTED, "scheduled skinny GEMM: grid");
-  static bool attr_set = false;  // raise the dynamic LDS limit once per process
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void *)gemv_sched_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr_set = true;
-  }
-  gemv_sched_kernel<<<dim3((unsigned)(max_entries * pl.groups)), 256, pl.lds, st>>>(p, s, pl.groups, pl.rg, pl.kparts,
-                                                                                   pl.kpb);
+  if (MT == 1) launch_sched_mt<1>(p, s, max_entries, pl, st);
+  else if (MT == 2) launch_sched_mt<2>(p, s, max_entries, pl, st);
+  else launch_sched_mt<4>(p, s, max_entries, pl, st);
   const int rc = check_launch("scheduled fp8 skinny GEMM");
   if (rc) return rc;
   const dim3 grid((unsigned)(max_entries * units));

@@ -61,8 +61,9 @@ def _want(h, idx, table, skip=lambda e: False):
                                        (2, 1, 300, False), (8, 4, 5, True), (1, 4, 1, True),
                                        (4, 2, 40, False), (12, 3, 60, False)])
 def test_moe_experts_dev_vs_expert_ffn(E, K, m, dup):
-    """Skinny groups (at most min(m, 64) slots: up to 16 rows in one launch, 17 and more in
-    another), GEMM tiles (larger groups) and groups made larger than m by repeated indices."""
+    """Groups on the skinny GEMM (up to 32 tokens), on the tiles (more) and made larger than m by
+    repeated indices; the header's counts: groups of at most min(m, 64) slots, 256-row units of the
+    larger ones."""
     print(f"[case] moe_experts_dev E={E} K={K} m={m} dup={dup}", flush=True)
     d, i = 256, 256
     h = _x((m, d), f"mdev{E}{K}{m}")
@@ -108,9 +109,8 @@ def test_moe_experts_dev_skips_and_counts():
 @pytest.mark.parametrize("m", [8, 40])
 def test_moe_experts_dev_r1_expert_shape(m):
     """Decode-sized batches at the R1 expert shape (hidden 7168, intermediate 2048): the K-part
-    sums of the skinny path at full size, for groups of at most 16 rows (m = 8) and of 17-64
-    rows (m = 40: each of the 4 experts gets about 20 rows), the class whose K parts and finish
-    are sized from the 64-row bound."""
+    sums of the skinny path at full size, in entries of at most 16 rows (m = 8) and of 32 (m = 40:
+    each of the 4 experts gets about 20 rows)."""
     print(f"[case] moe_experts_dev R1 shape m={m} K=2 E=4", flush=True)
     E, K, d, i = 4, 2, 7168, 2048
     h = _x((m, d), f"mdev-r1-{m}")
@@ -118,7 +118,7 @@ def test_moe_experts_dev_r1_expert_shape(m):
     idx = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(m)])
     counts = torch.bincount(idx.flatten(), minlength=E)
     if m > 16:
-        assert int(counts.min()) > 16, "every group should take the 17-64 row class"
+        assert int(counts.min()) > 16, "every group should be longer than 16 rows"
     table = {e: _mlp(d, i, f"mdev-r1-{e}") for e in range(E)}
     got, hdr = _run_dev(h, idx, _stacked(table, E), E, i)
     assert hdr[0] == m * K and hdr[3] == 0
@@ -127,7 +127,7 @@ def test_moe_experts_dev_r1_expert_shape(m):
 
 def test_moe_block_batch64_r1_shape_device_and_host_grouping_agree():
     """moe_block at batch 64 with R1-shaped experts (16 stacked experts, 8 per token): device
-    grouping (groups of 17-64 rows) against host grouping, and the device path's expert
+    grouping (groups of up to about 40 rows) against host grouping, and the device path's expert
     outputs against the oracle's expert_ffn per slot."""
     print("[case] moe_block batch 64 R1 expert shape, device vs host grouping", flush=True)
     E, K, m, d, i = 16, 8, 64, 7168, 2048
@@ -144,7 +144,7 @@ def test_moe_block_batch64_r1_shape_device_and_host_grouping_agree():
     torch.cuda.synchronize()
     idx = idx.reshape(m, K).cpu()
     counts = torch.bincount(idx.flatten(), minlength=E)
-    assert int(counts.max()) > 16, "some group should take the 17-64 row class"
+    assert int(counts.max()) > 16, "some group should be longer than 16 rows"
     assert_parity(dev_got, host_got, "moe_block batch 64: device vs host grouping")
     got, hdr = _run_dev(h.reshape(m, d), idx, stacked, E, i)
     assert hdr[0] == m * K and hdr[3] == 0
@@ -228,10 +228,10 @@ def test_moe_block_in_a_hip_graph():
 
 @pytest.mark.parametrize("d", [256, 384])
 def test_moe_experts_groups_at_the_tile_edges(d):
-    """Groups around every edge of the row tiles (16 rows on the skinny path, then 32, 64, 96 and
-    128 rows of a large tile, and more than one tile), a hidden size whose last 256-column tile is
-    half, and zero block scales in every projection: grouping on the device and on the host
-    against the oracle, and against each other bit for bit (the same tiles run either way)."""
+    """Groups around every edge of the row tiles (32, 64, 96 and 128 rows, and more than one tile), a
+    hidden size whose last 256-column tile is half, and zero block scales in every projection:
+    grouping on the device and on the host against the oracle, and against each other bit for bit
+    (a group above 64 rows puts all of them on the tiles, either way)."""
     print(f"[case] moe_experts tile edges d={d}", flush=True)
     rows = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 160, 257]
     E, i, m = len(rows), 256, sum(rows)
@@ -269,6 +269,32 @@ def test_moe_experts_dev_few_tokens_repeating_one_expert(m, K):
     assert_parity(got, _want(h, idx, table), f"moe_experts_dev repeated m={m} K={K}")
 
 
+@pytest.mark.parametrize("E,K,m,d,i", [(2, 1, 17, 7168, 2048), (8, 8, 17, 7168, 2048), (8, 8, 32, 7168, 2048),
+                                       (4, 2, 33, 7168, 2048), (4, 2, 64, 7168, 2048), (4, 4, 65, 7168, 2048),
+                                       (1, 1, 33, 7168, 2048), (24, 2, 33, 7168, 2048), (2, 1, 40, 32896, 256)])
+def test_few_experts_on_the_skinny_gemm(E, K, m, d, i):
+    """R1's expert shape with few experts, where the tiles would leave most of the machine idle:
+    entries of 16 and of 32 rows, groups that end one past them, and the switch at 32 / 33 tokens
+    (24 experts: the tiles), on the device and from a host list, against the oracle.  A hidden size
+    whose K parts the skinny GEMM cannot add takes the tiles."""
+    print(f"[case] moe_experts few experts E={E} K={K} m={m} d={d}", flush=True)
+    h = _x((m, d), f"mdev-few{m}-{d}")
+    g = torch.Generator().manual_seed(E * 101 + m)
+    idx = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(m)])
+    one = [_mlp(d, i, f"mdev-few{d}-{e}") for e in range(min(E, 3))]   # (the weights repeat)
+    table = {e: one[e % len(one)] for e in range(E)}
+    stacked = _stacked(table, E)
+    want = _want(h, idx, table)
+    got, hdr = _run_dev(h, idx, stacked, E, i)
+    assert hdr[0] == m * K and hdr[3] == 0
+    assert_parity(got, want, f"few experts, device E={E} K={K} m={m}")
+    tables, _ = ops._stacked_expert_tables(stacked, E, d, torch.device(DEV))
+    host = torch.empty(m, K, d, dtype=torch.bfloat16, device=DEV)
+    ops._moe_experts_call(h.to(DEV), idx.contiguous(), tables, i, E, host)
+    torch.cuda.synchronize()
+    assert_parity(host, want, f"few experts, host E={E} K={K} m={m}")
+
+
 def test_moe_experts_dev_hidden_of_4_gb():
     """Hidden states of more than 4 GB: a gathered row's byte offset does not fit 32 bits.  Rows
     from both ends and the middle equal the same rows in a small call bit for bit (a row's sums do
@@ -287,7 +313,8 @@ def test_moe_experts_dev_hidden_of_4_gb():
     table, n_inter = ops._stacked_device_table(stacked, E, d, torch.device(DEV))
     out = torch.empty(m, 1, d, dtype=torch.bfloat16, device=DEV)
     ops._moe_experts_dev_call(h, idx, table, n_inter, E, out)
-    rows = torch.cat([torch.arange(0, 40), torch.arange(32750, 32790), torch.arange(m - 40, m)]).to(DEV)
+    # (more than 64 rows per expert: on the tiles, as in the large call)
+    rows = torch.cat([torch.arange(0, 100), torch.arange(32700, 32800), torch.arange(m - 100, m)]).to(DEV)
     few = torch.empty(rows.numel(), 1, d, dtype=torch.bfloat16, device=DEV)
     ops._moe_experts_dev_call(h[rows].contiguous(), idx[rows].contiguous(), table, n_inter, E, few)
     torch.cuda.synchronize()
