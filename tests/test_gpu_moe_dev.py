@@ -269,6 +269,27 @@ def test_moe_experts_dev_few_tokens_repeating_one_expert(m, K):
     assert_parity(got, _want(h, idx, table), f"moe_experts_dev repeated m={m} K={K}")
 
 
+def test_expert_blocks_of_the_smallest_scales():
+    """Blocks of zeros under the smallest float scales between ordinary ones (a quantiser that clamps
+    their maximum), groups on the tiles of 32 to 128 rows."""
+    print("[case] moe_experts smallest scales", flush=True)
+    rows, d, i = [20, 40, 70, 110], 384, 384 + 128
+    E, m = len(rows), sum(rows)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).view(m, 1)
+    h = _x((m, d), "mdev-tiny")
+    table = {e: _mlp(d, i, f"mdev-tiny{e}") for e in range(E)}
+    for e in range(E):
+        for w, s in table[e].values():
+            for b in range(s.shape[0]):
+                j = (b + e) % s.shape[1]
+                z = w[128 * b:128 * b + 128, 128 * j:128 * j + 128]
+                z.copy_(torch.zeros_like(z))
+                s[b, j] = 2.0 ** -126 if b % 2 else 2.0 ** -149
+    stacked = _stacked(table, E)
+    got, _ = _run_dev(h, idx, stacked, E, i)
+    assert_parity(got, _want(h, idx, table), "smallest scales")
+
+
 @pytest.mark.parametrize("E,K,m,d,i", [(2, 1, 17, 7168, 2048), (8, 8, 17, 7168, 2048), (8, 8, 32, 7168, 2048),
                                        (4, 2, 33, 7168, 2048), (4, 2, 64, 7168, 2048), (4, 4, 65, 7168, 2048),
                                        (1, 1, 33, 7168, 2048), (24, 2, 33, 7168, 2048), (2, 1, 40, 32896, 256)])

@@ -118,3 +118,27 @@ def test_rows_four_gb_apart(m, stride, f32):
     got = ops.fp8_linear(far, w, s, out)
     assert torch.equal(got, ops.fp8_linear(x, w, s, out))
     _check(got, want, bound, not f32)
+
+
+@pytest.mark.parametrize("m,n,k", [(100, 384, 640), (129, 256, 1152), (160, 144, 2304)])
+def test_blocks_of_the_smallest_scales(m, n, k):
+    """Blocks of zeros under the smallest normal and denormal scales (a quantiser that clamps their
+    maximum) between ordinary blocks, and small values under a scale of 2^-80: in 96 and 128-row
+    tiles and in those of whole lines, with K parts and without."""
+    print(f"[case] tile linear smallest scales m={m} n={n} k={k}", flush=True)
+    x, w, s, _, _ = _case(m, n, k, "tiny")
+    w, s, nb, kb = w.cpu(), s.cpu(), -(-n // 128), k // 128
+    blk = lambda i, j: (slice(128 * i, 128 * i + 128), slice(128 * j, 128 * j + 128))
+    for i in range(nb):
+        for j, v in (((i + 1) % kb, 2.0 ** -126), ((i + 3) % kb, 2.0 ** -149)):
+            w[blk(i, j)] = torch.zeros_like(w[blk(i, j)])
+            s[i, j] = v
+    s[nb - 1, kb - 1] = 2.0 ** -80
+    full = w.double() * s.double().repeat_interleave(128, 0)[:n].repeat_interleave(128, 1)[:, :k]
+    want = x.double().cpu() @ full.T
+    bound = 2e-5 * (x.double().cpu().norm(dim=1)[:, None] * full.norm(dim=1)[None, :]) + 1e-30
+    need = lib().amla_fp8_linear_workspace_bytes(m, n, k)
+    wd, sd = w.to(DEV), s.to(DEV)
+    for ws in {need or None, None}:
+        _check(_raw(x, wd, sd, n, False, ws), want, bound, True)
+        _check(_raw(x, wd, sd, n, True, ws), want, bound, False)
