@@ -941,8 +941,7 @@ static MoeDevLayout moe_dev_layout(int64_t m, int64_t d, int top_k, int64_t n, i
     const size_t pb = b.kparts > 1 ? (size_t)b.kparts * S * d * 4 : 0;
     L.part = take(std::max<size_t>(std::max(pa, pb), 16));
   }
-  // never below the size callers could count on before the rows were gathered in place
-  L.total = std::max(off, (size_t)S * (2 * d + 3 * n) * 2);
+  L.total = off;
   return L;
 }
 
@@ -1075,7 +1074,14 @@ size_t amla_moe_experts_dev_workspace_bytes(int64_t m, int64_t d, int top_k, int
   if (m <= 0 || d <= 0 || top_k <= 0 || top_k > 64 || n_inter <= 0 || n_experts <= 0 ||
       n_experts > MSORT_MAXE || m * top_k > MOE_DEV_MAX_SLOTS)
     return 0;
-  return moe_dev_layout(m, d, top_k, n_inter, n_experts, moe_dev_skinny_rows(m, d, top_k, n_inter, n_experts)).total;
+  // and enough for any smaller call: above 32 tokens the tiles run where the
+  // K-part sums of the skinny GEMM do not fit, up to 32 these are needed
+  size_t total = 0;
+  for (int64_t t : {(int64_t)8, (int64_t)16, (int64_t)32, m})
+    if (t <= m)
+      total = std::max(total, moe_dev_layout(t, d, top_k, n_inter, n_experts,
+                                             moe_dev_skinny_rows(t, d, top_k, n_inter, n_experts)).total);
+  return total;
 }
 
 int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, const int64_t *indices,
@@ -1092,8 +1098,10 @@ int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, co
       !aligned16(expert_out))
     return fail(AMLA_EUNSUPPORTED,
                 "moe_experts_dev: needs hidden %% 128 == 0, intermediate %% 256 == 0 and 16-byte aligned rows");
-  const MoeDevLayout L =
+  MoeDevLayout L =
       moe_dev_layout(m, d, top_k, n_inter, n_experts, moe_dev_skinny_rows(m, d, top_k, n_inter, n_experts));
+  if (m > 32 && !L.tiles && (!workspace || workspace_bytes < L.total))
+    L = moe_dev_layout(m, d, top_k, n_inter, n_experts, 0);
   if (!workspace || workspace_bytes < L.total || !aligned16(workspace))
     return fail(AMLA_EWORKSPACE, "moe_experts_dev: needs %zu bytes of 16-byte aligned workspace (got %zu)", L.total,
                 workspace ? workspace_bytes : (size_t)0);

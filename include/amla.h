@@ -260,10 +260,12 @@ size_t amla_moe_experts_workspace_bytes(int64_t m, int64_t d, int top_k, int64_t
  *   n_inter % 256 == 0.
  * A slot whose index is >= n_experts, or whose expert has a NULL or misaligned
  * pointer in the table, is skipped like a negative one and counted: after the
- * call the first 16 bytes of the workspace hold int32 {routed slots, skinny
- * groups, GEMM tiles, skipped slots}.  Workspace of
+ * call the first 16 bytes of the workspace hold int32 {routed slots, experts
+ * with 1 .. min(m, 64) slots, 256-slot units of the experts with more, skipped
+ * slots}: they describe the routing, whichever kernels ran.  Workspace of
  * amla_moe_experts_dev_workspace_bytes(m, d, top_k, n_inter, n_experts) bytes
- * (0 for unsupported sizes); calls that share a workspace must not overlap. */
+ * (0 for unsupported sizes), enough for fewer tokens too; calls that share a
+ * workspace must not overlap. */
 int amla_moe_experts_dev(const void *hidden, int64_t m, int64_t d, int top_k, const int64_t *indices,
                          int64_t n_inter, int64_t n_experts, const void *const *weight_table, void *expert_out,
                          void *workspace, size_t workspace_bytes, void *stream);

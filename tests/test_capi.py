@@ -179,7 +179,10 @@ def test_moe_experts_dev_checks_sizes_on_the_host():
     p = p0 + 16 - p0 % 16 if p0 % 16 else p0
     m, d, top_k, n, E = 8, 256, 8, 256, 256
     need = L.amla_moe_experts_dev_workspace_bytes(m, d, top_k, n, E)
-    assert need >= 2 * m * top_k * d * 2 + 3 * m * top_k * n * 2
+    slots = m * top_k
+    assert need >= slots * 3 * n * 2 + 2 * slots * 4       # [gate | up] and h rows, the two row lists
+    # hidden rows are gathered and results scattered in place: 2000 tokens of R1's experts hold h and lists alone
+    assert L.amla_moe_experts_dev_workspace_bytes(2000, 7168, 8, 2048, E) < 16000 * (2048 * 2 + 64)
     assert L.amla_moe_experts_dev_workspace_bytes(m, d, top_k, n, 513) == 0      # more than 512 experts
     assert L.amla_moe_experts_dev_workspace_bytes(8193, d, 8, n, E) == 0          # 65544 slots
     assert L.amla_moe_experts_dev(None, m, d, top_k, p, n, E, p, p, p, need, None) == -1
@@ -221,6 +224,15 @@ def test_route_workspace_for_more_tokens_holds_fewer(E):
     L, p = _lib.lib(), 1 << 12
     _largest_smaller_call([m for m in ROWS if m > 64], lambda m: L.amla_moe_route_workspace_bytes(m, E),
                           lambda m: _least(lambda: L.amla_moe_route(p, m, 7168, p, E, 4, 2, 4, 1, p, p, None, 0, None)))
+
+
+@pytest.mark.parametrize("d,top_k,n,E", [(7168, 8, 2048, 256), (7168, 2, 2048, 4), (7168, 8, 2048, 8), (2048, 6, 1536, 64),
+                                         (256, 2, 256, 4), (32896, 1, 256, 2)])
+def test_moe_experts_dev_workspace_for_more_tokens_holds_fewer(d, top_k, n, E):
+    L, p = _lib.lib(), 1 << 12
+    _largest_smaller_call(
+        ROWS, lambda m: L.amla_moe_experts_dev_workspace_bytes(m, d, top_k, n, E),
+        lambda m: _least(lambda: L.amla_moe_experts_dev(p, m, d, top_k, p, n, E, p, p, None, 0, None)))
 
 
 @pytest.mark.parametrize("batch,rows", [(1, 333), (1, 8192), (1, 32768), (4, 256), (4, 1024), (13, 64), (13, 4096)])

@@ -75,6 +75,31 @@ def test_route_with_fewer_k_splits(m):
         assert torch.allclose(w, w0, rtol=1e-5, atol=1e-6) and (idx == i0).float().mean() > 0.999
 
 
+def test_experts_without_room_for_k_parts():
+    """Few experts, 40 tokens: the skinny GEMM with its K-part sums, or the tiles without."""
+    print("[case] experts workspace", flush=True)
+    E, K, m, d, n = 4, 2, 40, 7168, 2048
+    x = synth.randn((m, d), synth.seed_of("wse", m), 1.0).to(torch.bfloat16)
+    g = torch.Generator().manual_seed(3)
+    idx = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(m)])
+    w = {}
+    for i, (name, a, b) in enumerate((("gate_proj", n, d), ("up_proj", n, d), ("down_proj", d, n))):
+        w[name] = synth.quantize_fp8_blocks(synth.randn((a, b), synth.seed_of("wse-w", i), 0.02))
+    one = F.expert_ffn(x, w)                     # every expert the same weights, each at its own address
+    want = one[:, None].expand(m, K, d)
+    st = {k: (q[None].repeat(E, 1, 1).to(DEV), s[None].repeat(E, 1, 1).to(DEV)) for k, (q, s) in w.items()}
+    table, _ = ops._stacked_device_table(st, E, d, torch.device(DEV))
+    xd, idd, y = x.to(DEV), idx.to(DEV), torch.empty(m, K, d, dtype=torch.bfloat16, device=DEV)
+    call = lambda p, b: lib().amla_moe_experts_dev(xd.data_ptr(), m, d, K, idd.data_ptr(), n, E, table.data_ptr(),
+                                                   y.data_ptr(), p, b, ops._stream_ptr(xd))
+    full, least = lib().amla_moe_experts_dev_workspace_bytes(m, d, K, n, E), _least(call)
+    assert least < full
+    for b in (full, least, (full + least) // 2):
+        y.zero_()
+        _run(call, b)
+        assert_parity(y, want, f"experts in {b} bytes")
+
+
 @pytest.mark.parametrize("S,starts,rows", [(5, list(range(28, 54, 2)), 64), (181, [700], 1024), (70, [3, 0, 30], 128)])
 def test_prefill_in_the_form_and_parts_that_fit(S, starts, rows):
     """Latent attention where its scratch fits, decompressed where only that does; with and without
