@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from amla import _lib
+from _prefill import runs_latent, scratch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "amla.h")
@@ -251,6 +252,26 @@ def test_prefill_workspace_for_more_tokens_holds_fewer(batch, rows):
     _largest_smaller_call([s for s in ROWS if s <= rows and s * batch <= 4096],
                           lambda s: at(s, lambda: L.amla_mla_prefill_workspace_bytes(ctypes.byref(a))),
                           lambda s: at(s, lambda: _least(lambda: L.amla_mla_prefill(ctypes.byref(a), None))))
+
+
+@pytest.mark.parametrize("batch,new,rows", [(13, 5, 33), (13, 5, 64), (33, 2, 64), (22, 3, 96), (1, 65, 2021), (4, 9, 1214),
+                                            (1, 50, 8192), (1, 2, 1030)])
+def test_latent_prefill_scratch_holds_every_chunk(batch, new, rows):
+    """Up to 64 tokens run at a time, in chunks of equal size but for a smaller last one (65: 33 + 32),
+    which over two tiles of context is cut into more splits (64 + 32 slots against 33 + 33)."""
+    assert runs_latent(batch, new, rows)
+    tokens, tiles = batch * new, -(-rows // 32)
+    chunk = -(-tokens // -(-tokens // 64))
+    sizes = {min(chunk, tokens - t) for t in range(0, tokens, chunk)}
+    slots = max(n + min(256, n * tiles if n * tiles <= 64 else n * max(1, tiles // 2)) for n in sizes)
+    # fp32 partial O, (m, l), the absorbed queries (bf16)
+    assert scratch(batch, new, rows) >= slots * 128 * (512 * 4 + 2 * 4) + chunk * 128 * 576 * 2
+
+
+@pytest.mark.parametrize("batch,new,rows,latent", [(1, 1000, 1000, False), (1, 4096, 4096, False), (3, 70, 128, False),
+                                                   (1, 50, 8192, True), (13, 5, 64, True)])
+def test_form_of_a_prefill(batch, new, rows, latent):
+    assert runs_latent(batch, new, rows) == latent
 
 
 def test_sample_checks_sizes_on_the_host():

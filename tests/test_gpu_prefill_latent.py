@@ -2,15 +2,13 @@
 token and many, several sequences with their own start, more tokens than one launch holds, tile
 and split edges, chosen and not; against the oracle per sequence (its roundings), per head and
 after o_proj, with the cache rows written."""
-import ctypes
-
 import pytest
 import torch
 
 from oracle import ref_ops as R
 from amla import ops, synth
-from amla._lib import MlaArgs, lib
 from amla.config import DeepSeekConfig
+from _prefill import runs_latent
 from _tol import assert_bf16_ulps, assert_heads_parity, assert_parity
 
 pytestmark = pytest.mark.gpu
@@ -28,11 +26,12 @@ def _gpu(aw):
 
 
 @pytest.mark.parametrize("S,starts", [(2, [1023]), (7, [640]), (33, [1500]), (65, [1951]), (9, [513, 0, 1200, 70]),
-                                      (40, [900, 31])])
+                                      (40, [900, 31]), (5, list(range(28, 54, 2)))])
 def test_new_tokens_over_a_cache(layer, S, starts):
     print(f"[case] latent prefill S={S} starts={starts}", flush=True)
     B = len(starts)
     rows = max(starts) + S + 5
+    assert runs_latent(B, S, rows)
     hidden = synth.make_hidden(CFG, B, S, f"lp{S}")
     ckv, kpe = synth.make_kv_cache(CFG, B, rows, starts, f"lp{S}")
     tab = R.precompute_rope_freqs(CFG, rows)
@@ -66,12 +65,13 @@ def test_prompt_and_token_by_token_agree(layer):
     assert_bf16_ulps(ckv, c2, 2, "cache rows")
 
 
-@pytest.mark.parametrize("S,starts", [(5, [700]), (66, [3, 0, 30]), (130, [1])])
-def test_norm_weights_at_any_alignment(layer, S, starts):
+@pytest.mark.parametrize("S,starts,latent", [(5, [700], True), (66, [3, 0, 30], False), (130, [1], False)])
+def test_norm_weights_at_any_alignment(layer, S, starts, latent):
     """The row passes between the projections and the latent merge read the norm weights 16 bytes at
     a time where these are aligned: weights two bytes off give the same result."""
     print(f"[case] prefill norm weights S={S} starts={starts}", flush=True)
     B, rows = len(starts), max(starts) + S + 2
+    assert runs_latent(B, S, rows) == latent
     aw = _gpu(layer.attn_weights)
     hidden = synth.make_hidden(CFG, B, S, "lp-gamma").to(DEV)
     kv = [t.to(DEV) for t in synth.make_kv_cache(CFG, B, rows, starts, "lp-gamma")]
@@ -93,13 +93,6 @@ def test_norm_weights_at_any_alignment(layer, S, starts):
     assert_parity(both, want, f"both weights off S={S}")
 
 
-def _sizes(B, S, context):
-    a = MlaArgs()
-    a.batch, a.seq_len, a.hidden, a.heads, a.q_lora, a.kv_lora = B, S, 7168, 128, 1536, 512
-    a.qk_nope, a.qk_rope, a.v_dim, a.max_seq, a.rope_rows, a.max_context = 128, 64, 128, context, context, context
-    return lib().amla_mla_prefill_workspace_bytes(ctypes.byref(a))
-
-
 @pytest.mark.parametrize("S,p", [(12, 1500), (70, 4000)])
 def test_heads_lose_nothing_to_16_bit_sums(layer, S, p):
     """Rows about one latent vector under equal scores, where the roundings of a split's sums and of
@@ -107,7 +100,7 @@ def test_heads_lose_nothing_to_16_bit_sums(layer, S, p):
     bf16 (taken from the 64-bit values) and the one of p r_t, 2^-9 at most on each weight and, the
     row norms spread over several bf16 steps, under 2^-11 on a sum of them."""
     T = p + S
-    assert _sizes(1, S, T) < T * 128 * 256 * 2, "the decompressed form was chosen"
+    assert runs_latent(1, S, T)
     print(f"[case] latent prefill precision S={S} T={T}", flush=True)
     aw = _gpu(layer.attn_weights)
     aw["q_b_proj"] = (aw["q_b_proj"][0], aw["q_b_proj"][1] * 1e-12)
@@ -129,16 +122,3 @@ def test_heads_lose_nothing_to_16_bit_sums(layer, S, p):
     err, own = (heads[0].double().cpu() - want).norm() / n, (want.to(torch.bfloat16).double() - want).norm() / n
     print(f"    error {err:.6f}, rounding of the result {own:.6f}", flush=True)
     assert err ** 2 <= own ** 2 + 2.0 ** -22
-
-
-def test_scratch_covers_a_smaller_last_chunk():
-    """65 tokens run as 33 + 32: the smaller chunk may be cut into more one-tile splits."""
-    from amla._lib import MlaArgs
-    a = MlaArgs()
-    a.batch, a.seq_len, a.hidden, a.heads, a.q_lora, a.kv_lora = 1, 65, 7168, 128, 1536, 512
-    a.qk_nope, a.qk_rope, a.v_dim = 128, 64, 128
-    sizes = []
-    for ctx in (65, 128, 600, 4096, 32768):
-        a.max_seq = a.rope_rows = a.max_context = ctx
-        sizes.append(lib().amla_mla_prefill_workspace_bytes(ctypes.byref(a)))
-    assert all(s > 0 for s in sizes)

@@ -62,11 +62,15 @@ def test_tiles_and_k_parts(m, n, k, f32):
     _check(got, want, bound, not f32)
 
 
-def test_many_tiles_end_in_parts():
-    """More tiles than one round of the machine (512): whole tiles first, the rest in K parts."""
-    m, n, k = 128 * 65, 256 * 9, 512
-    need = lib().amla_fp8_linear_workspace_bytes(m, n, k)
-    print(f"[case] tile linear {65 * 9} tiles, workspace {need}", flush=True)
+@pytest.mark.parametrize("m,n,k", [(128 * 65, 256 * 8, 1152), (384, 256 * 173, 1152), (896, 256 * 74, 1152)])
+def test_many_tiles_end_in_parts(m, n, k):
+    """More tiles than one round of the machine (512): whole tiles first, the rest in K parts; 65 row
+    tiles, and 3 and 7 of them, which do not divide the round (a column tile's row tiles are then
+    split between the two)."""
+    tiles, need = -(-m // 128) * (n // 256), lib().amla_fp8_linear_workspace_bytes(m, n, k)
+    print(f"[case] tile linear {tiles} tiles, workspace {need}", flush=True)
+    rest, part = tiles - 512, 256 * 128 * 4
+    assert 0 < rest < 64 and need % (rest * part) == 0 and 2 <= need // (rest * part) <= 16
     x, w, s, want, bound = _case(m, n, k, "many")
     _check(ops.fp8_linear(x, w, s), want, bound, True)
 
