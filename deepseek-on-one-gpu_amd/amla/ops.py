@@ -278,7 +278,8 @@ def mla_attention(hidden: torch.Tensor, attn_weights: dict, kv_cache: tuple, pos
     """inference/ops.py:100-183 on gfx950 (``torch.ops.amla.mla_decode`` / ``mla_prefill``).
 
     S == 1 runs the absorbed decode; S > 1 the kv_b decompression + causal
-    flash prefill.  Writes the raw new rows into ``kv_cache`` at
+    flash prefill, or, for a few new tokens over many cached rows, the same
+    attention in latent space as the decode.  Writes the raw new rows into ``kv_cache`` at
     [position, position+S) like the reference.  ``max_context`` (largest
     position+S) is only needed when ``position`` is a device tensor.  When
     ``attn_out`` ((B, S, heads * v_head_dim) bf16) is given, the per-head

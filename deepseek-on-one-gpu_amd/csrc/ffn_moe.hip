@@ -9,11 +9,13 @@
 //                        gpu_transfer.py:60, has no counterpart)
 //   amla_moe_combine  <- the combine of moe_block, inference/forward.py:138-153
 //
-// swiglu runs gate and up as one skinny (M <= 64) or large fp8 GEMM over the
-// two stacked weights, one elementwise pass for silu * up over the stacked
-// rows, and the down projection; the rounding points are the reference's (bf16
-// after every linear, after silu and after the product).  The routed experts
-// of a MoE layer run as grouped skinny GEMMs (up to 32 experts per launch).
+// swiglu runs gate and up as one skinny fp8 GEMM over the two stacked weights
+// (M <= 64; silu * up in its K-part finish or in a pass over the stacked rows)
+// or on the GEMM tiles (silu * up in their epilogue), then the down projection;
+// the rounding points are the reference's (bf16 after every linear, after silu
+// and after the product).  The routed experts of a MoE layer run as grouped or
+// device-scheduled skinny GEMMs or tiles, all groups of a call in one form
+// (moe_skinny_us, moe_tiles_us).
 // Routing computes the fp32 logits with bf16 MFMAs (exact products, fp32
 // sums), then one wave per token does the sigmoid, the group ranking and the
 // top-k in fp32.
@@ -968,8 +970,9 @@ AMLA_DEV int block_scan_incl(int v, int *wsum, int lane, int wave) {
 //   ent[]     = (expert, first position, rows <= rows_max) of every group,
 //               cut at rows_max;
 //   count     = entries;
-//   hdr       = {routed slots, groups of 1 .. sb slots, 256-row tiles of the
-//               larger groups, skipped slots}, sb = min(tokens, 64).
+//   hdr       = {routed slots, groups of 1 .. sb slots, 256-slot units of the
+//               larger groups, skipped slots}, sb = min(tokens, 64): counts of the
+//               routing for the caller, no launch reads them.
 // Slots with a negative index are left out; an index >= E, or an expert with a
 // null or misaligned weight, is left out and counted as skipped.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const int64_t *__restrict__ idx, int S, int top_k, int E,

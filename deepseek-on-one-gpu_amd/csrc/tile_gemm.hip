@@ -23,10 +23,10 @@ namespace amla {
 // What bounds it: with few rows per expert the weight stream from HBM (64 rows
 // are 128 FLOP per weight byte), above about 128 rows the MFMAs.  MI355X, 256
 // R1 experts, top 8: 300 tokens (9 rows per expert) [gate | up] with silu * up
-// 1.28 ms (5.9 TB/s), down 0.66 ms, where the skinny GEMM with fp32 K parts and
-// finishing passes took 1.55 + 0.82 ms; 2000 tokens (62 rows) 1.66 + 0.89 ms
+// 1.27 ms (5.9 TB/s), down 0.68 ms, where the skinny GEMM with fp32 K parts and
+// finishing passes took 1.55 + 0.82 ms; 2000 tokens (62 rows) 1.59 + 0.87 ms
 // against 2.75 + 1.62 for that and 256 x 256 tiles for groups above 64 rows;
-// 8000 tokens (250 rows) 4.8 + 2.4 ms against 5.6 + 2.9.  Gathering and
+// 8000 tokens (250 rows) 4.4 + 2.2 ms against 5.6 + 2.9.  Gathering and
 // scattering the rows here saved two more passes (0.14 ms at 2000 tokens).
 //
 // Above 64 rows (TileHalves): two K stages of 64 in LDS, fp8 weight rows (64 B,
@@ -298,7 +298,8 @@ struct TileHalves {
 // lines of the weights, one segment of a K block at a time (16 KB: 128 rows x 128 B,
 // three in the ring, two ahead), the activation rows a K block at a time (two
 // buffers).  With stages of 64 K values of both segments every line was fetched
-// in two halves: LINES_FIG.
+// in two halves: [gate | up] of 256 experts at 300 tokens took 1344 us against
+// 1252, at 1000 tokens 1409 / 1317.
 //
 // LDS: weight row 128 B, chunk c of row r at c ^ ((r >> 1) & 7); activation row
 // 256 B, chunk c of row r at c ^ (r & 15): the 16 lanes of a fragment-read pass

@@ -172,7 +172,8 @@ int amla_mla_decode_noalloc(const amla_mla_args *args, void *stream);
 
 /* Replaces mla_attention(...) for S >= 1 with a causal mask over the new rows
  * (inference/ops.py:100-183 incl. :172-177): kv_b decompression of the cached
- * rows and flash attention with bf16 MFMA. */
+ * rows and flash attention with bf16 MFMA, or, for a few new tokens over many
+ * rows, the decode's attention in latent space with fp32 partial sums. */
 int amla_mla_prefill(const amla_mla_args *args, void *stream);
 
 /* Workspace bytes amla_mla_decode / amla_mla_prefill need for these args
@@ -230,8 +231,9 @@ size_t amla_moe_route_workspace_bytes(int64_t m, int64_t n_experts);
  * device pointers (only the chosen experts' entries are read; others may be
  * NULL), the weights of
  * expert e laid out as for amla_swiglu with intermediate size n_inter.  Each
- * chosen expert runs once over all of its tokens (gather, [gate | up] in one
- * skinny GEMM, silu * up, down, scatter).  hidden (m, d) bf16, expert_out
+ * chosen expert runs once over all of its tokens (gather, [gate | up], silu *
+ * up, down, scatter; every expert of a call on the skinny GEMM or every one on
+ * the GEMM tiles, by their number and sizes).  hidden (m, d) bf16, expert_out
  * (m, top_k, d) bf16; d % 128 == 0, n_inter % 256 == 0, top_k <= 64.
  * Workspace of amla_moe_experts_workspace_bytes(m, d, top_k, n_inter) bytes.
  * Up to 512 (token, k) slots the call is asynchronous like the others; above
