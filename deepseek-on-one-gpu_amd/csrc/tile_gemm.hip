@@ -61,20 +61,14 @@ struct TileArgs {
   bool wide;             // byte offsets of the tile's x rows may not fit 32 bits
 };
 
-// Block scales of a segment's K range that count as zero: zero itself and those
-// below 2^-64 of the largest (some quantisers give a block of zeros the smallest
-// float), as bits without the sign: those less than the returned ones.  Rescaling
-// the sums to units that small would overflow them.  A lane reads every 64th
-// scale, the first (lane_scale) before the copies go out, so that the wait for it
-// is not one for them.
-AMLA_DEV uint32_t scale_bits(float s) { return __float_as_uint(s) & 0x7fffffffu; }
-AMLA_DEV float lane_scale(const float *s, int kb0, int kb1) { return s[min(kb0 + (int)(threadIdx.x & 63), kb1 - 1)]; }
-AMLA_DEV uint32_t scale_floor(float first, const float *s, int kb0, int kb1) {
-  uint32_t top = scale_bits(first);
-  for (int k = kb0 + 64 + (threadIdx.x & 63); k < kb1; k += 64) top = max(top, scale_bits(s[k]));
-  const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)(wave_max_u32(top) >> 23));
-  return e > 64 ? (e - 64) << 23 : 1;
-}
+// A block scale that is zero, or below 2^-64 of the largest of the tile's K range
+// so far, counts as zero (some quantisers give a block of zeros the smallest
+// float): rescaling the sums to units that small would overflow them.  Scales are
+// compared as bits without the sign, on the scalar unit: `floor`, the smallest
+// that counts, grows with each block.  (All scales read ahead of the loop instead,
+// by the lanes: 1.5 us more per launch.)
+AMLA_DEV int scale_bits(float s) { return (int)(__float_as_uint(s) & 0x7fffffffu); }
+AMLA_DEV int scale_floor(int bits) { return max(bits - (64 << 23), 1); }
 
 // A tile's sums: acc[segment][row group of 32], in units of s_run[segment].
 template <int NJ>
@@ -176,7 +170,7 @@ struct TileHalves {
       for (int r = 0; r < 16; ++r) acc[g][j][r] = 0.f;
   // The accumulators are kept in units of the current K block's scale: acc *=
   // s_prev / s_cur between two blocks, * s_last at the end (fp32 rounding of
-  // the ratios, ~1e-5 relative over 128 blocks).  A zero scale (below sfloor)
+  // the ratios, ~1e-5 relative over 128 blocks).  A zero scale (below sfloor, scale_floor)
   // dequantises to zeros: the segment's fragments of that block are read from 16
   // zeroed bytes instead and the units stay.
 #pragma unroll
@@ -184,18 +178,11 @@ struct TileHalves {
   if (tid < 4) *reinterpret_cast<uint32_t *>(tsm + T_ZERO + 4 * tid) = 0;  // visible after the first barrier
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
+  int sfloor[2] = {scale_floor(scale_bits(s_run[0])), scale_floor(scale_bits(s_run[1]))};
+  bool zero[2] = {s_run[0] == 0.f, s_run[1] == 0.f};
+
   const int it0 = 2 * a.kb0, iters = 2 * a.kb1;
-  const float ls[2] = {lane_scale(a.s[0], a.kb0, a.kb1), lane_scale(a.s[1], a.kb0, a.kb1)};
-  __builtin_amdgcn_sched_barrier(0);
   dma(it0, 0);
-  uint32_t sfloor[2];
-  bool zero[2];
-#pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    sfloor[g] = scale_floor(ls[g], a.s[g], a.kb0, a.kb1);
-    zero[g] = scale_bits(s_run[g]) < sfloor[g];
-    if (zero[g]) s_run[g] = 0.f;
-  }
   // One stage of 64: four sub-steps of 16 (K 32 pr + 16 hh + 8 s2 .. +7 of each
   // half-wave).  While a sub-step multiplies, the fragments of the next are
   // read and converted between its MFMAs.  The rescaling between two blocks
@@ -287,6 +274,7 @@ struct TileHalves {
       for (int g = 0; g < 2; ++g) {
         zero[g] = scale_bits(sn[g]) < sfloor[g];
         if (!zero[g]) s_run[g] = sn[g];
+        sfloor[g] = max(sfloor[g], scale_floor(scale_bits(sn[g])));
       }
     }
   }
@@ -388,18 +376,11 @@ struct TileLines {
   for (int g = 0; g < 2; ++g) s_run[g] = srow[g][a.kb0];
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
-  const float ls[2] = {lane_scale(a.s[0], a.kb0, a.kb1), lane_scale(a.s[1], a.kb0, a.kb1)};
-  __builtin_amdgcn_sched_barrier(0);
   dma_w(a.kb0, 0, 0);
   dma_x(a.kb0, 0);
   dma_w(a.kb0, 1, 1);
-  uint32_t sfloor[2], keep[2];
-#pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    sfloor[g] = scale_floor(ls[g], a.s[g], a.kb0, a.kb1);
-    keep[g] = scale_bits(s_run[g]) < sfloor[g] ? 0u : ~0u;
-    if (!keep[g]) s_run[g] = 0.f;
-  }
+  int sfloor[2] = {scale_floor(scale_bits(s_run[0])), scale_floor(scale_bits(s_run[1]))};
+  uint32_t keep[2] = {s_run[0] == 0.f ? 0u : ~0u, s_run[1] == 0.f ? 0u : ~0u};
   int slot = 0, buf = 0;
   // One segment of a K block: eight sub-steps of 16 (K 32 pr + 16 hh + 8 s2 ..
   // +7 of each half-wave).  `other`: the other segment's sums change their units
@@ -463,6 +444,7 @@ struct TileLines {
       for (int g = 0; g < 2; ++g) {
         keep[g] = scale_bits(sn[g]) < sfloor[g] ? 0u : ~0u;
         if (keep[g]) s_run[g] = sn[g];
+        sfloor[g] = max(sfloor[g], scale_floor(scale_bits(sn[g])));
       }
     }
   }
