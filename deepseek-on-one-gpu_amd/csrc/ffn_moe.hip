@@ -619,12 +619,12 @@ constexpr int MOE_SKINNY_ROWS = 64;   // most rows of an entry on the skinny GEM
 // Measured on MI355X, hidden 7168 x intermediate 2048, top 2 of E experts (host
 // lists; us, skinny / tiles): E = 1 32 rows each 55 / 94, 64 rows 72 / 124;
 // E = 4 24 rows 69 / 95, 50 rows 88 / 125; E = 8 8 rows 86 / 99, 25 rows 103 /
-// 104; top 8 of 16 16 rows 184 / 146; of 64 12 rows 626 / 520; 2048 x 1536 E = 4
-// 24 rows 53 / 44.  Model of both projections in us (entries: groups, cut to the
+// 104; top 8 of 16 16 rows 184 / 146; of 64 12 rows 626 / 520; of 128 2 rows 896 /
+// 894, 3 rows 1014 / 945; 2048 x 1536 E = 4 24 rows 53 / 44.  Model of both projections in us (entries: groups, cut to the
 // rows a workgroup takes; K block times as in plan_gemm_split):
 static double moe_skinny_us(double entries, double slots, int rows_max, int64_t d, int64_t n) {
   const double bytes = 3.0 * n * d * entries;
-  return std::max(rows_max > 32 ? 63.0 : 45.0, bytes * (1.0 + 0.025 * slots / std::max(entries, 1.0)) / 6.1e6);
+  return std::max(rows_max > 32 ? 63.0 : 45.0, bytes * (1.0 + 0.04 * (slots / std::max(entries, 1.0) - 1.0)) / 6.2e6);
 }
 static double moe_tiles_us(double entries, double rows_max, int64_t d, int64_t n) {
   const double nj = std::ceil(std::min<double>(rows_max, TILE_ROWS) / 32), one = 0.9 + 0.3 * nj,
@@ -633,7 +633,7 @@ static double moe_tiles_us(double entries, double rows_max, int64_t d, int64_t n
     return k / 128 * (blocks <= 256 ? one : std::ceil(blocks / 512) * two);
   };
   return std::max(8.0 + pass(entries * (n / 128), d) + pass(entries * ((d + 255) / 256), n),
-                  3.0 * n * d * entries / 5.8e6);
+                  3.0 * n * d * entries / 6.1e6);
 }
 // K parts within what the skinny GEMM's finishing passes add up (hidden sizes
 // above 32768 are past it)
@@ -783,7 +783,7 @@ int amla_moe_experts(const void *hidden, int64_t m, int64_t d, int top_k, const 
     int max_run = 0;
     for (int r = 0; r < nruns; ++r) max_run = std::max(max_run, run_begin[r + 1] - run_begin[r]);
     const bool tiles = max_run > MOE_SKINNY_ROWS || !moe_skinny_fits(max_run, d, n) ||
-                       moe_tiles_us(nruns, max_run, d, n) < 0.95 * moe_skinny_us(nruns, ns, max_run, d, n);
+                       moe_tiles_us(nruns, max_run, d, n) < 0.97 * moe_skinny_us(nruns, ns, max_run, d, n);
     GemvParams pg = {};  // [gate | up] x (cnt, D) -> gu (cnt, 2n)
     pg.ldx = D;
     pg.N = 2 * n;
